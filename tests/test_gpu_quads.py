@@ -1,0 +1,87 @@
+"""The four-lane kernels of small working sets against the one-lane kernels.
+
+Up to a number of working slots the default shapes give every particle four
+lanes, which share its candidates and pairs and add the terms in the one-lane
+order: every field must hold the same bits as the explicit one-lane shapes,
+in both arithmetic modes, on both sides of the limits, and for stencils and
+lists longer than the four-lane kernels' windows.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import water_simulation_amd as ws
+from helpers import assert_bitexact
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+R = 0.01
+ONE_LANE = dict(density_alpha_nt=512, xsph_nt=256, change_nt=256, apply_nt=256)
+FIELDS = ("dfsph_density", "dfsph_alpha", "dfsph_kappa", "dfsph_density_adv")
+
+
+def cloud(n, clump):
+    """n particles resting on the floor of a 1 m box: a jittered lattice or,
+    with `clump`, half of it squeezed (long stencils, lists over their depth)
+    with a few coincident pairs."""
+    rng = np.random.default_rng(n)
+    side = int(np.ceil(n ** (1 / 3)))
+    g = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    x = 0.06 + 2 * R * g * (0.9 / max(1.0, side * 2 * R / 0.85)) + rng.uniform(-0.3 * R, 0.3 * R, g.shape)
+    if clump:
+        x[: n // 2] = 0.06 + 0.55 * (x[: n // 2] - 0.06)
+        x[n // 3 : n // 3 + 2] = x[0]
+    return x.astype(np.float32), rng.normal(0.0, 0.4, g.shape).astype(np.float32)
+
+
+def run(x, v, xb, cfg, shapes):
+    f = ws.ParticleStore(len(x))
+    f.resize(len(x))
+    f.set_positions(x)
+    f.set_velocities(v)
+    b = None
+    if xb is not None:
+        b = ws.ParticleStore(len(xb))
+        b.resize(len(xb))
+        b.set_positions(xb)
+    s = ws.DFSPHSolver(f, b, ws.DFSPHConfig(**cfg))
+    if shapes:
+        s.set_shapes(**shapes)
+    for _ in range(2):
+        s.step(5e-4)
+    out = {k: f.get_attribute(k) for k in FIELDS}
+    out.update(x=f.get_positions(), v=f.get_velocities())
+    st = s.stats()
+    s.close()
+    return out, st
+
+
+@pytest.mark.parametrize("fast", [False, True], ids=["exact", "fast"])
+@pytest.mark.parametrize("n,clump,walls,over", [
+    (1, False, True, {}),
+    (17, False, False, dict(pressure_form=1)),
+    (63, True, True, {}),
+    (257, True, True, dict(pressure_form=1, enable_divergence_solve=True)),
+    (4000, True, False, {}),
+    (40960, False, True, dict(pressure_form=1)),   # the limits and one tile more
+    (40961, False, True, dict(pressure_form=1)),
+    (65536, False, True, dict(pressure_form=1)),
+    (65537, False, True, dict(pressure_form=1)),
+    (98305, False, True, dict(pressure_form=1)),
+    (131073, False, True, dict(pressure_form=1)),
+])
+def test_four_lanes_equal_one_lane(n, clump, walls, over, fast):
+    x, v = cloud(n, clump)
+    xb = O.sample_aabb_boundary([0, 0, 0], [1, 1, 1], 2 * R, 3) if walls else None
+    cfg = dict(rest_density=1000.0, particle_radius=R, smoothing_length=2 * R, viscosity=0.01,
+               damping=0.5, domain_min=(0, 0, 0), domain_max=(1, 1, 1), max_density_iters=6,
+               max_divergence_iters=4, eta_density=1e-3, fast_math=fast)
+    cfg.update(over)
+    a, sa = run(x, v, xb, cfg, None)
+    b, sb = run(x, v, xb, cfg, ONE_LANE)
+    for k in b:
+        assert_bitexact(a[k], b[k], k)
+    for k in ("density_iters", "divergence_iters", "mean_density_error", "max_velocity"):
+        assert sa[k] == sb[k], (k, sa, sb)

@@ -1064,12 +1064,22 @@ __global__ __launch_bounds__(kTile) void k_change_st(Nbr P, PairList L,
 // partials written by k_change(iter), in a fixed order, and records the
 // error and the convergence decision (dfsph.cu:254-258; the divergence solve
 // tests every iteration).
+// quarters: part holds the four wave sums of every tile (k_change_q).
 __device__ __forceinline__ void finish_error(int mode, u32 iter, double thr, const SceneSeg& G,
-                                             const double* __restrict__ part, DeviceState* st) {
+                                             const double* __restrict__ part, int quarters,
+                                             DeviceState* st) {
     const int lane = threadIdx.x & 63;
     double s = 0.0;
+    if (quarters) {
+#pragma unroll 4
+        for (u32 t = lane; t < G.ntiles; t += 64) {
+            const double4 q = reinterpret_cast<const double4*>(part)[G.tile0 + t];
+            s += ((q.x + q.y) + q.z) + q.w;
+        }
+    } else {
 #pragma unroll 8
-    for (u32 t = lane; t < G.ntiles; t += 64) s += part[G.tile0 + t];
+        for (u32 t = lane; t < G.ntiles; t += 64) s += part[G.tile0 + t];
+    }
     const double tot = wave_sum(s);
     if (lane == 0) {
         const double e = tot / static_cast<double>(G.n);
@@ -1109,8 +1119,8 @@ template <int NT, int PU, bool F>
 __global__ __launch_bounds__(NT) void k_apply(Nbr P, PairList L, const float4* __restrict__ xk,
                                               const float* __restrict__ kappa, float rho0,
                                               int pform, u32 iter, int mode, double thr,
-                                              const double* __restrict__ part, DeviceState* st,
-                                              const float4* vin, float4* vout) {
+                                              const double* __restrict__ part, int quarters,
+                                              DeviceState* st, const float4* vin, float4* vout) {
     const u32 i = slot_index<NT>(P.remap);
     if (i >= P.nslots) return;
     const u32 sc = scene_of_slot(P, i);
@@ -1119,7 +1129,7 @@ __global__ __launch_bounds__(NT) void k_apply(Nbr P, PairList L, const float4* _
     if (conv < iter) return;  // scene-uniform: this iteration's k_change did not run either
     const SceneSeg& G = P.seg[sc];
     const u32 l = i - G.off;
-    if (l < 64) finish_error(mode, iter, thr, G, part, sst);
+    if (l < 64) finish_error(mode, iter, thr, G, part, quarters, sst);
     if (l >= G.n) return;
     const u32* cs = P.csf + G.key_base;
     const u32 shift = G.off - G.start;
@@ -1226,7 +1236,7 @@ __global__ __launch_bounds__(kTile) void k_apply_st(Nbr P, PairList L,
                                                     const float4* __restrict__ xk,
                                                     const float* __restrict__ kappa, float rho0,
                                                     int pform, u32 iter, int mode, double thr,
-                                                    const double* __restrict__ part,
+                                                    const double* __restrict__ part, int quarters,
                                                     DeviceState* st, const float4* vin,
                                                     float4* vout) {
     __shared__ float4 s_x[kStageCap];
@@ -1257,7 +1267,7 @@ __global__ __launch_bounds__(kTile) void k_apply_st(Nbr P, PairList L,
     __syncthreads();
     const bool staged = R.total != 0;
     const u32 l = i - G.off;
-    if (l < 64) finish_error(mode, iter, thr, G, part, sst);
+    if (l < 64) finish_error(mode, iter, thr, G, part, quarters, sst);
     if (l >= G.n) return;
     const u32* cs = P.csf + G.key_base;
     const u32 shift = G.off - G.start;
@@ -1958,12 +1968,675 @@ __global__ void k_frame_begin(FrameParams fp, FrameParams* __restrict__ dst,
     cfl_step(fp, seg[0], *st);
 }
 
+// ---- four lanes per particle ------------------------------------------------
+// Scenes that do not fill the card (quad_limits) are bound by the serial
+// walk of one lane over its particle's pairs: a pair is a dependent chain of a
+// gather, a square root and two quotients, and 256 CUs hold a workgroup or
+// less each.  Here the four lanes of a quad share a particle: lane g loads and
+// evaluates entries g, g + 4, ... , so four pairs run side by side and four
+// times the waves hide each other's latency.  The terms are then added in
+// list order, each broadcast from its lane by a DPP quad permutation, so every
+// sum rounds exactly as the one-lane kernels' sums do.  Neighbours come
+// straight from L2 (the whole scene fits there), without a staging round or a
+// barrier.  Every branch around a broadcast is uniform in a quad.
+constexpr int kQuad = 4;
+constexpr u32 kQuadGroup = NS / kQuad;  // slots of a 256-thread workgroup
+
+template <int K>
+__device__ __forceinline__ float quad_get(float v) {
+    return __int_as_float(
+        __builtin_amdgcn_mov_dpp(__float_as_int(v), K * 0x55, 0xF, 0xF, true));
+}
+template <int K>
+__device__ __forceinline__ u32 quad_get(u32 v) {
+    return static_cast<u32>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), K * 0x55, 0xF, 0xF, true));
+}
+// acc + t of lane 0, then of lane 1, 2, 3
+__device__ __forceinline__ void quad_add(float& acc, float t) {
+    acc += quad_get<0>(t);
+    acc += quad_get<1>(t);
+    acc += quad_get<2>(t);
+    acc += quad_get<3>(t);
+}
+__device__ __forceinline__ void quad_sub(float& acc, float t) {
+    acc -= quad_get<0>(t);
+    acc -= quad_get<1>(t);
+    acc -= quad_get<2>(t);
+    acc -= quad_get<3>(t);
+}
+// acc = fma(a, b, acc) with the a and b of lane 0, then of lane 1, 2, 3
+__device__ __forceinline__ void quad_fma(float& acc, float a, float b) {
+    acc = __builtin_fmaf(quad_get<0>(a), quad_get<0>(b), acc);
+    acc = __builtin_fmaf(quad_get<1>(a), quad_get<1>(b), acc);
+    acc = __builtin_fmaf(quad_get<2>(a), quad_get<2>(b), acc);
+    acc = __builtin_fmaf(quad_get<3>(a), quad_get<3>(b), acc);
+}
+
+// This lane's slot and place in its quad.
+struct QuadLane {
+    u32 i, g;
+    __device__ __forceinline__ explicit QuadLane(const Nbr& P) {
+        const u32 b = P.remap ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
+        i = b * kQuadGroup + (threadIdx.x >> 2);
+        g = threadIdx.x & 3u;
+    }
+};
+
+// The first kQuadHead quads of a particle's fluid list, requested before its
+// length is known (the list's storage always holds them), so the entries
+// arrive with the particle's own data.
+constexpr int kQuadHead = 8;
+static_assert(kQuadHead * kQuad <= kPairDepthFluid, "list storage of the head");
+struct QuadHead {
+    u32 e[kQuadHead];    // staged entry, or slot
+    float c[kQuadHead];  // recorded factor (tiles without a staging plan)
+    __device__ __forceinline__ QuadHead(const PairList& L, const StageRanges& R, u32 i, u32 g) {
+        if (R.total) {
+#pragma unroll
+            for (int u = 0; u < kQuadHead; ++u) {
+                e[u] = L.fi[stage_entry_at(4u * u + g, i, L.kf)];
+                c[u] = 0.0f;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < kQuadHead; ++u) {
+                const uint2 w = L.f[pair_at(4u * u + g, i, L.kf)];
+                e[u] = w.x;
+                c[u] = __uint_as_float(w.y);
+            }
+        }
+    }
+    __device__ __forceinline__ u32 slot(const StageRanges& R, int u, bool valid, u32 i) const {
+        return valid ? (R.total ? stage_source(R, e[u]) : e[u]) : i;
+    }
+};
+// Visits the fluid list of particle i by quads: load(n, u, slot) requests the
+// data of a lane's entry u of a batch of n, use(u, c, valid) adds its term.
+// Lanes past the list's end load their own particle and pass valid = false.
+template <class Ld, class Us>
+__device__ __forceinline__ void for_quads(const PairList& L, const StageRanges& R,
+                                          const QuadHead& H, u32 i, u32 g, u32 cf, Ld&& load,
+                                          Us&& use) {
+    const u32 nq = (cf + 3u) >> 2;
+    constexpr int kHalf = kQuadHead / 2;
+    const bool more = __any(nq > kHalf);  // wave-uniform
+#pragma unroll
+    for (int u = 0; u < kHalf; ++u) load(u, H.slot(R, u, 4u * u + g < cf, i));
+    if (more) {
+#pragma unroll
+        for (int u = kHalf; u < kQuadHead; ++u) load(u, H.slot(R, u, 4u * u + g < cf, i));
+    }
+#pragma unroll
+    for (int u = 0; u < kHalf; ++u) use(u, H.c[u], 4u * u + g < cf);
+    if (!more) return;
+#pragma unroll
+    for (int u = kHalf; u < kQuadHead; ++u) use(u, H.c[u], 4u * u + g < cf);
+    for (u32 q = kQuadHead; q < nq; ++q) {
+        const u32 k = 4u * q + g;
+        const bool valid = k < cf;
+        u32 j = i;
+        float c = 0.0f;
+        if (valid) fluid_entry(L, R, k, i, j, c);
+        load(0, j);
+        use(0, c, valid);
+    }
+}
+
+// The boundary list by quads: use(q, c, valid) with the boundary particle q.
+template <class Us>
+__device__ __forceinline__ void for_quads_boundary(const Nbr& P, const PairList& L, u32 i, u32 g,
+                                                   u32 cb, Us&& use) {
+    constexpr int kB = 4;
+    for (u32 q0 = 0; q0 < ((cb + 3u) >> 2); q0 += kB) {
+        uint2 e[kB];
+        float4 x[kB];
+#pragma unroll
+        for (int u = 0; u < kB; ++u) {
+            const u32 k = 4u * (q0 + u) + g;
+            e[u] = make_uint2(0u, 0u);
+            if (k < cb) e[u] = L.b[pair_at(k, i, L.kb)];
+        }
+#pragma unroll
+        for (int u = 0; u < kB; ++u) x[u] = P.xb[e[u].x];
+#pragma unroll
+        for (int u = 0; u < kB; ++u)
+            use(x[u], __uint_as_float(e[u].y), 4u * (q0 + u) + g < cb);
+    }
+}
+
+// k_xsph_st's sums, four lanes per particle.
+template <bool F>
+__global__ __launch_bounds__(NS) void k_xsph_q(Nbr P, PairList L, const float4* __restrict__ xs,
+                                               const float4* __restrict__ vin,
+                                               const float* __restrict__ rho,
+                                               float4* __restrict__ vout) {
+    const QuadLane Q(P);
+    const u32 i = Q.i, g = Q.g;
+    const SceneSeg& G = P.seg[scene_of_slot(P, i)];
+    const float eps = G.eps;
+    const float4 vi = vin[i];
+    const u32 l = i - G.off;
+    if (!(eps > 0.0f)) {  // scene-uniform
+        if (l < G.n && g == 0) vout[i] = vi;
+        return;
+    }
+    const StageRanges R = L.plan[i / kTile];
+    const float4 p = xs[i];
+    const float rho_i = rho[i];
+    const u32 cf = L.cnt[i] & 0xFFFFu;
+    const QuadHead H(L, R, i, g);
+    if (l >= G.n) return;
+    float dx = 0.0f, dy = 0.0f, dz = 0.0f;
+    if (cf <= L.kf) {
+        float tx = 0.0f, ty = 0.0f, tz = 0.0f;  // tolerance mode: see xsph_listed
+        float4 q[kQuadHead], w[kQuadHead];
+        float rj[kQuadHead];
+        for_quads(
+            L, R, H, i, g, cf,
+            [&](int u, u32 j) {
+                q[u] = xs[j];
+                w[u] = vin[j];
+                rj[u] = rho[j];
+            },
+            [&](int u, float, bool valid) {
+                if (F) {
+                    const float r2 =
+                        PairMath<true>::r2(p.x - q[u].x, p.y - q[u].y, p.z - q[u].z);
+                    const float s = r2 * __builtin_amdgcn_rsqf(r2) * P.sp.inv_l;
+                    const float inner =
+                        __builtin_fmaf(s * s, __builtin_fmaf(0.75f, s, -1.5f), 1.0f);
+                    const float t = 2.0f - s;
+                    const float wv = s < 1.0f ? inner : 0.25f * (t * t * t);
+                    const float k =
+                        valid ? wv * __builtin_amdgcn_rcpf(fmaxf(rho_i + rj[u], 2.0f * 1e-9f))
+                              : 0.0f;
+                    quad_fma(tx, k, w[u].x - vi.x);
+                    quad_fma(ty, k, w[u].y - vi.y);
+                    quad_fma(tz, k, w[u].z - vi.z);
+                } else {
+                    float ax = -0.0f, ay = -0.0f, az = -0.0f;  // adding -0.0f: no change
+                    xsph_term<false>(ax, ay, az, p, vi, rho_i, q[u], w[u], rj[u], eps, P, valid);
+                    quad_add(dx, ax);
+                    quad_add(dy, ay);
+                    quad_add(dz, az);
+                }
+            });
+        xsph_listed_scale<F>(dx, dy, dz, tx, ty, tz, eps, P);
+    } else {
+        for_stencil(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, [&](u32 s) {
+            if (s == i) return;
+            const float4 q = xs[s];
+            const float r2 = PairMath<F>::r2(p.x - q.x, p.y - q.y, p.z - q.z);
+            if (r2 >= P.sp.far2) return;  // W = 0
+            xsph_term_r2<F>(dx, dy, dz, r2, vi, rho_i, vin[s], rho[s], eps, P);
+        });
+    }
+    if (g == 0) vout[i] = make_float4(vi.x + dx, vi.y + dy, vi.z + dz, 0.0f);
+}
+
+// k_change_st's sums, four lanes per particle.  Writes one error partial per
+// 64 slots, the wave sum that the one-lane kernels add up per tile
+// (finish_error's `quarters`).
+template <int MODE, bool F>
+__global__ __launch_bounds__(NS) void k_change_q(Nbr P, PairList L, const float4* __restrict__ xs,
+                                                 const float4* __restrict__ vs,
+                                                 const float* __restrict__ rho,
+                                                 const float* __restrict__ alpha, float rho0,
+                                                 int pform, u32 iter, const DeviceState* st,
+                                                 double* __restrict__ part,
+                                                 float* __restrict__ rho_adv,
+                                                 float* __restrict__ kappa,
+                                                 float4* __restrict__ xk) {
+    __shared__ double s_err[kQuadGroup];
+    const QuadLane Q(P);
+    const u32 i = Q.i, g = Q.g;
+    const u32 sc = scene_of_slot(P, i);
+    const StageRanges R = L.plan[i / kTile];
+    const u32 conv = MODE == 0 ? st[sc].conv_iter : st[sc].div_conv_iter;
+    if (conv < iter) return;  // the whole workgroup belongs to one scene
+    const SceneSeg& G = P.seg[sc];
+    // slots [0, nslots) are allocated
+    const float4 p = xs[i];
+    const float4 vi = vs[i];
+    const float rho_i = rho[i];
+    const float alpha_i = alpha[i];
+    const u32 cw = L.cnt[i];
+    const QuadHead H(L, R, i, g);
+    double contrib = 0.0;
+    if (i - G.off < G.n) {
+        float rd = 0.0f;
+        // tolerance mode: the fluid terms sum c (u . r) in rf, times m once
+        float rf = 0.0f;
+        const u32 cf = cw & 0xFFFFu, cb = cw >> 16;
+        if (cf <= L.kf && cb <= L.kb) {
+            float4 q[kQuadHead];
+            float4 w[kQuadHead];
+            for_quads(
+                L, R, H, i, g, cf,
+                [&](int u, u32 j) {
+                    q[u] = xs[j];
+                    w[u] = vs[j];
+                },
+                [&](int u, float c0, bool valid) {
+                    const float c = R.total ? pair_c_listed<F>(p, q[u], P.sp) : c0;
+                    const float ux = vi.x - w[u].x, uy = vi.y - w[u].y, uz = vi.z - w[u].z;
+                    if (F) {
+                        const float dot = __builtin_fmaf(
+                            ux, p.x - q[u].x,
+                            __builtin_fmaf(uy, p.y - q[u].y, uz * (p.z - q[u].z)));
+                        quad_fma(rf, valid ? c : 0.0f, dot);
+                    } else {
+                        const float gx = (p.x - q[u].x) * c, gy = (p.y - q[u].y) * c,
+                                    gz = (p.z - q[u].z) * c;
+                        quad_add(rd, valid ? P.mass * (ux * gx + uy * gy + uz * gz) : -0.0f);
+                    }
+                });
+            for_quads_boundary(P, L, i, g, cb, [&](const float4& q, float c, bool valid) {
+                if (F) {
+                    const float dot = __builtin_fmaf(
+                        vi.x, p.x - q.x, __builtin_fmaf(vi.y, p.y - q.y, vi.z * (p.z - q.z)));
+                    quad_fma(rd, valid ? q.w * c : 0.0f, valid ? dot : 0.0f);
+                } else {
+                    const float gx = (p.x - q.x) * c, gy = (p.y - q.y) * c, gz = (p.z - q.z) * c;
+                    quad_add(rd, valid ? q.w * (vi.x * gx + vi.y * gy + vi.z * gz) : -0.0f);
+                }
+            });
+        } else {
+            float& racc = F ? rf : rd;
+            const float mf = F ? 1.0f : P.mass;
+            for_stencil(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, [&](u32 s) {
+                if (s == i) return;
+                const float4 q = xs[s];
+                const float r2 = PairMath<F>::r2(p.x - q.x, p.y - q.y, p.z - q.z);
+                if (r2 >= P.sp.far2) return;
+                rho_dot_fluid<F>(racc, p, vi, q, vs[s], stencil_c<F>(r2, P.sp), mf);
+            });
+            if (P.nb && !(F && L.gb)) {
+                for_stencil(P.gb, P.csb, 0u, p.x, p.y, p.z, [&](u32 s) {
+                    const float4 q = P.xb[s];
+                    const float r2 = PairMath<F>::r2(p.x - q.x, p.y - q.y, p.z - q.z);
+                    if (r2 >= P.sp.far2) return;
+                    rho_dot_boundary<F>(rd, p, vi, q, stencil_c<F>(r2, P.sp));
+                });
+            }
+        }
+        if (F) rd = __builtin_fmaf(P.mass, rf, rd);
+        if (F && L.gb) rd += dot_gb(vi, L.gb[i]);
+        float kap, err, adv;
+        if (MODE == 0) {
+            adv = rho_i + G.dt * rd;
+            err = fmaxf(0.0f, adv - rho0);
+            kap = err * alpha_i / G.dt2;
+        } else {
+            adv = rd;
+            err = fmaxf(0.0f, rd);
+            kap = err * alpha_i / G.dt;
+        }
+        const float khat = pform ? kap / fmaxf(rho_i, 1e-9f) : kap / fmaxf(rho_i * rho_i, 1e-9f);
+        if (g == 0) {
+            rho_adv[i] = adv;
+            kappa[i] = kap;
+            xk[i] = make_float4(p.x, p.y, p.z, khat);
+        }
+        contrib = static_cast<double>(err);
+    }
+    if (g == 0) s_err[threadIdx.x >> 2] = contrib;
+    __syncthreads();
+    if (threadIdx.x < 64) {  // the wave sum of the group's 64 slots
+        const double ws = wave_sum(s_err[threadIdx.x]);
+        if (threadIdx.x == 0) part[i / kQuadGroup] = ws;
+    }
+}
+
+// k_apply_st's sums, four lanes per particle.
+template <bool F>
+__global__ __launch_bounds__(NS) void k_apply_q(Nbr P, PairList L, const float4* __restrict__ xk,
+                                                const float* __restrict__ kappa, float rho0,
+                                                int pform, u32 iter, int mode, double thr,
+                                                const double* __restrict__ part, int quarters,
+                                                DeviceState* st, const float4* vin, float4* vout) {
+    const QuadLane Q(P);
+    const u32 i = Q.i, g = Q.g;
+    const u32 sc = scene_of_slot(P, i);
+    DeviceState* sst = st + sc;
+    const StageRanges R = L.plan[i / kTile];
+    const u32 conv = mode == 0 ? sst->conv_iter : sst->div_conv_iter;
+    if (conv < iter) return;  // the whole workgroup belongs to one scene
+    const SceneSeg& G = P.seg[sc];
+    const float4 p = xk[i];
+    const float4 v0 = vin[i];
+    const u32 cw = L.cnt[i];
+    const float k_i = kappa[i];
+    const QuadHead H(L, R, i, g);
+    const u32 l = i - G.off;
+    if (l < 64 / kQuad) finish_error(mode, iter, thr, G, part, quarters, sst);  // one wave
+    if (l >= G.n) return;
+    const float dt = G.dt;
+    const float ki = p.w;
+    float dx = 0.0f, dy = 0.0f, dz = 0.0f;
+    // tolerance mode: the fluid terms sum -(k_i + k_j) c r in a, times dt m once
+    float ax = 0.0f, ay = 0.0f, az = 0.0f;
+    auto mk = [&](float kj) { return F ? ki + kj : P.mass * (ki + kj); };
+    float bf = 0.0f;
+    if (P.nb) bf = pform ? k_i / fmaxf(rho0, 1e-9f) : k_i / fmaxf(rho0 * rho0, 1e-9f);
+    // one term of kappa_term from each lane, in lane order
+    auto add = [&](float& sx, float& sy, float& sz, const float4& q, float c, float c2, float h,
+                   bool valid) {
+        const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
+        if (F) {
+            const float k = valid ? -(h * c2 * c) : 0.0f;
+            quad_fma(sx, k, rx);
+            quad_fma(sy, k, ry);
+            quad_fma(sz, k, rz);
+        } else {
+            const float gx = rx * c, gy = ry * c, gz = rz * c;
+            quad_sub(sx, valid ? h * c2 * gx : 0.0f);  // subtracting +0.0f: no change
+            quad_sub(sy, valid ? h * c2 * gy : 0.0f);
+            quad_sub(sz, valid ? h * c2 * gz : 0.0f);
+        }
+    };
+    float& fx = F ? ax : dx;
+    float& fy = F ? ay : dy;
+    float& fz = F ? az : dz;
+    const float fdt = F ? 1.0f : dt;
+    const u32 cf = cw & 0xFFFFu, cb = cw >> 16;
+    if (cf <= L.kf && cb <= L.kb) {
+        float4 q[kQuadHead];
+        for_quads(
+            L, R, H, i, g, cf, [&](int u, u32 j) { q[u] = xk[j]; },
+            [&](int u, float c0, bool valid) {
+                const float c = R.total ? pair_c_listed<F>(p, q[u], P.sp) : c0;
+                add(fx, fy, fz, q[u], c, mk(q[u].w), fdt, valid);
+            });
+        for_quads_boundary(P, L, i, g, cb, [&](const float4& b, float c, bool valid) {
+            add(dx, dy, dz, b, c, b.w * (ki + bf), dt, valid);
+        });
+    } else {
+        for_stencil(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, [&](u32 s) {
+            if (s == i) return;
+            const float4 b = xk[s];
+            const float r2 = PairMath<F>::r2(p.x - b.x, p.y - b.y, p.z - b.z);
+            if (r2 >= P.sp.far2) return;
+            kappa_term<F>(fx, fy, fz, p, b, stencil_c<F>(r2, P.sp), mk(b.w), fdt);
+        });
+        if (P.nb && !(F && L.gb)) {
+            for_stencil(P.gb, P.csb, 0u, p.x, p.y, p.z, [&](u32 s) {
+                const float4 b = P.xb[s];
+                const float r2 = PairMath<F>::r2(p.x - b.x, p.y - b.y, p.z - b.z);
+                if (r2 >= P.sp.far2) return;
+                kappa_term<F>(dx, dy, dz, p, b, stencil_c<F>(r2, P.sp), b.w * (ki + bf), dt);
+            });
+        }
+    }
+    if (F) {
+        const float s = dt * P.mass;
+        dx = __builtin_fmaf(s, ax, dx);
+        dy = __builtin_fmaf(s, ay, dy);
+        dz = __builtin_fmaf(s, az, dz);
+    }
+    if (F && L.gb) {  // sum_b m_b (k_i + k_b) grad W_ib = (k_i + k_b) Gb_i
+        const float4 b = L.gb[i];
+        const float k = -(dt * (ki + bf));
+        dx = __builtin_fmaf(k, b.x, dx);
+        dy = __builtin_fmaf(k, b.y, dy);
+        dz = __builtin_fmaf(k, b.z, dz);
+    }
+    if (g == 0) vout[i] = make_float4(v0.x + dx, v0.y + dy, v0.z + dz, v0.w);
+}
+
+// k_density_alpha's sums, four lanes per particle.  The one-lane walk visits
+// a particle's ~27 candidates one after the other, each a gather and about a
+// hundred operations behind the loop tests of nine rows.  Here the quad first
+// writes its candidates' slots to LDS in the walk's order (each lane the rows
+// g, g + 4, g + 8, its place from the row counts), then takes four at a time.
+// A window of kCand slots holds most stencils; larger ones take several.
+constexpr u32 kCand = 64;
+constexpr u32 kCandStride = kCand + kQuad;  // quads of a wave on different banks
+constexpr u32 kCandRow = 30;                // a candidate: slot, x offset above bit 30
+
+// rows: 9 rows of up to three ranges [b, e) of sorted slots, visited in order
+// (row, range); lane g holds the rows g + 4 t as b[t][k], e[t][k].
+template <int NR>
+struct QuadRows {
+    u32 b[3][NR], e[3][NR];
+    u32 base[3];  // candidates before the row
+    u32 total;
+    __device__ __forceinline__ void count(u32 g) {
+        total = 0;
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            u32 n = 0;
+#pragma unroll
+            for (int k = 0; k < NR; ++k) n += e[t][k] - b[t][k];
+            const u32 n0 = quad_get<0>(n), n1 = quad_get<1>(n), n2 = quad_get<2>(n),
+                      n3 = quad_get<3>(n);
+            base[t] = total + (g > 0 ? n0 : 0u) + (g > 1 ? n1 : 0u) + (g > 2 ? n2 : 0u);
+            total += n0 + n1 + n2 + n3;
+        }
+    }
+};
+// The stencil of for_stencil_rows (F false: rows (dz, dy), ranges dx) or of
+// for_stencil_zrows (F true: rows (dx, dy), one range over dz).
+template <bool F>
+__device__ __forceinline__ QuadRows<F ? 1 : 3> quad_rows(const GridGeom& gg,
+                                                         const u32* __restrict__ cs, u32 g,
+                                                         float px, float py, float pz) {
+    constexpr int NR = F ? 1 : 3;
+    QuadRows<NR> W;
+    const int cx = gg.cx(px), cy = gg.cy(py), cz = gg.cz(pz);
+    const int lo = cz - 1 < 0 ? 0 : cz - 1;
+    const int hi = cz + 1 > gg.dz - 1 ? gg.dz - 1 : cz + 1;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+        const int r = static_cast<int>(g) + 4 * t;
+        const int a = r / 3 - 1, ny = cy + r % 3 - 1;
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const int nx = F ? cx + a : cx + k - 1;
+            const int z0 = F ? lo : cz + a, z1 = F ? hi : cz + a;
+            const bool in = r < 9 && nx >= 0 && nx < gg.dx && ny >= 0 && ny < gg.dy && z0 >= 0 &&
+                            z1 < gg.dz && z0 <= z1;
+            const u32 row = (static_cast<u32>(nx) * static_cast<u32>(gg.dy) +
+                             static_cast<u32>(ny)) * static_cast<u32>(gg.dz);
+            const u32 bk = cs[in ? row + static_cast<u32>(z0) : 0u];
+            const u32 ek = cs[in ? row + static_cast<u32>(z1) + 1u : 0u];
+            W.b[t][k] = in ? bk : 0u;
+            W.e[t][k] = in ? ek : 0u;
+        }
+    }
+    W.count(g);
+    return W;
+}
+// Visits the candidates by fours: use(valid, slot, xk, q) with the slot, its x
+// offset (dx + 1) and its position; lanes past the end get valid = false.
+template <bool F, class Us>
+__device__ __forceinline__ void for_candidates(const QuadRows<F ? 1 : 3>& W, u32* cand, u32 g,
+                                               u32 shift, const float4* __restrict__ x, Us&& use) {
+    for (u32 w0 = 0; w0 < W.total; w0 += kCand) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            u32 pos = W.base[t] - w0;  // wraps below the window: the test fails
+            const u32 rk = (g + 4u * t) / 3u;
+#pragma unroll
+            for (int k = 0; k < (F ? 1 : 3); ++k)
+                for (u32 s = W.b[t][k]; s < W.e[t][k]; ++s, ++pos)
+                    if (pos < kCand)
+                        cand[pos] = (s + shift) | ((F ? rk : static_cast<u32>(k)) << kCandRow);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const u32 n = min(W.total - w0, kCand);
+        constexpr int U = 4;
+        for (u32 q0 = 0; q0 < n; q0 += 4 * U) {
+            u32 s[U];
+            float4 q[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const u32 k = q0 + 4u * u + g;
+                s[u] = cand[k < n ? k : 0u];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) q[u] = x[s[u] & ((1u << kCandRow) - 1u)];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                use(q0 + 4u * u + g < n, s[u] & ((1u << kCandRow) - 1u), s[u] >> kCandRow, q[u]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+}
+
+// Sums of grad_terms over the quad's four pairs in lane order; a lane without
+// a pair passes wv = mx = my = mz = 0 of the sign that changes nothing.
+template <bool F>
+__device__ __forceinline__ void quad_grad_terms(float& rho, float& sx, float& sy, float& sz,
+                                                float& sq, bool in, float m, float wv, float c,
+                                                float rx, float ry, float rz) {
+    if (F) {
+        const float mc = m * c;
+        const float mx = in ? rx * mc : -0.0f, my = in ? ry * mc : -0.0f,
+                    mz = in ? rz * mc : -0.0f;
+        quad_fma(rho, in ? m : 0.0f, in ? wv : 0.0f);
+        quad_add(sx, mx);
+        quad_add(sy, my);
+        quad_add(sz, mz);
+        auto sq_of = [&](float a, float b, float d) {
+            sq = __builtin_fmaf(a, a, __builtin_fmaf(b, b, __builtin_fmaf(d, d, sq)));
+        };
+        sq_of(quad_get<0>(mx), quad_get<0>(my), quad_get<0>(mz));
+        sq_of(quad_get<1>(mx), quad_get<1>(my), quad_get<1>(mz));
+        sq_of(quad_get<2>(mx), quad_get<2>(my), quad_get<2>(mz));
+        sq_of(quad_get<3>(mx), quad_get<3>(my), quad_get<3>(mz));
+    } else {
+        const float mx = m * (rx * c), my = m * (ry * c), mz = m * (rz * c);
+        quad_add(rho, in ? m * wv : -0.0f);
+        quad_add(sx, in ? mx : -0.0f);
+        quad_add(sy, in ? my : -0.0f);
+        quad_add(sz, in ? mz : -0.0f);
+        quad_add(sq, in ? mx * mx + my * my + mz * mz : -0.0f);
+    }
+}
+
+template <bool F>
+__global__ __launch_bounds__(NS) void k_density_alpha_q(Nbr P, PairList L,
+                                                        const float4* __restrict__ xs,
+                                                        float* __restrict__ rho_out,
+                                                        float* __restrict__ alpha_out,
+                                                        DeviceState* open) {
+    __shared__ u32 s_cand[kQuadGroup * kCandStride];
+    if (open && blockIdx.x == 0 && threadIdx.x == 0 && open->advected) {
+        open->conv_iter = P.seg[0].n ? kNone : 0u;
+        open->advected = 0u;
+    }
+    const QuadLane Q(P);
+    const u32 i = Q.i, g = Q.g;
+    const SceneSeg& G = P.seg[scene_of_slot(P, i)];
+    const float4 p = xs[i];
+    if (i - G.off >= G.n) return;
+    u32* const cand = s_cand + (threadIdx.x >> 2) * kCandStride;
+    const u32 below = (1u << g) - 1u;
+    const u32 quad0 = threadIdx.x & 60u;  // first lane of the quad in its wave
+    float rho = 0.0f, sx = 0.0f, sy = 0.0f, sz = 0.0f, sq = 0.0f;
+    u32 cf = 0, cb = 0;
+    bool unlisted = false;  // an in-support fluid pair with a zero gradient
+    const StageRanges R = L.plan[i / kTile];
+    const bool staged = R.total != 0u;
+    const StageOffsets O(R);
+    uint16_t* const fi = L.fi + stage_entry_at(0u, i, L.kf);
+    uint2* const f8 = L.f + pair_at(0u, i, L.kf);
+    for_candidates<F>(
+        quad_rows<F>(P.gf, P.csf + G.key_base, g, p.x, p.y, p.z), cand, g, G.off - G.start, xs,
+        [&](bool valid, u32 s, u32 xk, const float4& q) {
+            const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
+            const float r2 = PairMath<F>::r2(rx, ry, rz);
+            const bool in = valid && !(r2 >= P.sp.far2);  // else W = 0 and c = 0
+            float wv, c;
+            PairMath<F>::wc(in ? r2 : 0.0f, P.sp, wv, c);
+            quad_grad_terms<F>(rho, sx, sy, sz, sq, in, P.mass, wv, c, rx, ry, rz);
+            // the self pair (d = 0) has c = 0 and is not listed
+            const bool list = in && c != 0.0f;
+            const u32 m = static_cast<u32>(__ballot(list) >> quad0) & 15u;
+            if (list) {
+                const u32 k = cf + static_cast<u32>(__popc(m & below));
+                if (k < L.kf) {
+                    const u32 e = s + (xk == 0u ? O.off[0] : xk == 1u ? O.off[1] : O.off[2]);
+                    if (staged) fi[((k >> 2) << 8) | (k & 3u)] = static_cast<uint16_t>(e);
+                    else f8[k << 6] = make_uint2(s, __float_as_uint(c));
+                }
+            } else if (in && s != i) {
+                unlisted = true;
+            }
+            cf += static_cast<u32>(__popc(m));
+        });
+    // a pair the list leaves out sends this particle to the stencil walk
+    if ((static_cast<u32>(__ballot(unlisted) >> quad0) & 15u) != 0u) cf = 0xFFFFu;
+    float gbx = 0.0f, gby = 0.0f, gbz = 0.0f;  // tolerance mode: sum_b m_b grad W_ib
+    if (P.nb && boundary_near(P.gb, P.bnear, p.x, p.y, p.z)) {
+        for_candidates<F>(
+            quad_rows<F>(P.gb, P.csb, g, p.x, p.y, p.z), cand, g, 0u, P.xb,
+            [&](bool valid, u32 s, u32, const float4& q) {
+                const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
+                const float r2 = PairMath<F>::r2(rx, ry, rz);
+                const bool in = valid && !(r2 >= P.sp.far2);
+                float wv, c;
+                PairMath<F>::wc(in ? r2 : 0.0f, P.sp, wv, c);
+                quad_grad_terms<F>(rho, sx, sy, sz, sq, in, q.w, wv, c, rx, ry, rz);
+                if (F && L.gb) {
+                    const float mc = in ? q.w * c : 0.0f;
+                    quad_fma(gbx, rx, mc);
+                    quad_fma(gby, ry, mc);
+                    quad_fma(gbz, rz, mc);
+                } else {
+                    const bool list = in && c != 0.0f;
+                    const u32 m = static_cast<u32>(__ballot(list) >> quad0) & 15u;
+                    const u32 k = cb + static_cast<u32>(__popc(m & below));
+                    if (list && k < L.kb) L.b[pair_at(k, i, L.kb)] = make_uint2(s, __float_as_uint(c));
+                    cb += static_cast<u32>(__popc(m));
+                }
+            });
+    }
+    if (g != 0) return;
+    if (F && L.gb) L.gb[i] = make_float4(gbx, gby, gbz, 0.0f);
+    L.cnt[i] = pack_counts(cf, cb);
+    rho_out[i] = rho;
+    const float denom = F ? __builtin_fmaf(sx, sx, __builtin_fmaf(sy, sy, __builtin_fmaf(sz, sz, sq)))
+                          : sx * sx + sy * sy + sz * sz + sq;
+    alpha_out[i] = (denom > 1e-9f) ? (rho / denom) : 0.0f;
+}
+
 // ---- launch-shape dispatch ------------------------------------------------
 u32 grid_for(u32 nslots, u32 nt) { return div_up(nslots, nt); }
+
+// Working slots up to which the default shapes (0, and 256 threads for
+// density/alpha) take the four-lane kernels.  Where the chip is idle they
+// shorten a lane's serial chain; once every CU holds several workgroups the
+// staged kernels move fewer bytes per pair.  Measured per launch (stirred
+// block with walls, us, one lane -> four lanes):
+//   exact   density  4k 50.7 -> 15.6   65k 46.0 -> 26.2   130k 46.2 -> 39.6
+//           change   4k  8.3 ->  6.1   65k 11.6 -> 10.6    95k 12.6 -> 12.8
+//           apply    4k  7.5 ->  5.8   65k 11.0 ->  9.0    95k 11.6 -> 11.6
+//           XSPH     4k  9.8 ->  5.0   49k 10.5 ->  9.8    65k 10.5 -> 10.7
+//   tolerance mode
+//           density  4k 28.4 -> 12.9   65k 26.3 -> 21.4    95k 27.5 -> 26.4
+//           change   4k  8.0 ->  5.4   33k  7.3 ->  6.2    49k  7.3 ->  7.3
+//           apply    4k  6.6 ->  4.5   33k  6.0 ->  5.3    49k  6.2 ->  6.8
+//           XSPH     4k  8.4 ->  4.6   65k  8.4 ->  8.0    95k 10.4 -> 10.5
+struct QuadLimits {
+    u32 density, xsph, sweeps;
+};
+constexpr QuadLimits quad_limits(bool fast) {
+    return fast ? QuadLimits{98304, 65536, 40960} : QuadLimits{131072, 65536, 65536};
+}
+bool sweeps_by_quads(u32 nt, u32 nslots, bool fast) {
+    return nt == 0 && nslots <= quad_limits(fast).sweeps;
+}
 
 template <bool F>
 void density_alpha_mode(u32 nt, hipStream_t s, u32 nslots, const Nbr& P, const PairList& L,
                         const float4* xs, float* rho, float* alpha, DeviceState* open) {
+    if (nt == 256 && nslots <= quad_limits(F).density) {
+        k_density_alpha_q<F><<<nslots / kQuadGroup, NS, 0, s>>>(P, L, xs, rho, alpha, open);
+        WSIM_LAUNCH_CHECK();
+        return;
+    }
     switch (nt) {
     case 64: k_density_alpha<64, F><<<grid_for(nslots, 64), 64, 0, s>>>(P, L, xs, rho, alpha, nullptr, open); break;
     case 128: k_density_alpha<128, F><<<grid_for(nslots, 128), 128, 0, s>>>(P, L, xs, rho, alpha, nullptr, open); break;
@@ -1986,6 +2659,11 @@ template <bool F>
 void xsph_mode(u32 nt, hipStream_t s, u32 nslots, const Nbr& P, const PairList& L,
                const float4* xs, const float4* vin, const float* rho, float4* vout) {
     constexpr int XPU = 4;
+    if (nt == 0 && nslots <= quad_limits(F).xsph) {
+        k_xsph_q<F><<<nslots / kQuadGroup, NS, 0, s>>>(P, L, xs, vin, rho, vout);
+        WSIM_LAUNCH_CHECK();
+        return;
+    }
     switch (nt) {
     case 0: k_xsph_st<XPU, F><<<nslots / kTile, kTile, 0, s>>>(P, L, xs, vin, rho, vout); break;
     case 64: k_xsph<64, XPU, F><<<grid_for(nslots, 64), 64, 0, s>>>(P, L, xs, vin, rho, vout); break;
@@ -2047,6 +2725,14 @@ void change_staged(hipStream_t s, u32 nslots, const Nbr& P, const PairList& L, c
 template <int MODE, bool F>
 void change_mode(u32 nt, u32 pu, hipStream_t s, u32 nslots, const Nbr& P, const PairList& L,
                  const ChangeArgs& a) {
+    if (pu != 2 && pu != 4 && pu != 8) fail(kInvalidArgument, "change pairs per trip");
+    if (sweeps_by_quads(nt, nslots, F)) {
+        k_change_q<MODE, F><<<nslots / kQuadGroup, NS, 0, s>>>(
+            P, L, a.xs, a.vs, a.rho, a.alpha, a.rho0, a.pform, a.iter, a.st, a.part, a.rho_adv,
+            a.kappa, a.xk);
+        WSIM_LAUNCH_CHECK();
+        return;
+    }
     if (nt == 0) {
         switch (pu) {
         case 2: change_staged<MODE, 2, F>(s, nslots, P, L, a); break;
@@ -2081,6 +2767,7 @@ struct ApplyArgs {
     int mode;
     double thr;
     const double* part;
+    int quarters;  // part as k_change_q writes it
     DeviceState* st;
     const float4* vin;
     float4* vout;
@@ -2090,8 +2777,8 @@ struct ApplyArgs {
 template <int NT, int PU, bool F>
 void apply_one(hipStream_t s, u32 nslots, const Nbr& P, const PairList& L, const ApplyArgs& a) {
     k_apply<NT, PU, F><<<grid_for(nslots, NT), NT, 0, s>>>(P, L, a.xk, a.kappa, a.rho0, a.pform,
-                                                           a.iter, a.mode, a.thr, a.part, a.st,
-                                                           a.vin, a.vout);
+                                                           a.iter, a.mode, a.thr, a.part,
+                                                           a.quarters, a.st, a.vin, a.vout);
 }
 
 template <int NT, bool F>
@@ -2108,14 +2795,22 @@ void apply_pu(u32 pu, hipStream_t s, u32 nslots, const Nbr& P, const PairList& L
 template <int PU, bool F>
 void apply_staged(hipStream_t s, u32 nslots, const Nbr& P, const PairList& L, const ApplyArgs& a) {
     k_apply_st<PU, F><<<nslots / kTile, kTile, 0, s>>>(P, L, a.xk, a.kappa, a.rho0, a.pform,
-                                                       a.iter, a.mode, a.thr, a.part, a.st, a.vin,
-                                                       a.vout);
+                                                       a.iter, a.mode, a.thr, a.part,
+                                                       a.quarters, a.st, a.vin, a.vout);
 }
 
 // nt == 0 selects the LDS-staged kernel.
 template <bool F>
 void apply_mode(u32 nt, u32 pu, hipStream_t s, u32 nslots, const Nbr& P, const PairList& L,
                 const ApplyArgs& a) {
+    if (pu != 2 && pu != 4 && pu != 8) fail(kInvalidArgument, "apply pairs per trip");
+    if (sweeps_by_quads(nt, nslots, F)) {
+        k_apply_q<F><<<nslots / kQuadGroup, NS, 0, s>>>(P, L, a.xk, a.kappa, a.rho0, a.pform,
+                                                        a.iter, a.mode, a.thr, a.part, a.quarters,
+                                                        a.st, a.vin, a.vout);
+        WSIM_LAUNCH_CHECK();
+        return;
+    }
     if (nt == 0) {
         switch (pu) {
         case 2: apply_staged<2, F>(s, nslots, P, L, a); break;
@@ -2333,7 +3028,7 @@ void DFSPHSolver::init(const std::vector<u32>& counts, const std::vector<float>&
     }
     state_sorted_ = grid_sorted_ = defer_store_ = false;
     plan_ = DeviceBuffer<StageRanges>(slots_cap / kTile);
-    part_d_ = DeviceBuffer<double>(slots_cap / kTile);
+    part_d_ = DeviceBuffer<double>(slots_cap / kQuadGroup);
     part_f_ = DeviceBuffer<float>(slots_cap / 64);
     part_u_ = DeviceBuffer<u32>(slots_cap / 64);
     part_e_ = DeviceBuffer<u32>(slots_cap / 64);
@@ -2875,8 +3570,9 @@ void DFSPHSolver::phase_iterations(int mode, u32 begin, u32 end) {
                   static_cast<int>(cfg_.pressure_form), 0, dstate_.data(), part_d_.data(),
                   rho_adv_.data(), kappa_.data(), xk_.data(), cfg_.fast_math != 0};
     ApplyArgs aa{xk_.data(), kappa_.data(), cfg_.rest_density, static_cast<int>(cfg_.pressure_form),
-                 0, mode, thr, part_d_.data(), dstate_.data(), vs_.data(), vs_.data(),
-                 cfg_.fast_math != 0};
+                 0, mode, thr, part_d_.data(),
+                 sweeps_by_quads(shapes_.change_nt, nslots_, cfg_.fast_math != 0) ? 1 : 0,
+                 dstate_.data(), vs_.data(), vs_.data(), cfg_.fast_math != 0};
     for (u32 it = begin; it < end; ++it) {
         ca.iter = aa.iter = it;
         tbegin(mode == 0 ? kKDensityChange : kKDivChange, static_cast<int>(it));
@@ -3134,7 +3830,8 @@ void DFSPHSolver::iterations_taped(u32 begin, u32 end, SubstepTape& t) {
                   static_cast<int>(cfg_.pressure_form), 0, dstate_.data(), part_d_.data(),
                   nullptr, kappa_.data(), nullptr, false};
     ApplyArgs aa{nullptr, kappa_.data(), cfg_.rest_density, static_cast<int>(cfg_.pressure_form), 0, 0,
-                 thr, part_d_.data(), dstate_.data(), nullptr, nullptr, false};
+                 thr, part_d_.data(), sweeps_by_quads(shapes_.change_nt, nslots_, false) ? 1 : 0,
+                 dstate_.data(), nullptr, nullptr, false};
     for (u32 it = begin; it < end; ++it) {
         ca.iter = aa.iter = it;
         ca.vs = t.w.data() + it * ns;
@@ -3260,6 +3957,7 @@ void DFSPHSolver::autotune(int reps) {
                   rho_adv_.data(), kappa_.data(), xk_.data(), cfg_.fast_math != 0};
     ApplyArgs aa{xk_.data(), kappa_.data(), cfg_.rest_density, static_cast<int>(cfg_.pressure_form),
                  0, 0, static_cast<double>(cfg_.eta_density * cfg_.rest_density), part_d_.data(),
+                 sweeps_by_quads(shapes_.change_nt, nslots_, cfg_.fast_math != 0) ? 1 : 0,
                  dstate_.data(), vs_.data(), vs_.data(), cfg_.fast_math != 0};
     try {
         // cell_start pass
