@@ -52,21 +52,33 @@ __device__ inline u32 wave_lower_bound(const u32* __restrict__ keys, u32 n, u32 
     return lo;
 }
 
-__global__ __launch_bounds__(256) void k_cell_keys(const float* __restrict__ xyz, u32 n, GridGeom g,
-                                                   u32* __restrict__ keys, u32* __restrict__ vals,
-                                                   u32* span) {
+// Cell keys and original indices.  Workgroup t writes the sort's tile t and
+// counts the first digit of its keys (radix_count_*), which saves the sort
+// its first upsweep.
+__global__ __launch_bounds__(kRadixThreads) void k_cell_keys(const float* __restrict__ xyz, u32 n,
+                                                             GridGeom g, u32* __restrict__ keys,
+                                                             u32* __restrict__ vals, u32* span,
+                                                             u32 dmask, u32* __restrict__ hist,
+                                                             u32 tiles) {
+    __shared__ u32 cnt[256];
     advance_span(span);
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const u64 o = 3ull * i;
-    keys[i] = g.key_of(xyz[o], xyz[o + 1], xyz[o + 2]);
-    vals[i] = i;
+    radix_count_begin(cnt);
+#pragma unroll
+    for (int r = 0; r < kRadixTile / kRadixThreads; ++r) {
+        const u32 i = blockIdx.x * kRadixTile + r * kRadixThreads + threadIdx.x;
+        if (i >= n) continue;
+        const u64 o = 3ull * i;
+        const u32 key = g.key_of(xyz[o], xyz[o + 1], xyz[o + 2]);
+        keys[i] = key;
+        vals[i] = i;
+        radix_count_key(cnt, key & dmask);
+    }
+    radix_count_end(cnt, dmask, hist, tiles);
 }
 
-// Scene of original index i: the last s with starts[s] <= i (empty scenes
-// share their start with the next scene and are skipped).
-__device__ inline u32 scene_of_index(const u32* __restrict__ starts, u32 scenes, u32 i) {
-    u32 lo = 0, hi = scenes - 1;
+// Scene of original index i among [lo, hi]: the last s with starts[s] <= i
+// (empty scenes share their start with the next scene and are skipped).
+__device__ inline u32 scene_of_index(const u32* __restrict__ starts, u32 lo, u32 hi, u32 i) {
     while (lo < hi) {
         const u32 mid = (lo + hi + 1) >> 1;
         if (starts[mid] <= i) lo = mid;
@@ -75,15 +87,32 @@ __device__ inline u32 scene_of_index(const u32* __restrict__ starts, u32 scenes,
     return lo;
 }
 
-__global__ __launch_bounds__(256) void k_seg_keys(const float* __restrict__ xyz, u32 n, GridGeom g,
-                                                  const u32* __restrict__ starts, u32 scenes,
-                                                  u32* __restrict__ keys, u32* __restrict__ vals) {
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const u64 o = 3ull * i;
-    const u32 s = scene_of_index(starts, scenes, i);
-    keys[i] = s * (g.C + 1u) + g.key_of(xyz[o], xyz[o + 1], xyz[o + 2]);
-    vals[i] = i;
+// k_cell_keys with every scene's keys behind those of the scenes before it.
+// The tile's first and last scene are found once for the workgroup (mostly
+// the same scene), the particles search between them.
+__global__ __launch_bounds__(kRadixThreads) void k_seg_keys(const float* __restrict__ xyz, u32 n,
+                                                            GridGeom g,
+                                                            const u32* __restrict__ starts,
+                                                            u32 scenes, u32* __restrict__ keys,
+                                                            u32* __restrict__ vals, u32 dmask,
+                                                            u32* __restrict__ hist, u32 tiles) {
+    __shared__ u32 cnt[256];
+    const u32 first = blockIdx.x * kRadixTile;
+    const u32 s0 = scene_of_index(starts, 0u, scenes - 1, first);
+    const u32 s1 = scene_of_index(starts, s0, scenes - 1, min(first + kRadixTile, n) - 1);
+    radix_count_begin(cnt);
+#pragma unroll
+    for (int r = 0; r < kRadixTile / kRadixThreads; ++r) {
+        const u32 i = first + r * kRadixThreads + threadIdx.x;
+        if (i >= n) continue;
+        const u64 o = 3ull * i;
+        const u32 s = scene_of_index(starts, s0, s1, i);
+        const u32 key = s * (g.C + 1u) + g.key_of(xyz[o], xyz[o + 1], xyz[o + 2]);
+        keys[i] = key;
+        vals[i] = i;
+        radix_count_key(cnt, key & dmask);
+    }
+    radix_count_end(cnt, dmask, hist, tiles);
 }
 
 // Each workgroup owns CPT * 256 consecutive cells.
@@ -240,11 +269,13 @@ void CellGrid::build(const float* positions_xyz, size_t count) {
     if (count > capacity_) reserve(count);
     count_ = count;
     const u32 n = static_cast<u32>(count);
-    k_cell_keys<<<div_up(n, 256), 256, 0, stream_>>>(positions_xyz, n, g_, k_[0].data(), v_[0].data(),
-                                                     span());
+    const u32 tiles = radix_tiles(n);
+    k_cell_keys<<<tiles, kRadixThreads, 0, stream_>>>(positions_xyz, n, g_, k_[0].data(),
+                                                      v_[0].data(), span(), first_digit_mask(),
+                                                      hist_.data(), tiles);
     WSIM_LAUNCH_CHECK();
     cur_ = radix_sort_pairs(k_[0].data(), v_[0].data(), k_[1].data(), v_[1].data(), count,
-                            key_bits(g_.C), hist_.data(), stream_);
+                            key_bits(g_.C), hist_.data(), stream_, true);
     build_cell_start(k_[cur_].data(), n, g_.C + 1, cs_.data(), stream_, cpt_, span());
 }
 
@@ -283,12 +314,15 @@ void CellGrid::build_segmented(const float* positions_xyz, size_t count, const u
     if (count == 0) return;
     if (count > capacity_) reserve(count);
     const u32 n = static_cast<u32>(count);
-    k_seg_keys<<<div_up(n, 256), 256, 0, stream_>>>(positions_xyz, n, g_, starts, scenes,
-                                                    k_[0].data(), v_[0].data());
-    WSIM_LAUNCH_CHECK();
     const u32 ncs = scenes * (g_.C + 1) + 1;
+    const u32 tiles = radix_tiles(n);
+    k_seg_keys<<<tiles, kRadixThreads, 0, stream_>>>(positions_xyz, n, g_, starts, scenes,
+                                                     k_[0].data(), v_[0].data(),
+                                                     radix_first_digit_mask(key_bits(ncs - 2)),
+                                                     hist_.data(), tiles);
+    WSIM_LAUNCH_CHECK();
     cur_ = radix_sort_pairs(k_[0].data(), v_[0].data(), k_[1].data(), v_[1].data(), count,
-                            key_bits(ncs - 2), hist_.data(), stream_);
+                            key_bits(ncs - 2), hist_.data(), stream_, true);
     build_cell_start(k_[cur_].data(), n, ncs, cs_.data(), stream_, cpt_);
 }
 

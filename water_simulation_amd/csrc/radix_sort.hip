@@ -19,6 +19,15 @@
 // keys a pass is bound by launch and latency, not bytes, and the wide tiles
 // halve the per-tile histogram matrix and its strided accesses (against
 // 1024-key tiles) while keeping each lane's serial ranking work short.
+//
+// Smaller sorts are launches and latency alone, so they take fewer kernels:
+// up to kRadixFew tiles the downsweep adds up its digit offsets itself from a
+// tile-major count matrix (64 KB at most, read once by every tile), without
+// rs_scan_rows; up to kRadixSmall keys one workgroup runs every digit pass
+// with the keys in registers and LDS (rs_small).  A whole grid build of 1.2 M
+// cells, us, three kernels a digit -> now: 1,000 keys 42.3 -> 15.6, 4,000
+// 43.4 -> 21.6, 8,192 42.6 -> 30.8 (one workgroup) and 8,193 41.8 -> 29.9
+// (tiles): the lines cross there; 100,000 42.8 -> 36.1, 131,072 43.0 -> 35.0.
 #include "device_math.hpp"
 #include "radix_sort.hpp"
 
@@ -118,6 +127,10 @@ __global__ __launch_bounds__(RS_DIGITS) void rs_scan_rows(u32* __restrict__ hist
     if (tid == 0) totals[blockIdx.x] = s_carry;
 }
 
+// FEW: offs is the tile-major count matrix of the pass; each digit's total and
+// its count in the tiles before this one are added up here (four threads per
+// digit, every load of a thread in flight at once) and totals is unused.
+template <bool FEW>
 __global__ __launch_bounds__(RS_THREADS) void rs_downsweep(
     const u32* __restrict__ kin, const u32* __restrict__ vin, u32* __restrict__ kout,
     u32* __restrict__ vout, u32 n, int shift, int nbits, const u32* __restrict__ offs,
@@ -134,8 +147,26 @@ __global__ __launch_bounds__(RS_THREADS) void rs_downsweep(
     // this tile's offset in each digit's run and the digit totals (threads
     // [0, 256), one digit each), loaded with the keys
     const bool digit_thread = static_cast<u32>(tid) <= dmask;
-    const u32 goff = digit_thread ? offs[static_cast<u64>(tid) * nblocks + blockIdx.x] : 0u;
-    const u32 dtot = digit_thread ? totals[tid] : 0u;
+    u32 goff = 0, dtot = 0;
+    constexpr int kParts = RS_THREADS / RS_DIGITS;
+    __shared__ u32 s_part[FEW ? 2 * kParts : 1][RS_DIGITS];
+    if constexpr (FEW) {
+        const u32 d = tid & (RS_DIGITS - 1), q = tid / RS_DIGITS;
+        u32 before = 0, all = 0;
+        if (d <= dmask) {
+#pragma unroll 8
+            for (u32 t = q; t < nblocks; t += kParts) {
+                const u32 c = offs[t * RS_DIGITS + d];
+                all += c;
+                before += t < blockIdx.x ? c : 0u;
+            }
+        }
+        s_part[q][d] = before;
+        s_part[kParts + q][d] = all;
+    } else {
+        goff = digit_thread ? offs[static_cast<u64>(tid) * nblocks + blockIdx.x] : 0u;
+        dtot = digit_thread ? totals[tid] : 0u;
+    }
     for (int i = tid; i < RS_WAVES * RS_DIGITS; i += RS_THREADS) (&s_wc[0][0])[i] = 0;
     __syncthreads();
 
@@ -181,6 +212,13 @@ __global__ __launch_bounds__(RS_THREADS) void rs_downsweep(
             s_wc[ww][d] = total;
             total += c;
         }
+        if constexpr (FEW) {
+#pragma unroll
+            for (int q = 0; q < kParts; ++q) {
+                goff += s_part[q][d];
+                dtot += s_part[kParts + q][d];
+            }
+        }
         s_goff[d] = goff;
     }
     // digit base: scan of the digit totals
@@ -214,6 +252,89 @@ __global__ __launch_bounds__(RS_THREADS) void rs_downsweep(
     }
 }
 
+// Every digit pass of n <= RS_THREADS * ITEMS keys in one workgroup: ranks as
+// in rs_downsweep, the reordered keys handed to the next pass through LDS.
+// Keys and values are read and written once, so in and out may be the same.
+// The bits are split evenly over the passes (shorter ballot chains).
+template <int ITEMS>
+__global__ __launch_bounds__(RS_THREADS) void rs_small(const u32* kin, const u32* vin, u32* kout,
+                                                       u32* vout, u32 n, int bits) {
+    __shared__ u32 s_wc[RS_WAVES][RS_DIGITS];
+    __shared__ u32 s_start[RS_DIGITS];
+    __shared__ u32 s_tmp[RS_DIGITS / kWave];
+    __shared__ u32 s_k[RS_THREADS * ITEMS];
+    __shared__ u32 s_v[RS_THREADS * ITEMS];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const u32 base = w * (kWave * ITEMS) + lane;
+    const u64 lanes_below = (1ull << lane) - 1ull;
+    u32 key[ITEMS], val[ITEMS], rank[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const u32 idx = base + r * kWave;
+        key[r] = idx < n ? kin[idx] : 0u;
+        val[r] = idx < n ? vin[idx] : 0u;
+    }
+    const int passes = (bits + 7) / 8, per = (bits + passes - 1) / passes;
+    for (int shift = 0; shift < bits; shift += per) {
+        const int nbits = min(per, bits - shift);
+        const u32 dmask = (1u << nbits) - 1u;
+        for (int i = tid; i < RS_WAVES * RS_DIGITS; i += RS_THREADS) (&s_wc[0][0])[i] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            const bool valid = base + r * kWave < n;
+            const u32 d = (key[r] >> shift) & dmask;
+            const u64 m = match_digit(d, nbits) & __ballot(valid);
+            const u32 below = static_cast<u32>(__popcll(m & lanes_below));
+            u32 cur = 0;
+            if (valid) cur = s_wc[w][d];
+            __builtin_amdgcn_wave_barrier();
+            if (valid && below == 0) s_wc[w][d] = cur + static_cast<u32>(__popcll(m));
+            __builtin_amdgcn_wave_barrier();
+            rank[r] = cur + below;
+        }
+        __syncthreads();
+        u32 total = 0;
+        if (tid < RS_DIGITS) {
+#pragma unroll
+            for (int ww = 0; ww < RS_WAVES; ++ww) {
+                const u32 c = s_wc[ww][tid];
+                s_wc[ww][tid] = total;
+                total += c;
+            }
+        }
+        const u32 start = block_exclusive_scan256(total, s_tmp);
+        if (tid < RS_DIGITS) s_start[tid] = start;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            if (base + r * kWave < n) {
+                const u32 d = (key[r] >> shift) & dmask;
+                const u32 pos = s_start[d] + s_wc[w][d] + rank[r];
+                s_k[pos] = key[r];
+                s_v[pos] = val[r];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            const u32 idx = base + r * kWave;
+            if (idx < n) {
+                key[r] = s_k[idx];
+                val[r] = s_v[idx];
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const u32 idx = base + r * kWave;
+        if (idx < n) {
+            kout[idx] = key[r];
+            vout[idx] = val[r];
+        }
+    }
+}
+
 }  // namespace
 
 // Per-tile digit counts plus the 256 digit totals.
@@ -227,6 +348,16 @@ int radix_sort_pairs(u32* k0, u32* v0, u32* k1, u32* v1, size_t n, int bits, u32
     if (n > 0xFFFFF000ull) fail(kInvalidArgument, "radix_sort_pairs: too many elements");
     const u32 nn = static_cast<u32>(n);
     const u32 nblocks = div_up(n, RS_TILE);
+    static_assert(kRadixSmall == 8 * RS_THREADS, "items per thread below");
+    if (nn <= kRadixSmall) {
+        if (nn <= RS_THREADS) rs_small<1><<<1, RS_THREADS, 0, stream>>>(k0, v0, k0, v0, nn, bits);
+        else if (nn <= 2 * RS_THREADS) rs_small<2><<<1, RS_THREADS, 0, stream>>>(k0, v0, k0, v0, nn, bits);
+        else if (nn <= 4 * RS_THREADS) rs_small<4><<<1, RS_THREADS, 0, stream>>>(k0, v0, k0, v0, nn, bits);
+        else rs_small<8><<<1, RS_THREADS, 0, stream>>>(k0, v0, k0, v0, nn, bits);
+        WSIM_LAUNCH_CHECK();
+        return 0;
+    }
+    const bool few = nblocks <= kRadixFew;
     u32* kin = k0;
     u32* vin = v0;
     u32* kout = k1;
@@ -239,10 +370,15 @@ int radix_sort_pairs(u32* k0, u32* v0, u32* k1, u32* v1, size_t n, int bits, u32
             WSIM_LAUNCH_CHECK();
         }
         u32* totals = hist + static_cast<size_t>(RS_DIGITS) * nblocks;
-        rs_scan_rows<<<1u << nbits, RS_DIGITS, 0, stream>>>(hist, nblocks, totals);
-        WSIM_LAUNCH_CHECK();
-        rs_downsweep<<<nblocks, RS_THREADS, 0, stream>>>(kin, vin, kout, vout, nn, shift, nbits,
-                                                         hist, nblocks, totals);
+        if (few) {
+            rs_downsweep<true><<<nblocks, RS_THREADS, 0, stream>>>(kin, vin, kout, vout, nn, shift,
+                                                                   nbits, hist, nblocks, nullptr);
+        } else {
+            rs_scan_rows<<<1u << nbits, RS_DIGITS, 0, stream>>>(hist, nblocks, totals);
+            WSIM_LAUNCH_CHECK();
+            rs_downsweep<false><<<nblocks, RS_THREADS, 0, stream>>>(
+                kin, vin, kout, vout, nn, shift, nbits, hist, nblocks, totals);
+        }
         WSIM_LAUNCH_CHECK();
         u32* tk = kin;
         u32* tv = vin;
