@@ -243,10 +243,7 @@ private:
     size_t leaf_count_ = 0;
     DeviceBuffer<u32> k_[2], v_[2], hist_;
     DeviceBuffer<u32> left_, right_, parent_;
-    DeviceBuffer<uint2> range_;      // leaf range [lo, hi] of every internal node
-    DeviceBuffer<float> boxes_, seg_;  // node boxes; segment tree over the leaf boxes
-    DeviceBuffer<u64> seg_off_;
-    std::vector<u64> seg_off_host_;
+    DeviceBuffer<float> boxes_, seg_;  // node boxes; segment tree above the leaf boxes
     int cur_ = 0;
 };
 
