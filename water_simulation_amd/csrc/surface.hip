@@ -196,6 +196,7 @@ __global__ __launch_bounds__(kMeshThreads) void k_mesh_splat(const double* __res
 
 struct KnnGrid {
     double lo0, lo1, lo2, cell;
+    double guess;  // squared radius of about k + 4 points
     int d0, d1, d2;
 };
 
@@ -269,17 +270,12 @@ __device__ __forceinline__ void knn_scan(u32 lo, u32 hi, double px, double py, d
 constexpr int kKnnLaneRings = 3;
 
 template <int K>
-__global__ __launch_bounds__(kMeshThreads) void k_knn_smooth(const double* __restrict__ P, u32 n,
-                                                             KnnGrid g,
-                                                             const u32* __restrict__ sorted,
-                                                             const double* __restrict__ Ps,
-                                                             const u32* __restrict__ cs,
-                                                             double* __restrict__ out,
-                                                             u32* __restrict__ far_count,
-                                                             u32* __restrict__ far) {
-    // one thread per point in cell order: a wave's points share cells
-    const u32 q = blockIdx.x * kMeshThreads + threadIdx.x;
-    if (q >= n) return;
+__device__ __forceinline__ void knn_lane(const double* __restrict__ P, KnnGrid g,
+                                         const u32* __restrict__ sorted,
+                                         const double* __restrict__ Ps,
+                                         const u32* __restrict__ cs, double* __restrict__ out,
+                                         u32* __restrict__ far_count, u32* __restrict__ far,
+                                         u32 q) {
     const u32 i = sorted[q];
     const double px = Ps[3ull * q], py = Ps[3ull * q + 1], pz = Ps[3ull * q + 2];
     const int h0 = knn_cell(px, g.lo0, g.cell, g.d0);
@@ -332,6 +328,204 @@ __global__ __launch_bounds__(kMeshThreads) void k_knn_smooth(const double* __res
     out[3ull * i] = sx / static_cast<double>(K);
     out[3ull * i + 1] = sy / static_cast<double>(K);
     out[3ull * i + 2] = sz / static_cast<double>(K);
+}
+
+// One thread per listed point (dense or far neighbourhoods that
+// k_knn_group leaves).
+template <int K>
+__global__ __launch_bounds__(kMeshThreads) void k_knn_smooth(
+    const double* __restrict__ P, KnnGrid g, const u32* __restrict__ sorted,
+    const double* __restrict__ Ps, const u32* __restrict__ cs, const u32* __restrict__ count,
+    const u32* __restrict__ list, double* __restrict__ out, u32* __restrict__ far_count,
+    u32* __restrict__ far) {
+    const u32 n = *count;
+    for (u32 k = blockIdx.x * kMeshThreads + threadIdx.x; k < n; k += gridDim.x * kMeshThreads)
+        knn_lane<K>(P, g, sorted, Ps, cs, out, far_count, far, list[k]);
+}
+
+// Appends q of every active lane to the list, one atomic a wave.
+__device__ __forceinline__ void wave_append(u32* __restrict__ list, u32* __restrict__ count,
+                                            u32 q) {
+    const unsigned long long act = __ballot(1);
+    const int first = __ffsll(act) - 1, lane = threadIdx.x & 63;
+    u32 at = 0;
+    if (lane == first) at = atomicAdd(count, static_cast<u32>(__popcll(act)));
+    at = __shfl(at, first, 64);
+    list[at + static_cast<u32>(__popcll(act & ((1ull << lane) - 1ull)))] = q;
+}
+
+// G lanes per point over the rings 0..R at once.  A lane that keeps the K
+// nearest of all candidates in registers spends its time on the insertion (15
+// steps of binary64 compares whenever any lane of the wave accepts) and
+// leaves small clouds to one wave per CU.  Here the group splits the
+// candidates, lists those within a limit in LDS (a few more than K), each
+// listed point finds its rank among them, and the K first are summed in
+// ascending (d^2, id) order, one lane per coordinate.  The limit is
+//   GUESS: g.guess, the squared radius that holds about K + 4 points at the
+//     expected spacing, in one visit of the candidates;
+//   else: the first of kKnnBins bins of [0, reach^2) at which K points are
+//     counted, in two visits.
+// Either way it lies below the reach, the point's own distance to the faces
+// of the scanned block (none where the block ends the grid).  Points with
+// fewer than K neighbours in the limit go to `few`, with more than the list
+// holds to `many`.  A pass over 1,001,385 points, 15 neighbours, with the
+// guess: 312 us with 8 lanes, 412 with 4, 403 with 16 (one lane a point:
+// 1,267); 17,056 points: 18 us with 8 lanes (256).  Bins in both visits for
+// every point: 799 us.
+constexpr int kKnnBins = 32;
+constexpr int kKnnLists = 5;  // of points, between the passes of knn_pass
+constexpr int knn_cap(int k) { return k <= 16 ? 32 : 64; }  // listed points
+template <int K, int R, int G, bool GUESS>
+__global__ __launch_bounds__(kMeshThreads) void k_knn_group(
+    u32 n, const u32* __restrict__ list_count, const u32* __restrict__ list, KnnGrid g,
+    const u32* __restrict__ sorted, const double* __restrict__ Ps, const u32* __restrict__ cs,
+    double* __restrict__ out, u32* __restrict__ few_count, u32* __restrict__ few,
+    u32* __restrict__ many_count, u32* __restrict__ many) {
+    constexpr u32 kCap = knn_cap(K);
+    static_assert(K <= kCap && kCap <= 256, "list holds the K nearest, places in 8 bits");
+    constexpr int W = 2 * R + 1, kRows = W * W;
+    constexpr int kPts = kMeshThreads / G;
+    __shared__ u32 s_lo[kPts][kRows], s_hi[kPts][kRows];
+    __shared__ u32 s_bin[GUESS ? 1 : kPts][kKnnBins / 2];  // two 16-bit counts a word
+    __shared__ u32 s_cnt[kPts];
+    __shared__ double s_d[kPts][kCap];
+    __shared__ u32 s_slot[kPts][kCap];
+    __shared__ uint8_t s_ord[kPts][K];
+    const int pt = threadIdx.x / G, lane = threadIdx.x % G;
+    const u32 total = list ? *list_count : n;
+    // LDS below is private to the group, whose lanes share a wave
+    auto sync = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+    for (u32 f = blockIdx.x * kPts + pt; f < total; f += gridDim.x * kPts) {
+        const u32 q = list ? list[f] : f;
+        const double px = Ps[3ull * q], py = Ps[3ull * q + 1], pz = Ps[3ull * q + 2];
+        const int h0 = knn_cell(px, g.lo0, g.cell, g.d0);
+        const int h1 = knn_cell(py, g.lo1, g.cell, g.d1);
+        const int h2 = knn_cell(pz, g.lo2, g.cell, g.d2);
+        const int c0 = max(h2 - R, 0), c1 = min(h2 + R, g.d2 - 1);
+        for (int r = lane; r < kRows; r += G) {
+            const int a = h0 - R + r / W, b = h1 - R + r % W;
+            const bool in = a >= 0 && a < g.d0 && b >= 0 && b < g.d1;
+            const u32 row = in ? (static_cast<u32>(a) * g.d1 + b) * g.d2 : 0u;
+            s_lo[pt][r] = in ? cs[row + c0] : 0u;
+            s_hi[pt][r] = in ? cs[row + c1 + 1] : 0u;
+        }
+        if (lane == 0) s_cnt[pt] = 0;
+        // distance to the faces of the scanned block that other cells touch
+        double reach = INFINITY;
+        auto face = [&](double p, double lo, int h, int d) {
+            if (h - R > 0) reach = fmin(reach, p - (lo + (h - R) * g.cell));
+            if (h + R < d - 1) reach = fmin(reach, (lo + (h + R + 1) * g.cell) - p);
+        };
+        face(px, g.lo0, h0, g.d0);
+        face(py, g.lo1, h1, g.d1);
+        face(pz, g.lo2, h2, g.d2);
+        const bool all = reach == INFINITY;  // the block is the whole grid
+        if (all) {  // every candidate lies within the grid's diagonal
+            const double a = g.d0 * g.cell, b = g.d1 * g.cell, c = g.d2 * g.cell;
+            reach = 1.1 * sqrt(a * a + b * b + c * c);
+        }
+        reach = fmax(reach * (1.0 - 1e-9), 0.0);
+        // the group shares every row, or with many rows each lane takes its own
+        constexpr bool kOwnRows = R > 1;
+        auto visit = [&](auto&& use) {
+            for (int r = kOwnRows ? lane : 0; r < kRows; r += kOwnRows ? G : 1) {
+                const u32 hi = s_hi[pt][r];
+                for (u32 s = s_lo[pt][r] + (kOwnRows ? 0 : lane); s < hi; s += kOwnRows ? 1 : G) {
+                    const double dx = Ps[3ull * s] - px, dy = Ps[3ull * s + 1] - py,
+                                 dz = Ps[3ull * s + 2] - pz;
+                    use(s, (dx * dx + dy * dy) + dz * dz);
+                }
+            }
+        };
+        auto append = [&](u32 s, double d) {
+            const u32 k = atomicAdd(&s_cnt[pt], 1u);
+            if (k < kCap) {
+                s_d[pt][k] = d;
+                s_slot[pt][k] = s;
+            }
+        };
+        u32 m = 0;  // listed points
+        bool overfull = false;
+        if constexpr (GUESS) {
+            const double lim = fmin(g.guess, reach * reach);
+            sync();
+            visit([&](u32 s, double d) {
+                if (d < lim) append(s, d);
+            });
+            sync();
+            m = s_cnt[pt];
+        } else {
+            for (int k = lane; k < kKnnBins / 2; k += G) s_bin[pt][k] = 0;
+            sync();
+            u32 have = 0;
+            for (int r = 0; r < kRows; ++r) have += s_hi[pt][r] - s_lo[pt][r];
+            overfull = have > 0xFFFFu;
+            const float scale =
+                reach > 0.0 ? static_cast<float>(static_cast<double>(kKnnBins) / (reach * reach))
+                            : INFINITY;
+            int top = -1;  // last bin of the list
+            if (!overfull) {
+                // the bin is monotone in d; the last one may miss points
+                // beyond the block and never counts
+                visit([&](u32, double d) {
+                    const float bin = static_cast<float>(d) * scale;
+                    if (bin < static_cast<float>(kKnnBins - 1)) {
+                        const u32 b = static_cast<u32>(bin);
+                        atomicAdd(&s_bin[pt][b >> 1], b & 1u ? 0x10000u : 1u);
+                    }
+                });
+                sync();
+#pragma unroll
+                for (int b = 0; b < kKnnBins - 1; ++b) {
+                    const u32 c = (s_bin[pt][b >> 1] >> (16 * (b & 1))) & 0xFFFFu;
+                    if (m < static_cast<u32>(K)) {
+                        m += c;
+                        top = b;
+                    }
+                }
+            }
+            if (m >= static_cast<u32>(K) && m <= kCap) {
+                const float lim = static_cast<float>(top + 1);
+                visit([&](u32 s, double d) {
+                    if (static_cast<float>(d) * scale < lim) append(s, d);
+                });
+                sync();
+            }
+        }
+        if (overfull || m < static_cast<u32>(K) || m > kCap) {
+            if (lane == 0) {
+                if (!overfull && m < static_cast<u32>(K)) wave_append(few, few_count, q);
+                else wave_append(many, many_count, q);
+            }
+            continue;
+        }
+        for (u32 e = lane; e < m; e += G) {
+            const double d = s_d[pt][e];
+            u32 rank = 0, tied = 0;
+            for (u32 k = 0; k < m; ++k) {
+                const double o = s_d[pt][k];
+                rank += o < d ? 1u : 0u;
+                tied += o == d ? 1u : 0u;  // itself included
+            }
+            if (tied > 1u && rank < static_cast<u32>(K)) {  // lower ids first
+                const u32 id = sorted[s_slot[pt][e]];
+                for (u32 k = 0; k < m; ++k)
+                    if (s_d[pt][k] == d && sorted[s_slot[pt][k]] < id) ++rank;
+            }
+            if (rank < static_cast<u32>(K)) s_ord[pt][rank] = static_cast<uint8_t>(e);
+        }
+        sync();
+        if (lane < 3) {
+            double v[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) v[k] = Ps[3ull * s_slot[pt][s_ord[pt][k]] + lane];
+            double sum = 0.0;
+#pragma unroll
+            for (int k = 0; k < K; ++k) sum = sum + v[k];
+            out[3ull * sorted[q] + lane] = sum / static_cast<double>(K);
+        }
+        sync();
+    }
 }
 
 // The listed points, one wave each: the lanes take the (a, b) rows of every
@@ -1019,6 +1213,49 @@ static double numpy_sum(const double* a, size_t n) {
     return numpy_sum(a, n2) + numpy_sum(a + n2, n - n2);
 }
 
+// One smoothing pass over the gridded points: the guessed radius in rings 0..1,
+// then the points it held too many or too few neighbours for (surfaces, other
+// spacings; rings 0..4 reach k points at four times the expected spacing),
+// then dense and far neighbourhoods.
+template <int K>
+static void knn_pass(const double* in, u32 n, const KnnGrid& kg, const u32* sorted,
+                     const double* ps, const u32* cs, double* out, u32* counts, u32* lists,
+                     hipStream_t s) {
+    constexpr u32 kNear = 8, kWide = 16, kWave4 = 64;
+    auto list = [&](int k) { return lists + static_cast<u64>(k) * n; };
+    enum { few, many, fewer, rest, far };
+    static_assert(far + 1 == kKnnLists, "one list each");
+    auto blocks = [&](u32 lanes) { return div_up(n, kMeshThreads / lanes); };
+    k_knn_group<K, 1, kNear, true><<<blocks(kNear), kMeshThreads, 0, s>>>(
+        n, nullptr, nullptr, kg, sorted, ps, cs, out, counts + few, list(few), counts + many,
+        list(many));
+    WSIM_LAUNCH_CHECK();
+    k_knn_group<K, 1, kNear, false><<<std::min<u32>(blocks(kNear), 2048), kMeshThreads, 0, s>>>(
+        n, counts + many, list(many), kg, sorted, ps, cs, out, counts + few, list(few),
+        counts + rest, list(rest));
+    WSIM_LAUNCH_CHECK();
+    k_knn_group<K, 2, kWide, false><<<std::min<u32>(blocks(kWide), 2048), kMeshThreads, 0, s>>>(
+        n, counts + few, list(few), kg, sorted, ps, cs, out, counts + fewer, list(fewer),
+        counts + rest, list(rest));
+    WSIM_LAUNCH_CHECK();
+    k_knn_group<K, 4, kWave4, false><<<std::min<u32>(blocks(kWave4), 2048), kMeshThreads, 0, s>>>(
+        n, counts + fewer, list(fewer), kg, sorted, ps, cs, out, counts + rest, list(rest),
+        counts + rest, list(rest));
+    WSIM_LAUNCH_CHECK();
+    const u32 gd = std::min<u32>(div_up(n, static_cast<u32>(kMeshThreads)), 1024);
+    k_knn_smooth<K><<<gd, kMeshThreads, 0, s>>>(in, kg, sorted, ps, cs, counts + rest, list(rest),
+                                                out, counts + far, list(far));
+    WSIM_LAUNCH_CHECK();
+    const u32 gf = std::min<u32>(gd, 256);  // 4 waves per block walk the list
+    k_knn_far<K><<<gf, kMeshThreads, 0, s>>>(in, kg, sorted, ps, cs, counts + far, list(far), out);
+    WSIM_LAUNCH_CHECK();
+}
+
+// Radius of a sphere that holds k points at one per unit volume.
+static double knn_radius(double k) {
+    return std::cbrt(k * 3.0 / (4.0 * 3.14159265358979));
+}
+
 std::vector<double> gaussian_weights(double sigma, int* radius) {
     // scipy.ndimage._gaussian_kernel1d, order 0, truncate 4.0: phi / phi.sum()
     const int R = static_cast<int>(4.0 * sigma + 0.5);
@@ -1095,7 +1332,17 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
         bounds(pts_[cur].data(), mn, mx);
         KnnGrid kg{};
         kg.lo0 = mn[0], kg.lo1 = mn[1], kg.lo2 = mn[2];
-        kg.cell = 4.0 * P.particle_radius;
+        // The spacing: a particle diameter, or less where the points' box
+        // holds more of them.  The guess holds about k + 4 points at it, and
+        // a cell's edge is the guess, so rings 0..1 reach it (a pass of
+        // 1,001,385 points: 312 us; 353 with cells 1.15 times as wide; with
+        // 0.85 most points fall short and take 1,400).
+        const double dia = 2.0 * P.particle_radius;
+        const double box = (mx[0] - mn[0] + dia) * (mx[1] - mn[1] + dia) * (mx[2] - mn[2] + dia);
+        const double spacing = std::min(dia, std::cbrt(box / static_cast<double>(n)));
+        const double gr = knn_radius(P.k_neighbors + 4.0) * spacing;
+        kg.guess = gr * gr;
+        kg.cell = gr;
         u64 cells = 0;
         for (;;) {
             kg.d0 = static_cast<int>((mx[0] - mn[0]) / kg.cell) + 1;
@@ -1117,7 +1364,8 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
         const int w = radix_sort_pairs(knn_keys_[0].data(), knn_vals_[0].data(), knn_keys_[1].data(),
                                        knn_vals_[1].data(), n, key_bits(static_cast<u32>(cells - 1)),
                                        knn_hist_.data(), s);
-        build_cell_start(knn_keys_[w].data(), nn, static_cast<u32>(cells + 1), knn_cs_.data(), s);
+        build_cell_start(knn_keys_[w].data(), nn, static_cast<u32>(cells + 1), knn_cs_.data(), s,
+                         0);
         const u32* sorted = knn_vals_[w].data();
         double* out = pts_[cur ^ 1].data();
         if (knn_ps_.size() < 3 * n) knn_ps_ = DeviceBuffer<double>(3 * n);
@@ -1126,35 +1374,18 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
         const double* in = pts_[cur].data();
         const double* ps = knn_ps_.data();
         const u32* cs = knn_cs_.data();
-        if (knn_far_.size() < n) knn_far_ = DeviceBuffer<u32>(n);
-        if (knn_farc_.size() < 1) knn_farc_ = DeviceBuffer<u32>(1);
-        u32* fc = knn_farc_.data();
-        u32* fl = knn_far_.data();
-        WSIM_HIP(hipMemsetAsync(fc, 0, sizeof(u32), s));
-        const u32 gf = std::min<u32>(gp, 256);  // 4 waves per block walk the list
+        if (knn_far_.size() < kKnnLists * n) knn_far_ = DeviceBuffer<u32>(kKnnLists * n);
+        if (knn_farc_.size() < kKnnLists) knn_farc_ = DeviceBuffer<u32>(kKnnLists);
+        u32* fc = knn_farc_.data();  // counts of the lists
+        WSIM_HIP(hipMemsetAsync(fc, 0, kKnnLists * sizeof(u32), s));
+        u32* lists = knn_far_.data();
         switch (P.k_neighbors) {
-        case 8:
-            k_knn_smooth<8><<<gp, kMeshThreads, 0, s>>>(in, nn, kg, sorted, ps, cs, out, fc, fl);
-            k_knn_far<8><<<gf, kMeshThreads, 0, s>>>(in, kg, sorted, ps, cs, fc, fl, out);
-            break;
-        case 10:
-            k_knn_smooth<10><<<gp, kMeshThreads, 0, s>>>(in, nn, kg, sorted, ps, cs, out, fc, fl);
-            k_knn_far<10><<<gf, kMeshThreads, 0, s>>>(in, kg, sorted, ps, cs, fc, fl, out);
-            break;
-        case 15:
-            k_knn_smooth<15><<<gp, kMeshThreads, 0, s>>>(in, nn, kg, sorted, ps, cs, out, fc, fl);
-            k_knn_far<15><<<gf, kMeshThreads, 0, s>>>(in, kg, sorted, ps, cs, fc, fl, out);
-            break;
-        case 20:
-            k_knn_smooth<20><<<gp, kMeshThreads, 0, s>>>(in, nn, kg, sorted, ps, cs, out, fc, fl);
-            k_knn_far<20><<<gf, kMeshThreads, 0, s>>>(in, kg, sorted, ps, cs, fc, fl, out);
-            break;
-        default:
-            k_knn_smooth<30><<<gp, kMeshThreads, 0, s>>>(in, nn, kg, sorted, ps, cs, out, fc, fl);
-            k_knn_far<30><<<gf, kMeshThreads, 0, s>>>(in, kg, sorted, ps, cs, fc, fl, out);
-            break;
+        case 8: knn_pass<8>(in, nn, kg, sorted, ps, cs, out, fc, lists, s); break;
+        case 10: knn_pass<10>(in, nn, kg, sorted, ps, cs, out, fc, lists, s); break;
+        case 15: knn_pass<15>(in, nn, kg, sorted, ps, cs, out, fc, lists, s); break;
+        case 20: knn_pass<20>(in, nn, kg, sorted, ps, cs, out, fc, lists, s); break;
+        default: knn_pass<30>(in, nn, kg, sorted, ps, cs, out, fc, lists, s); break;
         }
-        WSIM_LAUNCH_CHECK();
         cur ^= 1;
     }
     const double* pts = pts_[cur].data();
