@@ -426,7 +426,7 @@ __global__ __launch_bounds__(kMeshThreads) void k_knn_group(
         }
         reach = fmax(reach * (1.0 - 1e-9), 0.0);
         // the group shares every row, or with many rows each lane takes its own
-        constexpr bool kOwnRows = R > 1;
+        constexpr bool kOwnRows = R > 2;
         auto visit = [&](auto&& use) {
             for (int r = kOwnRows ? lane : 0; r < kRows; r += kOwnRows ? G : 1) {
                 const u32 hi = s_hi[pt][r];
@@ -801,15 +801,24 @@ struct McDev {
     uint8_t tri[256][kMaxTri * 3];
 };
 
-// Marching cubes over wave segments.  A segment is 64 consecutive c of one
-// (a, b) row, handled by one wave; segments in linear order cover the grid
-// in grid-point order, so an exclusive scan of per-segment counts plus a
-// prefix across the wave numbers every vertex by (grid point, axis) and
-// every triangle by (cube, table order).  A grid point owns the crossing
-// edges from it along +a, +b, +c (edge mask bits 0, 1, 2); a cube starts at
-// its lowest corner.
-constexpr int kMcPlanes = 16;     // a planes walked by each k_mc_segments thread
-constexpr int kMcEmitPlanes = 64;  // a planes (segments) per wave of the emit passes: one per lane
+// Marching cubes over segments: 64 consecutive c of one (a, b) row.  Segments
+// in linear order cover the grid in grid-point order, so an exclusive scan of
+// per-segment counts plus a prefix across the segment numbers every vertex by
+// (grid point, axis) and every triangle by (cube, table order).  A grid point
+// owns the crossing edges from it along +a, +b, +c (edge mask bits 0, 1, 2); a
+// cube starts at its lowest corner.
+//
+// The grid is read once, into one inside bit per point (k_mc_bits).  Crossing
+// edges and cube configurations then come from the 64-bit words of a segment
+// and its neighbours, a thread per segment (k_mc_count), and only the segments
+// with something to emit, packed in a list, get a wave each (k_mc_vertices,
+// k_mc_triangles).
+struct McGrid {
+    int r0, r1, r2;
+    u32 ntx;    // segments per row
+    u32 nseg;
+    const u64* bits;
+};
 
 // exclusive prefix over the wave of small per-lane counts (< 2^bits)
 __device__ __forceinline__ u32 wave_prefix(u32 v, int bits) {
@@ -820,121 +829,247 @@ __device__ __forceinline__ u32 wave_prefix(u32 v, int bits) {
     return r;
 }
 
-// corner k of a cube sits at (a + (k & 1), b + (k >> 1 & 1), c + (k >> 2 & 1))
-__device__ __forceinline__ int mc_config(const float* __restrict__ g, u64 i, u64 sa, u64 sb,
-                                         float iso) {
-    int cfg = 0;
-    for (int k = 0; k < 8; ++k) {
-        const u64 j = i + (k & 1) * sa + ((k >> 1) & 1) * sb + ((k >> 2) & 1);
-        cfg |= (g[j] > iso ? 1 : 0) << k;
+// Inside bits, eight segments per wave with their loads in flight together.
+__global__ __launch_bounds__(256) void k_mc_bits(const float* __restrict__ g, u32 nseg, int r2,
+                                                 u32 ntx, float iso, u64* __restrict__ bits) {
+    constexpr u32 U = 8;
+    const u32 lane = threadIdx.x & 63;
+    const u32 wave = static_cast<u32>(
+        __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x * 4 + (threadIdx.x >> 6))));
+    for (u32 s0 = wave * U; s0 < nseg; s0 += gridDim.x * 4 * U) {
+        float v[U];
+#pragma unroll
+        for (u32 u = 0; u < U; ++u) {
+            const u32 row = (s0 + u) / ntx;
+            const u32 c = (s0 + u - row * ntx) * 64u + lane;
+            v[u] = s0 + u < nseg && c < static_cast<u32>(r2)
+                       ? g[static_cast<u64>(row) * static_cast<u32>(r2) + c]
+                       : -INFINITY;
+        }
+#pragma unroll
+        for (u32 u = 0; u < U; ++u) {
+            const u64 m = __ballot(v[u] > iso);
+            if (lane == u && s0 + u < nseg) bits[s0 + u] = m;
+        }
     }
-    return cfg;
 }
 
-// Vertex and triangle counts per segment.  Each thread walks kMcPlanes
-// planes of a at one (b, c), keeping the inside bits of the (b, c), (b+1, c),
-// (b, c+1), (b+1, c+1) points of the current plane (bits 0..3), so it loads
-// four grid values per grid point.
-__global__ __launch_bounds__(256) void k_mc_segments(const float* __restrict__ g, int r0, int r1,
-                                                     int r2, float iso,
-                                                     const McDev* __restrict__ T, u32 ntx,
-                                                     u32* __restrict__ segE,
-                                                     u32* __restrict__ segT) {
-    const int lane = threadIdx.x & 63;
-    const int b = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (b >= r1) return;  // whole wave
-    const int c = blockIdx.x * 64 + lane;
-    const int a0 = blockIdx.z * kMcPlanes;
-    const int a1 = min(a0 + kMcPlanes, r0);
-    const bool cv = c < r2, bn = b + 1 < r1, cn = c + 1 < r2;
-    auto plane = [&](int a) -> u32 {
-        if (!cv) return 0u;
-        const u64 i = (static_cast<u64>(a) * r1 + b) * r2 + c;
-        u32 q = g[i] > iso ? 1u : 0u;
-        if (bn && g[i + r2] > iso) q |= 2u;
-        if (cn && g[i + 1] > iso) q |= 4u;
-        if (bn && cn && g[i + r2 + 1] > iso) q |= 8u;
-        return q;
-    };
-    u32 cur = plane(a0);
-    for (int a = a0; a < a1; ++a) {
-        const bool an = a + 1 < r0;
-        const u32 nxt = an ? plane(a + 1) : 0u;
-        u32 e = 0, t = 0;
-        if (cv) {
-            const u32 in0 = cur & 1u;
-            u32 m = 0;
-            if (an && (nxt & 1u) != in0) m |= 1u;
-            if (bn && ((cur >> 1) & 1u) != in0) m |= 2u;
-            if (cn && ((cur >> 2) & 1u) != in0) m |= 4u;
-            e = static_cast<u32>(__popc(m));
-            if (an && bn && cn) {
-                // plane bit j = db + 2 dc is corner 2j (this plane) and 2j + 1 (next)
-                u32 cfg = 0;
-                for (int j = 0; j < 4; ++j)
-                    cfg |= (((cur >> j) & 1u) << (2 * j)) | (((nxt >> j) & 1u) << (2 * j + 1));
-                t = T->ntri[cfg];
+// The words of segment s and of its neighbours that its edges and cubes read:
+// row[k] and the same points one further along c (cnext[k]), k = da + 2 db;
+// rows beyond the grid read 0.
+struct McWords {
+    u64 row[4], cnext[4];
+    u64 valid, cvalid;  // points of the segment; those with a point at c + 1
+    bool an, bn;        // a + 1, b + 1 inside the grid
+    u32 a, b, tx;
+    __device__ __forceinline__ McWords(const McGrid& M, u32 s) {
+        const u32 r = s / M.ntx;
+        tx = s - r * M.ntx;
+        a = r / static_cast<u32>(M.r1);
+        b = r - a * static_cast<u32>(M.r1);
+        an = a + 1 < static_cast<u32>(M.r0);
+        bn = b + 1 < static_cast<u32>(M.r1);
+        const u32 left = static_cast<u32>(M.r2) - tx * 64u;  // points from here to the row's end
+        valid = left >= 64u ? ~0ull : (1ull << left) - 1ull;
+        cvalid = left > 64u ? ~0ull : (1ull << (left - 1u)) - 1ull;
+        const bool tn = tx + 1 < M.ntx;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const bool in = (!(k & 1) || an) && (!(k & 2) || bn);
+            const u32 t = s + ((k & 1) ? static_cast<u32>(M.r1) * M.ntx : 0u) + ((k & 2) ? M.ntx : 0u);
+            row[k] = in ? M.bits[t] : 0ull;
+            const u64 nx = in && tn ? M.bits[t + 1] : 0ull;
+            cnext[k] = (row[k] >> 1) | (nx << 63);
+        }
+    }
+    // crossing edges along axis 0, 1, 2
+    __device__ __forceinline__ u64 edges(int axis) const {
+        if (axis == 0) return an ? (row[0] ^ row[1]) & valid : 0ull;
+        if (axis == 1) return bn ? (row[0] ^ row[2]) & valid : 0ull;
+        return (row[0] ^ cnext[0]) & cvalid;
+    }
+    // cubes with corners on both sides
+    __device__ __forceinline__ u64 cubes() const {
+        if (!an || !bn) return 0ull;
+        u64 any = 0ull, all = ~0ull;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            any |= row[k] | cnext[k];
+            all &= row[k] & cnext[k];
+        }
+        return any & ~all & cvalid;
+    }
+    // configuration of the cube at bit c: corner k at (k & 1, k >> 1 & 1, k >> 2)
+    __device__ __forceinline__ u32 config(u32 c) const {
+        u32 cfg = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            cfg |= static_cast<u32>((row[k] >> c) & 1ull) << k;
+            cfg |= static_cast<u32>((cnext[k] >> c) & 1ull) << (k + 4);
+        }
+        return cfg;
+    }
+};
+
+// Counts of kScanBlock segments and their exclusive scan within the block:
+// vertices, triangles and segments with either, packed in one word.
+constexpr int kScanPer = 4;
+constexpr int kScanBlock = kMeshThreads * kScanPer;
+constexpr int kTriShift = 24, kActShift = 48;  // 192 and 320 per segment at most
+__device__ __forceinline__ u32 scan_verts(u64 v) { return static_cast<u32>(v) & 0xFFFFFFu; }
+__device__ __forceinline__ u32 scan_tris(u64 v) { return static_cast<u32>(v >> kTriShift) & 0xFFFFFFu; }
+__device__ __forceinline__ u32 scan_act(u64 v) { return static_cast<u32>(v >> kActShift); }
+
+__global__ __launch_bounds__(kMeshThreads) void k_mc_count(McGrid M, const McDev* __restrict__ T,
+                                                           u64* __restrict__ local,
+                                                           u64* __restrict__ sums) {
+    __shared__ uint8_t s_ntri[256];
+    __shared__ u64 s_wave[kMeshThreads / 64];
+    s_ntri[threadIdx.x] = T->ntri[threadIdx.x];
+    __syncthreads();
+    const u32 first = blockIdx.x * kScanBlock + threadIdx.x * kScanPer;
+    u64 v[kScanPer], tot = 0;
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) {
+        v[k] = 0;
+        if (first + k < M.nseg) {
+            const McWords W(M, first + k);
+            const u32 e = static_cast<u32>(__popcll(W.edges(0)) + __popcll(W.edges(1)) +
+                                           __popcll(W.edges(2)));
+            u32 t = 0;
+            for (u64 m = W.cubes(); m; m &= m - 1)
+                t += s_ntri[W.config(static_cast<u32>(__ffsll(static_cast<unsigned long long>(m)) - 1))];
+            v[k] = static_cast<u64>(e) | (static_cast<u64>(t) << kTriShift) |
+                   (static_cast<u64>(e || t ? 1u : 0u) << kActShift);
+        }
+        tot += v[k];
+    }
+    const u32 lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    u64 x = tot;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const u64 y = __shfl_up(x, o, 64);
+        if (lane >= static_cast<u32>(o)) x += y;
+    }
+    if (lane == 63) s_wave[w] = x;
+    __syncthreads();
+    u64 run = x - tot;
+    for (u32 k = 0; k < w; ++k) run += s_wave[k];
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) {
+        if (first + k < M.nseg) local[first + k] = run;
+        run += v[k];
+    }
+    if (threadIdx.x == kMeshThreads - 1) sums[blockIdx.x] = run;
+}
+
+// Exclusive scan of the block sums by one workgroup; totals: vertices,
+// triangles, segments to emit.
+constexpr int kSumThreads = 1024;
+struct McBase {
+    u32 verts, tris, act;
+};
+__global__ __launch_bounds__(kSumThreads) void k_mc_sums(const u64* __restrict__ sums, u32 nb,
+                                                         McBase* __restrict__ base,
+                                                         u64* __restrict__ totals) {
+    __shared__ u64 s_wave[3][kSumThreads / 64];
+    const u32 lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    u64 carry[3] = {0, 0, 0};
+    for (u32 b0 = 0; b0 < nb; b0 += kSumThreads) {
+        const u32 b = b0 + threadIdx.x;
+        const u64 v = b < nb ? sums[b] : 0ull;
+        const u64 own[3] = {scan_verts(v), scan_tris(v), scan_act(v)};
+        u64 x[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            x[q] = own[q];
+            for (int o = 1; o < 64; o <<= 1) {
+                const u64 y = __shfl_up(x[q], o, 64);
+                if (lane >= static_cast<u32>(o)) x[q] += y;
             }
+            if (lane == 63) s_wave[q][w] = x[q];
         }
-        u32 p = e | (t << 16);  // at most 3 x 64 and 8 x 64 per wave
-        for (int o = 32; o > 0; o >>= 1) p += __shfl_xor(p, o, 64);
-        if (lane == 0) {
-            const u64 seg = (static_cast<u64>(a) * r1 + b) * ntx + blockIdx.x;
-            segE[seg] = p & 0xFFFFu;
-            segT[seg] = p >> 16;
+        __syncthreads();
+        u64 off[3], all[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            off[q] = carry[q] + x[q] - own[q];
+            all[q] = 0;
+            for (u32 k = 0; k < kSumThreads / 64; ++k) {
+                if (k < w) off[q] += s_wave[q][k];
+                all[q] += s_wave[q][k];
+            }
+            carry[q] += all[q];
         }
-        cur = nxt;
+        if (b < nb)
+            base[b] = McBase{static_cast<u32>(off[0]), static_cast<u32>(off[1]),
+                             static_cast<u32>(off[2])};
+        __syncthreads();
     }
+    if (threadIdx.x < 3)
+        totals[threadIdx.x] = threadIdx.x == 0 ? carry[0] : threadIdx.x == 1 ? carry[1] : carry[2];
 }
 
-// Vertices of the segments that have any; each grid point with crossing
-// edges also records its edge mask and first vertex for k_mc_triangles.
+// The list of segments to emit, in order.
+__global__ __launch_bounds__(kMeshThreads) void k_mc_list(u32 nseg, const u64* __restrict__ local,
+                                                          const u64* __restrict__ sums,
+                                                          const McBase* __restrict__ base,
+                                                          u32* __restrict__ list) {
+    const u32 s = blockIdx.x * kMeshThreads + threadIdx.x;
+    if (s >= nseg) return;
+    const u32 blk = s / kScanBlock;
+    const u32 here = scan_act(local[s]);
+    const bool last = s + 1 == nseg || (s + 1) % kScanBlock == 0;
+    if (scan_act(last ? sums[blk] : local[s + 1]) != here) list[base[blk].act + here] = s;
+}
+
+// Vertices of the listed segments, a wave each; every grid point with crossing
+// edges also records its edge mask and first vertex.  wide (with vpt): the
+// binary64 copies that the smoothing starts from, instead of verts.
 __global__ __launch_bounds__(256) void k_mc_vertices(const float* __restrict__ g, MeshGeom G,
-                                                     float iso, u32 ntx,
-                                                     const u32* __restrict__ segE,
-                                                     const u32* __restrict__ segEoff,
+                                                     McGrid M, float iso, u32 count,
+                                                     const u32* __restrict__ list,
+                                                     const u64* __restrict__ local,
+                                                     const McBase* __restrict__ base,
                                                      uint8_t* __restrict__ emask,
                                                      u32* __restrict__ eoff,
                                                      float* __restrict__ verts,
+                                                     double* __restrict__ wide,
                                                      u32* __restrict__ vpt) {
-    const int r0 = G.r0, r1 = G.r1, r2 = G.r2;
-    const int b = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (b >= r1) return;
-    const int lane = threadIdx.x & 63;
-    const int c = blockIdx.x * 64 + lane;
-    // the wave's segments with vertices: lane l reads plane a0 + l's count
-    const int a0 = blockIdx.z * kMcEmitPlanes;
-    const u32 cnt = a0 + lane < r0
-                        ? segE[(static_cast<u64>(a0 + lane) * r1 + b) * ntx + blockIdx.x]
-                        : 0u;
-    for (unsigned long long act = __ballot(cnt != 0); act; act &= act - 1) {
-        const int a = a0 + __ffsll(act) - 1;
-        const u64 seg = (static_cast<u64>(a) * r1 + b) * ntx + blockIdx.x;
-        const u64 st[3] = {static_cast<u64>(r1) * r2, static_cast<u64>(r2), 1};
-        const u64 i = (static_cast<u64>(a) * r1 + b) * r2 + c;
-        u32 m = 0;
-        float g0 = 0.0f;
-        if (c < r2) {
-            g0 = g[i];
-            const bool in0 = g0 > iso;
-            if (a + 1 < r0 && ((g[i + st[0]] > iso) != in0)) m |= 1u;
-            if (b + 1 < r1 && ((g[i + st[1]] > iso) != in0)) m |= 2u;
-            if (c + 1 < r2 && ((g[i + st[2]] > iso) != in0)) m |= 4u;
-        }
-        u32 v = segEoff[seg] + wave_prefix(static_cast<u32>(__popc(m)), 2);
+    const u32 lane = threadIdx.x & 63;
+    for (u32 k = blockIdx.x * 4 + (threadIdx.x >> 6); k < count; k += gridDim.x * 4) {
+        const u32 s = static_cast<u32>(__builtin_amdgcn_readfirstlane(static_cast<int>(list[k])));
+        const McWords W(M, s);
+        const u64 xa = W.edges(0), xb = W.edges(1), xc = W.edges(2);
+        const u32 m = (static_cast<u32>(xa >> lane) & 1u) | ((static_cast<u32>(xb >> lane) & 1u) << 1) |
+                      ((static_cast<u32>(xc >> lane) & 1u) << 2);
         if (!m) continue;
+        const u64 below = (1ull << lane) - 1ull;
+        u32 v = base[s / kScanBlock].verts + scan_verts(local[s]) +
+                static_cast<u32>(__popcll(xa & below) + __popcll(xb & below) + __popcll(xc & below));
+        const int a = static_cast<int>(W.a), b = static_cast<int>(W.b);
+        const int c = static_cast<int>(W.tx * 64u + lane);
+        const u64 st[3] = {static_cast<u64>(M.r1) * M.r2, static_cast<u64>(M.r2), 1};
+        const u64 i = (static_cast<u64>(a) * M.r1 + b) * M.r2 + c;
+        const double v0 = static_cast<double>(g[i]);
+        double v1[3];
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax)
+            v1[ax] = (m >> ax) & 1u ? static_cast<double>(g[i + st[ax]]) : 0.0;
         emask[i] = static_cast<uint8_t>(m);
         eoff[i] = v;
         const int idx[3] = {a, b, c};
         const double lo[3] = {G.lo0, G.lo1, G.lo2}, sp[3] = {G.sp0, G.sp1, G.sp2};
-        const double v0 = static_cast<double>(g0);
+#pragma unroll
         for (int ax = 0; ax < 3; ++ax) {
             if (!((m >> ax) & 1u)) continue;
-            const double v1 = static_cast<double>(g[i + st[ax]]);
-            const double t = (static_cast<double>(iso) - v0) / (v1 - v0);
-            for (int k = 0; k < 3; ++k) {
-                const double f = k == ax ? static_cast<double>(idx[k]) + t : static_cast<double>(idx[k]);
-                verts[3 * static_cast<u64>(v) + k] = static_cast<float>(f * sp[k] + lo[k]);
+            const double t = (static_cast<double>(iso) - v0) / (v1[ax] - v0);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const double f = q == ax ? static_cast<double>(idx[q]) + t : static_cast<double>(idx[q]);
+                const float p = static_cast<float>(f * sp[q] + lo[q]);
+                if (wide) wide[3 * static_cast<u64>(v) + q] = static_cast<double>(p);
+                else verts[3 * static_cast<u64>(v) + q] = p;
             }
             if (vpt) vpt[v] = static_cast<u32>(i) << 2 | static_cast<u32>(ax);
             ++v;
@@ -942,52 +1077,52 @@ __global__ __launch_bounds__(256) void k_mc_vertices(const float* __restrict__ g
     }
 }
 
-// Triangles of the segments that have any: each vertex is the owner grid
-// point's first vertex plus the crossing edges it owns on lower axes.
-__global__ __launch_bounds__(256) void k_mc_triangles(const float* __restrict__ g, int r0, int r1,
-                                                      int r2, float iso,
-                                                      const McDev* __restrict__ T, u32 ntx,
-                                                      const u32* __restrict__ segT,
-                                                      const u32* __restrict__ segToff,
+// Offsets of a cube edge's owner corner and the edge's axis: bit ax clear, the
+// other two bits from the edge id (lower axis first).
+__device__ __forceinline__ u64 edge_owner(u64 cube, int e, u64 sa, u64 sb, int& ax) {
+    ax = e >> 2;
+    const int b0 = e & 1, b1 = (e >> 1) & 1;
+    const int oa = ax == 0 ? 0 : b0;
+    const int ob = ax == 0 ? b0 : ax == 1 ? 0 : b1;
+    const int oc = ax == 2 ? 0 : b1;
+    return cube + (oa ? sa : 0ull) + (ob ? sb : 0ull) + static_cast<u64>(oc);
+}
+
+// Triangles of the listed segments, a wave each: every vertex is the owner
+// grid point's first vertex plus the crossing edges it owns on lower axes.
+__global__ __launch_bounds__(256) void k_mc_triangles(McGrid M, const McDev* __restrict__ T,
+                                                      u32 count, const u32* __restrict__ list,
+                                                      const u64* __restrict__ local,
+                                                      const McBase* __restrict__ base,
                                                       const uint8_t* __restrict__ emask,
                                                       const u32* __restrict__ eoff,
                                                       u32* __restrict__ tris) {
-    const int b = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (b >= r1) return;
-    const int lane = threadIdx.x & 63;
-    const int c = blockIdx.x * 64 + lane;
-    // the wave's segments with triangles: lane l reads plane a0 + l's count
-    const int a0 = blockIdx.z * kMcEmitPlanes;
-    const u32 cnt = a0 + lane < r0
-                        ? segT[(static_cast<u64>(a0 + lane) * r1 + b) * ntx + blockIdx.x]
-                        : 0u;
-    for (unsigned long long act = __ballot(cnt != 0); act; act &= act - 1) {
-        const int a = a0 + __ffsll(act) - 1;
-        const u64 seg = (static_cast<u64>(a) * r1 + b) * ntx + blockIdx.x;
-        const u64 st[3] = {static_cast<u64>(r1) * r2, static_cast<u64>(r2), 1};
-        const u64 i = (static_cast<u64>(a) * r1 + b) * r2 + c;
-        u32 nt = 0;
-        int cfg = 0;
-        if (c + 1 < r2 && a + 1 < r0 && b + 1 < r1) {
-            cfg = mc_config(g, i, st[0], st[1], iso);
-            nt = T->ntri[cfg];
-        }
-        const u32 t0 = segToff[seg] + wave_prefix(nt, 4);
+    __shared__ __align__(16) McDev sT;
+    for (u32 k = threadIdx.x; k < sizeof(McDev) / 4; k += 256)
+        reinterpret_cast<u32*>(&sT)[k] = reinterpret_cast<const u32*>(T)[k];
+    __syncthreads();
+    const u32 lane = threadIdx.x & 63;
+    const u64 sa = static_cast<u64>(M.r1) * M.r2, sb = static_cast<u64>(M.r2);
+    for (u32 k = blockIdx.x * 4 + (threadIdx.x >> 6); k < count; k += gridDim.x * 4) {
+        const u32 s = static_cast<u32>(__builtin_amdgcn_readfirstlane(static_cast<int>(list[k])));
+        const McWords W(M, s);
+        const u64 act = W.cubes();
+        if (!act) continue;  // wave-uniform
+        const bool mine = (act >> lane) & 1ull;
+        const u32 cfg = mine ? W.config(lane) : 0u;
+        const u32 nt = mine ? sT.ntri[cfg] : 0u;
+        const u32 t0 = base[s / kScanBlock].tris + scan_tris(local[s]) + wave_prefix(nt, 4);
+        const u64 i = (static_cast<u64>(W.a) * M.r1 + W.b) * M.r2 + W.tx * 64u + lane;
         for (u32 t = 0; t < nt; ++t) {
+            u32 out[3];
+#pragma unroll
             for (int q = 0; q < 3; ++q) {
-                const int e = T->tri[cfg][3 * t + q];
-                const int ax = e >> 2, bb = e & 3;
-                // owner corner: bit ax clear, the other two bits from bb (lower axis first)
-                int off[3] = {0, 0, 0}, k = 0;
-                for (int x = 0; x < 3; ++x) {
-                    if (x == ax) continue;
-                    off[x] = (bb >> k) & 1;
-                    ++k;
-                }
-                const u64 o = i + off[0] * st[0] + off[1] * st[1] + off[2] * st[2];
-                const u32 rank = static_cast<u32>(__popc(emask[o] & ((1u << ax) - 1u)));
-                tris[3 * static_cast<u64>(t0 + t) + q] = eoff[o] + rank;
+                int ax;
+                const u64 o = edge_owner(i, sT.tri[cfg][3 * t + q], sa, sb, ax);
+                out[q] = eoff[o] + static_cast<u32>(__popc(emask[o] & ((1u << ax) - 1u)));
             }
+#pragma unroll
+            for (int q = 0; q < 3; ++q) tris[3 * static_cast<u64>(t0 + t) + q] = out[q];
         }
     }
 }
@@ -1005,12 +1140,79 @@ __global__ __launch_bounds__(256) void k_mc_triangles(const float* __restrict__ 
 // neighbours there, 24 over the four cubes around its edge.
 constexpr int kAdjCap = 24;
 
-// Neighbours of every vertex, from the (up to) four cubes around its grid
-// edge: the other vertices of the table triangles that contain the edge.
-__global__ __launch_bounds__(256) void k_mc_adjacency(const float* __restrict__ g, int r0, int r1,
-                                                      int r2, float iso,
-                                                      const McDev* __restrict__ T, u64 nvert,
-                                                      const u32* __restrict__ vpt,
+// Neighbours of the vertex on grid edge (i, ax), in ascending order, from the
+// (up to) four cubes around the edge: the other vertices of the table
+// triangles that contain it.  Returns their number, or CAP + 1 if there are
+// more than CAP.
+template <int CAP>
+__device__ __forceinline__ u32 mc_neighbours(const McGrid& M, const McDev& T, u32 i32, int ax,
+                                             const uint8_t* __restrict__ emask,
+                                             const u32* __restrict__ eoff, u32 (&L)[CAP]) {
+    const u32 plane = static_cast<u32>(M.r1) * static_cast<u32>(M.r2);
+    const int a = static_cast<int>(i32 / plane), rem = static_cast<int>(i32 % plane);
+    const int idx[3] = {a, rem / M.r2, rem % M.r2};
+    const int r[3] = {M.r0, M.r1, M.r2};
+    const u64 st[3] = {plane, static_cast<u64>(M.r2), 1};
+    // inside bits of points c and c + 1 of row (a, b)
+    auto two = [&](int ra, int rb, int c) -> u32 {
+        const u32 t = (static_cast<u32>(ra) * M.r1 + rb) * M.ntx + (static_cast<u32>(c) >> 6);
+        const u32 k = static_cast<u32>(c) & 63u;
+        if (k < 63u) return static_cast<u32>(M.bits[t] >> k) & 3u;
+        return static_cast<u32>(M.bits[t] >> 63) | (static_cast<u32>(M.bits[t + 1] & 1ull) << 1);
+    };
+#pragma unroll
+    for (int k = 0; k < CAP; ++k) L[k] = 0xFFFFFFFFu;
+    u32 n = 0;
+    const int u = ax == 0 ? 1 : 0, w = ax == 2 ? 1 : 2;  // the other axes, lower first
+    for (int o = 0; o < 4; ++o) {
+        const int ou = o & 1, ow = o >> 1;
+        // the cube whose lowest corner is this point - ou e_u - ow e_w
+        int q0[3] = {idx[0], idx[1], idx[2]};
+        q0[u] -= ou;
+        q0[w] -= ow;
+        if (q0[u] < 0 || q0[w] < 0 || q0[u] + 1 >= r[u] || q0[w] + 1 >= r[w]) continue;
+        const u64 qi = static_cast<u64>(i32) - ou * st[u] - ow * st[w];
+        u32 cfg = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const u32 c2 = two(q0[0] + (k & 1), q0[1] + (k >> 1), q0[2]);
+            cfg |= ((c2 & 1u) << k) | ((c2 >> 1) << (k + 4));
+        }
+        const int mine = 4 * ax + (ou | (ow << 1));  // this edge within that cube
+        for (u32 t = 0; t < T.ntri[cfg]; ++t) {
+            const uint8_t* tri = T.tri[cfg] + 3 * t;
+            if (tri[0] != mine && tri[1] != mine && tri[2] != mine) continue;
+            for (int q = 0; q < 3; ++q) {
+                const int e = tri[q];
+                if (e == mine) continue;
+                int eax;
+                const u64 oi = edge_owner(qi, e, st[0], st[1], eax);
+                u32 y = eoff[oi] + static_cast<u32>(__popc(emask[oi] & ((1u << eax) - 1u)));
+                bool seen = false;
+#pragma unroll
+                for (int k2 = 0; k2 < CAP; ++k2) seen |= L[k2] == y;
+                if (seen) continue;
+                if (n == static_cast<u32>(CAP)) return CAP + 1;
+#pragma unroll
+                for (int k2 = 0; k2 < CAP; ++k2) {  // sorted insert
+                    const bool less = y < L[k2];
+                    const u32 tk = L[k2];
+                    L[k2] = less ? y : tk;
+                    y = less ? tk : y;
+                }
+                ++n;
+            }
+        }
+    }
+    return n;
+}
+
+// Neighbours of every vertex, a thread each: in a short register list first
+// (a vertex has about six; every insertion passes the whole list), in the
+// full one for the few with more.
+constexpr int kAdjShort = 9;
+__global__ __launch_bounds__(256) void k_mc_adjacency(McGrid M, const McDev* __restrict__ T,
+                                                      u64 nvert, const u32* __restrict__ vpt,
                                                       const uint8_t* __restrict__ emask,
                                                       const u32* __restrict__ eoff,
                                                       u32* __restrict__ adj,
@@ -1022,76 +1224,26 @@ __global__ __launch_bounds__(256) void k_mc_adjacency(const float* __restrict__ 
     __syncthreads();
     const u64 v = static_cast<u64>(blockIdx.x) * 256 + threadIdx.x;
     if (v >= nvert) return;
-    // this vertex's grid edge: from grid point i (< 2^30) along axis ax
-    const u32 code = vpt[v];
-    const u32 i32 = code >> 2;
-    const int ax = static_cast<int>(code & 3u);
-    const u32 plane = static_cast<u32>(r1) * static_cast<u32>(r2);
-    const int idx[3] = {static_cast<int>(i32 / plane), static_cast<int>((i32 % plane) / r2),
-                        static_cast<int>(i32 % static_cast<u32>(r2))};
-    const u64 i = i32;
-    const int r[3] = {r0, r1, r2};
-    const u64 st[3] = {plane, static_cast<u64>(r2), 1};
-    // ascending list in registers, 0xFFFFFFFF past its end
-    u32 L[kAdjCap];
-#pragma unroll
-    for (int k = 0; k < kAdjCap; ++k) L[k] = 0xFFFFFFFFu;
-    u32 n = 0;
-    const int u = ax == 0 ? 1 : 0, w = ax == 2 ? 1 : 2;  // the other axes, lower first
-    for (int o = 0; o < 4; ++o) {
-        const int ou = o & 1, ow = o >> 1;
-        // the cube whose lowest corner is this point - ou e_u - ow e_w
-        if (idx[u] - ou < 0 || idx[w] - ow < 0 || idx[u] - ou + 1 >= r[u] ||
-            idx[w] - ow + 1 >= r[w])
-            continue;
-        const u64 qi = i - ou * st[u] - ow * st[w];
-        const int cfg = mc_config(g, qi, st[0], st[1], iso);
-        const int mine = 4 * ax + (ou | (ow << 1));  // this edge within that cube
-        for (u32 t = 0; t < sT.ntri[cfg]; ++t) {
-            const uint8_t* tri = sT.tri[cfg] + 3 * t;
-            if (tri[0] != mine && tri[1] != mine && tri[2] != mine) continue;
-            for (int q = 0; q < 3; ++q) {
-                const int e = tri[q];
-                if (e == mine) continue;
-                const int eax = e >> 2, bb = e & 3;
-                int off[3] = {0, 0, 0}, k = 0;
-                for (int x = 0; x < 3; ++x) {
-                    if (x == eax) continue;
-                    off[x] = (bb >> k) & 1;
-                    ++k;
-                }
-                const u64 oi = qi + off[0] * st[0] + off[1] * st[1] + off[2] * st[2];
-                u32 y = eoff[oi] + static_cast<u32>(__popc(emask[oi] & ((1u << eax) - 1u)));
-                bool seen = false;
-#pragma unroll
-                for (int k2 = 0; k2 < kAdjCap; ++k2) seen |= L[k2] == y;
-                if (seen) continue;
-                if (n == kAdjCap) {
-                    atomicOr(over, 1u);
-                    continue;
-                }
-#pragma unroll
-                for (int k2 = 0; k2 < kAdjCap; ++k2) {  // sorted insert
-                    const bool less = y < L[k2];
-                    const u32 tk = L[k2];
-                    L[k2] = less ? y : tk;
-                    y = less ? tk : y;
-                }
-                ++n;
-            }
-        }
-    }
+    const u32 code = vpt[v];  // this vertex's grid edge: from grid point i (< 2^30) along an axis
     u32* row = adj + v * kAdjCap;
+    u32 L[kAdjShort];
+    u32 n = mc_neighbours<kAdjShort>(M, sT, code >> 2, static_cast<int>(code & 3u), emask, eoff, L);
+    if (n <= static_cast<u32>(kAdjShort)) {
 #pragma unroll
-    for (int k = 0; k < kAdjCap; ++k)
-        if (static_cast<u32>(k) < n) row[k] = L[k];
+        for (int k = 0; k < kAdjShort; ++k)
+            if (static_cast<u32>(k) < n) row[k] = L[k];
+    } else {
+        u32 F[kAdjCap];
+        n = mc_neighbours<kAdjCap>(M, sT, code >> 2, static_cast<int>(code & 3u), emask, eoff, F);
+        if (n > static_cast<u32>(kAdjCap)) {
+            atomicOr(over, 1u);
+            n = kAdjCap;
+        }
+#pragma unroll
+        for (int k = 0; k < kAdjCap; ++k)
+            if (static_cast<u32>(k) < n) row[k] = F[k];
+    }
     deg[v] = n;
-}
-
-__global__ __launch_bounds__(kMeshThreads) void k_verts_widen(const float* __restrict__ in,
-                                                              u64 n, double* __restrict__ out) {
-    const u64 i = static_cast<u64>(blockIdx.x) * kMeshThreads + threadIdx.x;
-    if (i < n) out[i] = static_cast<double>(in[i]);
 }
 
 __global__ __launch_bounds__(kMeshThreads) void k_verts_narrow(const double* __restrict__ in,
@@ -1126,69 +1278,7 @@ __global__ __launch_bounds__(kMeshThreads) void k_mesh_laplacian(const double* _
     out[3 * v + 2] = pz + 0.5 * (sz / tw - pz);
 }
 
-// ---- exclusive scan of u32 counts (1024 per block) ----------------------------
-constexpr int kScanPer = 4;
-constexpr int kScanBlock = kMeshThreads * kScanPer;
-
-__global__ __launch_bounds__(kMeshThreads) void k_scan_local(const u32* __restrict__ in,
-                                                             u32* __restrict__ out, u64 n,
-                                                             u32* __restrict__ sums) {
-    __shared__ u32 s[kMeshThreads];
-    const u64 base = static_cast<u64>(blockIdx.x) * kScanBlock + threadIdx.x * kScanPer;
-    u32 v[kScanPer], tot = 0;
-    for (int k = 0; k < kScanPer; ++k) {
-        v[k] = base + k < n ? in[base + k] : 0u;
-        tot += v[k];
-    }
-    s[threadIdx.x] = tot;
-    __syncthreads();
-    for (int o = 1; o < kMeshThreads; o <<= 1) {
-        const u32 add = threadIdx.x >= static_cast<u32>(o) ? s[threadIdx.x - o] : 0u;
-        __syncthreads();
-        s[threadIdx.x] += add;
-        __syncthreads();
-    }
-    u32 run = s[threadIdx.x] - tot;
-    for (int k = 0; k < kScanPer; ++k) {
-        if (base + k < n) out[base + k] = run;
-        run += v[k];
-    }
-    if (threadIdx.x == kMeshThreads - 1) sums[blockIdx.x] = s[threadIdx.x];
-}
-
-__global__ __launch_bounds__(kMeshThreads) void k_scan_add(u32* __restrict__ out, u64 n,
-                                                           const u32* __restrict__ offs) {
-    const u64 base = static_cast<u64>(blockIdx.x) * kScanBlock + threadIdx.x * kScanPer;
-    const u32 add = offs[blockIdx.x];
-    for (int k = 0; k < kScanPer; ++k)
-        if (base + k < n) out[base + k] += add;
-}
-
 }  // namespace
-
-// Exclusive scan of n counts into out; returns the total (synchronous).
-static u64 scan_u32(const u32* in, u32* out, u64 n, hipStream_t s) {
-    if (n == 0) return 0;
-    const u64 nb = (n + kScanBlock - 1) / kScanBlock;
-    DeviceBuffer<u32> sums(nb), offs(nb);
-    k_scan_local<<<static_cast<u32>(nb), kMeshThreads, 0, s>>>(in, out, n, sums.data());
-    WSIM_LAUNCH_CHECK();
-    std::vector<u32> h(nb);
-    WSIM_HIP(hipMemcpyAsync(h.data(), sums.data(), nb * sizeof(u32), hipMemcpyDeviceToHost, s));
-    WSIM_HIP(hipStreamSynchronize(s));
-    u64 run = 0;
-    for (u64 k = 0; k < nb; ++k) {
-        const u64 t = h[k];
-        h[k] = static_cast<u32>(run);
-        run += t;
-        if (run > 0xFFFFFFFFull) fail(kOutOfRange, "SurfaceMesher: more than 2^32 - 1 elements");
-    }
-    WSIM_HIP(hipMemcpyAsync(offs.data(), h.data(), nb * sizeof(u32), hipMemcpyHostToDevice, s));
-    k_scan_add<<<static_cast<u32>(nb), kMeshThreads, 0, s>>>(out, n, offs.data());
-    WSIM_LAUNCH_CHECK();
-    WSIM_HIP(hipStreamSynchronize(s));
-    return run;
-}
 
 // numpy's float64 sum: sequential below 8 elements, eight running sums
 // combined pairwise up to 128, halves (a multiple of 8 first) beyond.
@@ -1510,44 +1600,64 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
     DeviceBuffer<McDev> dT(1);
     WSIM_HIP(hipMemcpyAsync(dT.data(), &T, sizeof(McTable), hipMemcpyHostToDevice, s));
     const u32 ntx = static_cast<u32>((res[2] + 63) / 64);
-    const u64 nseg = static_cast<u64>(res[0]) * res[1] * ntx;
-    fit(segE_, nseg);
-    fit(segT_, nseg);
-    fit(segEoff_, nseg);
-    fit(segToff_, nseg);
-    const u32 by = static_cast<u32>((res[1] + 3) / 4);
-    const dim3 gs(ntx, by, static_cast<u32>((res[0] + kMcPlanes - 1) / kMcPlanes));
-    k_mc_segments<<<gs, 256, 0, s>>>(grid_.data(), res[0], res[1], res[2], iso, dT.data(), ntx,
-                                     segE_.data(), segT_.data());
+    const u64 rows = static_cast<u64>(res[0]) * res[1];
+    const u64 nseg = rows * ntx;  // < 2^31: at most one per voxel
+    const u32 nb = static_cast<u32>((nseg + kScanBlock - 1) / kScanBlock);
+    fit(bits_, nseg + 1);
+    fit(local_, nseg);
+    fit(sums_, nb);
+    fit(base_, 3ull * nb);
+    fit(totals_, 3);
+    auto* base = reinterpret_cast<McBase*>(base_.data());
+    const u32 gb = static_cast<u32>(std::min<u64>((nseg + 31) / 32, 8192));
+    k_mc_bits<<<gb, 256, 0, s>>>(grid_.data(), static_cast<u32>(nseg), res[2], ntx, iso,
+                                 bits_.data());
     WSIM_LAUNCH_CHECK();
-    const u64 nvert = scan_u32(segE_.data(), segEoff_.data(), nseg, s);
-    const u64 ntri = scan_u32(segT_.data(), segToff_.data(), nseg, s);
+    const McGrid M{res[0], res[1], res[2], ntx, static_cast<u32>(nseg), bits_.data()};
+    k_mc_count<<<nb, kMeshThreads, 0, s>>>(M, dT.data(), local_.data(), sums_.data());
+    WSIM_LAUNCH_CHECK();
+    k_mc_sums<<<1, kSumThreads, 0, s>>>(sums_.data(), nb, base, totals_.data());
+    WSIM_LAUNCH_CHECK();
+    u64 totals[3];
+    WSIM_HIP(hipMemcpyAsync(totals, totals_.data(), sizeof(totals), hipMemcpyDeviceToHost, s));
+    WSIM_HIP(hipStreamSynchronize(s));
+    const u64 nvert = totals[0], ntri = totals[1];
+    const u32 nact = static_cast<u32>(totals[2]);
+    if (nvert > 0xFFFFFFFFull || ntri > 0xFFFFFFFFull)
+        fail(kOutOfRange, "SurfaceMesher: more than 2^32 - 1 elements");
     fit(verts_, 3 * std::max<u64>(nvert, 1));
     fit(tris_, 3 * std::max<u64>(ntri, 1));
-    const dim3 ge(ntx, by, static_cast<u32>((res[0] + kMcEmitPlanes - 1) / kMcEmitPlanes));
     const bool post = P.smooth_post_iters > 0 && nvert > 0;
     if (post) {
         if (nv > (1ull << 30)) fail(kOutOfRange, "SurfaceMesher: grid too large for smoothing");
         fit(vpt_, nvert);
+        for (auto& b : vd_) fit(b, 3 * nvert);
     }
-    k_mc_vertices<<<ge, 256, 0, s>>>(grid_.data(), G, iso, ntx, segE_.data(), segEoff_.data(),
-                                     emask_.data(), eoff_.data(), verts_.data(),
-                                     post ? vpt_.data() : nullptr);
-    WSIM_LAUNCH_CHECK();
-    k_mc_triangles<<<ge, 256, 0, s>>>(grid_.data(), res[0], res[1], res[2], iso, dT.data(), ntx,
-                                      segT_.data(), segToff_.data(), emask_.data(), eoff_.data(),
-                                      tris_.data());
-    WSIM_LAUNCH_CHECK();
+    if (nact) {
+        fit(list_, nact);
+        k_mc_list<<<static_cast<u32>((nseg + kMeshThreads - 1) / kMeshThreads), kMeshThreads, 0, s>>>(
+            static_cast<u32>(nseg), local_.data(), sums_.data(), base, list_.data());
+        WSIM_LAUNCH_CHECK();
+        const u32 ge = std::min<u32>(div_up(nact, 4), 16384);
+        k_mc_vertices<<<ge, 256, 0, s>>>(grid_.data(), G, M, iso, nact, list_.data(), local_.data(),
+                                         base, emask_.data(), eoff_.data(), verts_.data(),
+                                         post ? vd_[0].data() : nullptr,
+                                         post ? vpt_.data() : nullptr);
+        WSIM_LAUNCH_CHECK();
+        k_mc_triangles<<<std::min<u32>(ge, 4096), 256, 0, s>>>(
+            M, dT.data(), nact, list_.data(), local_.data(), base, emask_.data(), eoff_.data(),
+            tris_.data());
+        WSIM_LAUNCH_CHECK();
+    }
     // 7. Laplacian mesh smoothing (:138-139)
     if (post) {
         fit(adj_, nvert * kAdjCap);
         fit(deg_, nvert);
         fit(adj_over_, 1);
-        for (auto& b : vd_) fit(b, 3 * nvert);
         WSIM_HIP(hipMemsetAsync(adj_over_.data(), 0, sizeof(u32), s));
         k_mc_adjacency<<<static_cast<u32>((nvert + 255) / 256), 256, 0, s>>>(
-            grid_.data(), res[0], res[1], res[2], iso, dT.data(), nvert, vpt_.data(),
-            emask_.data(), eoff_.data(), adj_.data(), deg_.data(), adj_over_.data());
+            M, dT.data(), nvert, vpt_.data(), emask_.data(), eoff_.data(), adj_.data(), deg_.data(),
+            adj_over_.data());
         WSIM_LAUNCH_CHECK();
         u32 over = 0;
         WSIM_HIP(hipMemcpyAsync(&over, adj_over_.data(), sizeof(u32), hipMemcpyDeviceToHost, s));
@@ -1556,8 +1666,6 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
         const u64 n3 = 3 * nvert;
         const u32 g3 = static_cast<u32>((n3 + kMeshThreads - 1) / kMeshThreads);
         const u32 g1 = static_cast<u32>((nvert + kMeshThreads - 1) / kMeshThreads);
-        k_verts_widen<<<g3, kMeshThreads, 0, s>>>(verts_.data(), n3, vd_[0].data());
-        WSIM_LAUNCH_CHECK();
         int cur = 0;
         for (int it = 0; it < P.smooth_post_iters; ++it) {
             k_mesh_laplacian<<<g1, kMeshThreads, 0, s>>>(vd_[cur].data(), nvert, adj_.data(),
