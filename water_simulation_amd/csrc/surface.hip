@@ -675,8 +675,10 @@ __global__ __launch_bounds__(kMeshThreads) void k_mesh_blur(const float* __restr
     out[i] = static_cast<float>(acc);
 }
 
-// Tiled blur passes.  A strided pass (axis 0 or 1) stages, per workgroup,
-// 64 consecutive c values x (kBlurTile + 2R) positions along the axis in LDS,
+// Tiled blur passes.  A strided pass (axis 1 over each (b, c) plane, rows of
+// r2 values; axis 0 over the whole grid, rows of r1 r2 values, so its tiles
+// need not end with a row of c) stages, per workgroup, 64 consecutive
+// columns x (kBlurTile + 2R) positions along the axis in LDS,
 // with the 'reflect' ends resolved while loading, so every input is read from
 // HBM about (kBlurTile + 2R) / kBlurTile times instead of 2R + 1 times; each
 // of the 4 wave rows then forms kBlurTile / 4 outputs, taps outermost so each
@@ -692,93 +694,178 @@ __device__ __forceinline__ int reflect_fast(int k, int n) {
     return k >= 0 && k < n ? k : reflect_index(k, n);
 }
 
-template <typename In>
+// RT > 0: a tap radius R <= RT at compile time.  Each thread then widens its
+// kBlurTile / 4 + 2 RT inputs once and keeps them in registers for all taps,
+// instead of two LDS reads and two conversions per tap and output; the taps
+// between R and RT have weight 0 and add +0 (80.5 million voxels, R = 10:
+// axis 0 385 -> 273 us, axis 1 343 -> 207 us).
+template <typename In, int RT>
 __global__ __launch_bounds__(256) void k_blur_strided(const In* __restrict__ in,
-                                                      float* __restrict__ out, int r0, int r1,
-                                                      int r2, int axis,
-                                                      const double* __restrict__ w, int R) {
+                                                      float* __restrict__ out, u32 width, int len,
+                                                      u64 plane, const double* __restrict__ w,
+                                                      int Rrt) {
+    const int R = RT > 0 ? RT : Rrt;
     extern __shared__ float sb[];  // [(kBlurTile + 2R) * 64]
     const int lx = threadIdx.x & 63, ly = threadIdx.x >> 6;
-    const int c = blockIdx.x * 64 + lx;
+    const u32 c = blockIdx.x * 64 + lx;  // column of the plane: < width
     const int p0 = blockIdx.y * kBlurTile;
-    const int len = axis == 0 ? r0 : r1;
-    const u64 step = axis == 0 ? static_cast<u64>(r1) * r2 : static_cast<u64>(r2);
-    // position 0 of this column: (0, b, c) for axis 0, (a, 0, c) for axis 1
-    const u64 base = axis == 0 ? static_cast<u64>(blockIdx.z) * r2 + c
-                               : static_cast<u64>(blockIdx.z) * r1 * r2 + c;
-    const bool cin = c < r2;
+    const u64 step = width;
+    const u64 base = blockIdx.z * plane + c;  // position 0 of this column
+    const bool cin = c < width;
     const int rows = kBlurTile + 2 * R;
-    for (int k = ly; k < rows; k += 4)
-        sb[k * 64 + lx] =
-            cin ? blur_in(in, base + static_cast<u64>(reflect_fast(p0 - R + k, len)) * step)
-                : 0.0f;
+    if constexpr (RT > 0) {
+        // every load of a thread in flight before its first LDS store
+        constexpr int N = (kBlurTile + 2 * RT) / 4;
+        static_assert((kBlurTile + 2 * RT) % 4 == 0, "whole rounds of rows");
+        float v[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            v[k] = cin ? blur_in(in, base + static_cast<u64>(reflect_fast(p0 - R + ly + 4 * k, len)) *
+                                                step)
+                       : 0.0f;
+#pragma unroll
+        for (int k = 0; k < N; ++k) sb[(ly + 4 * k) * 64 + lx] = v[k];
+    } else {
+        for (int k = ly; k < rows; k += 4)
+            sb[k * 64 + lx] =
+                cin ? blur_in(in, base + static_cast<u64>(reflect_fast(p0 - R + k, len)) * step)
+                    : 0.0f;
+    }
     __syncthreads();
     constexpr int M = kBlurTile / 4;
     double acc[M];
-    const double w0 = w[R];
+    if constexpr (RT > 0) {
+        double x[M + 2 * RT];
+        const float* col = sb + ly * M * 64 + lx;
 #pragma unroll
-    for (int m = 0; m < M; ++m) acc[m] = static_cast<double>(sb[(ly + 4 * m + R) * 64 + lx]) * w0;
-    for (int j = 1; j <= R; ++j) {
-        const double wj = w[R + j];
+        for (int k = 0; k < M + 2 * RT; ++k) x[k] = static_cast<double>(col[k * 64]);
+        const double w0 = w[RT];
 #pragma unroll
-        for (int m = 0; m < M; ++m) {
-            const int k = ly + 4 * m + R;
-            acc[m] += (static_cast<double>(sb[(k - j) * 64 + lx]) +
-                       static_cast<double>(sb[(k + j) * 64 + lx])) * wj;
+        for (int m = 0; m < M; ++m) acc[m] = x[m + RT] * w0;
+#pragma unroll
+        for (int j = 1; j <= RT; ++j) {
+            const double wj = w[RT + j];
+#pragma unroll
+            for (int m = 0; m < M; ++m) acc[m] += (x[m + RT - j] + x[m + RT + j]) * wj;
+        }
+    } else {
+        const double w0 = w[R];
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+            acc[m] = static_cast<double>(sb[(ly * M + m + R) * 64 + lx]) * w0;
+        for (int j = 1; j <= R; ++j) {
+            const double wj = w[R + j];
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int k = ly * M + m + R;
+                acc[m] += (static_cast<double>(sb[(k - j) * 64 + lx]) +
+                           static_cast<double>(sb[(k + j) * 64 + lx])) * wj;
+            }
         }
     }
     if (!cin) return;
 #pragma unroll
     for (int m = 0; m < M; ++m) {
-        const int p = p0 + ly + 4 * m;
+        const int p = p0 + ly * M + m;
         if (p < len) out[base + static_cast<u64>(p) * step] = static_cast<float>(acc[m]);
     }
 }
 
-// The contiguous pass (axis 2): a workgroup takes kBlurRows (a, b) rows in
-// turn, 256 consecutive c plus 2R halo in LDS at a time, one output per
-// thread, and writes the maximum of its outputs to part[] (blurred densities
-// are >= 0, so 0 is neutral).
-// RT > 0 fixes the tap radius at compile time (RT == R); RT == 0 takes R.
-constexpr int kBlurRows = 4;  // (a, b) rows per workgroup of the contiguous pass
+// The contiguous pass (axis 2): each wave takes kBlurRows (a, b) rows in turn,
+// 256 consecutive c plus 2R halo in LDS at a time, four consecutive outputs
+// per lane (the inputs read as 16-byte words and widened once: 80.5 million
+// voxels, R = 10, 375 -> 215 us), and the workgroup writes the maximum of
+// its outputs to part[] (blurred densities are >= 0, so 0 is neutral).
+// RT > 0: a tap radius R <= RT at compile time (weight 0 beyond R); RT == 0
+// takes R, one tap after the other from LDS.
+constexpr int kBlurRows = 4;  // (a, b) rows per wave of the contiguous pass
+constexpr int kBlurSeg = 256;
+__host__ __device__ constexpr int blur_row_floats(int R) { return (kBlurSeg + 2 * R + 3) / 4 * 4; }
 
 template <int RT>
 __global__ __launch_bounds__(256) void k_blur_rows(const float* __restrict__ in,
-                                                   float* __restrict__ out, int r1, int r2,
+                                                   float* __restrict__ out, u64 rows, int r2,
                                                    const double* __restrict__ w, int Rrt,
                                                    float* __restrict__ part) {
     const int R = RT > 0 ? RT : Rrt;
-    constexpr int kTapUnroll = RT > 0 ? RT : 1;
-    extern __shared__ float sb[];  // [256 + 2R]
+    extern __shared__ __align__(16) float sb[];  // one row segment per wave
     __shared__ float wmax[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float* const seg = sb + wave * blur_row_floats(R);
     float vmax = 0.0f;
-    const int b1 = min((static_cast<int>(blockIdx.x) + 1) * kBlurRows, r1);
-    for (int b = blockIdx.x * kBlurRows; b < b1; ++b) {
-        const u64 row = (static_cast<u64>(blockIdx.y) * r1 + b) * r2;
-        for (int c0 = 0; c0 < r2; c0 += 256) {
-            __syncthreads();  // the previous segment's taps are read
-            for (int k = threadIdx.x; k < 256 + 2 * R; k += 256)
-                sb[k] = in[row + reflect_fast(c0 - R + k, r2)];
-            __syncthreads();
-            const int k = threadIdx.x + R;
-            double acc = static_cast<double>(sb[k]) * w[R];
-#pragma unroll kTapUnroll
-            for (int j = 1; j <= R; ++j)
-                acc += (static_cast<double>(sb[k - j]) + static_cast<double>(sb[k + j])) * w[R + j];
-            const int c = c0 + threadIdx.x;
-            const float v = static_cast<float>(acc);
-            if (c < r2) {
-                out[row + c] = v;
-                vmax = fmaxf(vmax, v);
+    const u64 first = (static_cast<u64>(blockIdx.x) * 4 + wave) * kBlurRows;
+    const u64 last = min(first + kBlurRows, rows);
+    // the wave's own LDS: its instructions stay in order
+    auto sync = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+    // RT > 0: the next segment's loads are in flight while this one is summed
+    constexpr int kLoads = RT > 0 ? (kBlurSeg + 2 * RT + 63) / 64 : 1;
+    float ahead[kLoads];
+    auto request = [&](u64 r, int c0) {
+        const u64 row = r * r2;
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u)
+            ahead[u] = in[row + reflect_fast(min(c0 - R + lane + 64 * u, c0 + kBlurSeg + R - 1), r2)];
+    };
+    if constexpr (RT > 0)
+        if (first < last) request(first, 0);
+    for (u64 r = first; r < last; ++r) {
+        const u64 row = r * r2;
+        for (int c0 = 0; c0 < r2; c0 += kBlurSeg) {
+            sync();
+            if constexpr (RT > 0) {
+#pragma unroll
+                for (int u = 0; u < kLoads; ++u)
+                    if (lane + 64 * u < blur_row_floats(RT)) seg[lane + 64 * u] = ahead[u];
+                const bool more = c0 + kBlurSeg < r2;
+                if (more || r + 1 < last) request(more ? r : r + 1, more ? c0 + kBlurSeg : 0);
+            } else {
+                for (int k = lane; k < kBlurSeg + 2 * R; k += 64)
+                    seg[k] = in[row + reflect_fast(c0 - R + k, r2)];
+            }
+            sync();
+            double acc[4];
+            if constexpr (RT > 0) {
+                constexpr int N = (4 + 2 * RT + 3) / 4 * 4;
+                double x[N];
+#pragma unroll
+                for (int k = 0; k < N; k += 4) {
+                    // the last lane's padding lies inside the segment's
+                    const float4 f = *reinterpret_cast<const float4*>(seg + 4 * lane + k);
+                    x[k] = f.x, x[k + 1] = f.y, x[k + 2] = f.z, x[k + 3] = f.w;
+                }
+#pragma unroll
+                for (int m = 0; m < 4; ++m) acc[m] = x[m + RT] * w[RT];
+#pragma unroll
+                for (int j = 1; j <= RT; ++j) {
+                    const double wj = w[RT + j];
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) acc[m] += (x[m + RT - j] + x[m + RT + j]) * wj;
+                }
+            } else {
+                for (int m = 0; m < 4; ++m) {
+                    const int k = 4 * lane + m + R;
+                    acc[m] = static_cast<double>(seg[k]) * w[R];
+                    for (int j = 1; j <= R; ++j)
+                        acc[m] += (static_cast<double>(seg[k - j]) + static_cast<double>(seg[k + j])) *
+                                  w[R + j];
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const int c = c0 + 4 * lane + m;
+                const float v = static_cast<float>(acc[m]);
+                if (c < r2) {
+                    out[row + c] = v;
+                    vmax = fmaxf(vmax, v);
+                }
             }
         }
     }
     for (int o = 32; o > 0; o >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, o, 64));
-    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = vmax;
+    if (lane == 0) wmax[wave] = vmax;
     __syncthreads();
     if (threadIdx.x == 0)
-        part[static_cast<u64>(blockIdx.y) * gridDim.x + blockIdx.x] =
-            fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+        part[blockIdx.x] = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
 }
 
 __global__ __launch_bounds__(kMeshThreads) void k_mesh_max(const float* __restrict__ g, u64 nv,
@@ -1529,6 +1616,11 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
     if (P.smooth_sigma > 0.0) {
         w = gaussian_weights(P.smooth_sigma, &R);
         if (P.weights) std::memcpy(w.data(), P.weights, w.size() * sizeof(double));
+        if (R <= 16) {  // the compile-time radii of the tiled passes (0 weights change no sum)
+            const size_t pad = static_cast<size_t>((R <= 10 ? 10 : 16) - R);
+            w.insert(w.begin(), pad, 0.0);
+            w.insert(w.end(), pad, 0.0);
+        }
         dw = DeviceBuffer<double>(w.size());
         WSIM_HIP(hipMemcpyAsync(dw.data(), w.data(), w.size() * sizeof(double),
                                 hipMemcpyHostToDevice, s));
@@ -1548,29 +1640,34 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
     };
     float gmax;
     if (P.smooth_sigma > 0.0 && R <= kBlurMaxR) {
-        // counts -> grid_ (axis 0) -> tmp_ (axis 1) -> grid_ (axis 2)
-        const size_t lds = static_cast<size_t>(kBlurTile + 2 * R) * 64 * sizeof(float);
-        const u32 tx = static_cast<u32>((res[2] + 63) / 64);
-        const dim3 g0(tx, static_cast<u32>((res[0] + kBlurTile - 1) / kBlurTile), static_cast<u32>(res[1]));
-        k_blur_strided<u32><<<g0, 256, lds, s>>>(count, grid_.data(), res[0], res[1], res[2], 0,
-                                                 dw.data(), R);
-        WSIM_LAUNCH_CHECK();
-        const dim3 g1(tx, static_cast<u32>((res[1] + kBlurTile - 1) / kBlurTile), static_cast<u32>(res[0]));
-        k_blur_strided<float><<<g1, 256, lds, s>>>(grid_.data(), tmp_.data(), res[0], res[1],
-                                                   res[2], 1, dw.data(), R);
-        WSIM_LAUNCH_CHECK();
-        const dim3 g2(static_cast<u32>((res[1] + kBlurRows - 1) / kBlurRows),
-                      static_cast<u32>(res[0]));
-        const u64 nparts = static_cast<u64>(g2.x) * g2.y;
+        // counts -> grid_ (axis 0) -> tmp_ (axis 1) -> grid_ (axis 2), with
+        // compile-time radii up to 16 (weights padded with zeros)
+        const int RT = R <= 10 ? 10 : R <= 16 ? 16 : R;
+        const u32 area = static_cast<u32>(res[1]) * static_cast<u32>(res[2]);
+        const dim3 g0((area + 63) / 64, static_cast<u32>((res[0] + kBlurTile - 1) / kBlurTile), 1);
+        const dim3 g1(static_cast<u32>((res[2] + 63) / 64),
+                      static_cast<u32>((res[1] + kBlurTile - 1) / kBlurTile), static_cast<u32>(res[0]));
+        const u64 rows = static_cast<u64>(res[0]) * res[1];
+        const u64 nparts = (rows + 4 * kBlurRows - 1) / (4 * kBlurRows);
         fit(part_, nparts);
-        const size_t lr = (256 + 2 * R) * sizeof(float);
-        if (R == 10)  // sigma 2.5, the tool's default: unrolled taps
-            k_blur_rows<10><<<g2, 256, lr, s>>>(tmp_.data(), grid_.data(), res[1], res[2],
-                                                dw.data(), R, part_.data());
-        else
-            k_blur_rows<0><<<g2, 256, lr, s>>>(tmp_.data(), grid_.data(), res[1], res[2],
-                                               dw.data(), R, part_.data());
-        WSIM_LAUNCH_CHECK();
+        auto blur = [&](auto rt) {
+            constexpr int T = decltype(rt)::value;
+            const size_t lds = static_cast<size_t>(kBlurTile + 2 * RT) * 64 * sizeof(float);
+            k_blur_strided<u32, T><<<g0, 256, lds, s>>>(count, grid_.data(), area, res[0], nv,
+                                                        dw.data(), RT);
+            WSIM_LAUNCH_CHECK();
+            k_blur_strided<float, T><<<g1, 256, lds, s>>>(grid_.data(), tmp_.data(),
+                                                          static_cast<u32>(res[2]), res[1], area,
+                                                          dw.data(), RT);
+            WSIM_LAUNCH_CHECK();
+            k_blur_rows<T><<<static_cast<u32>(nparts), 256,
+                             4 * blur_row_floats(RT) * sizeof(float), s>>>(
+                tmp_.data(), grid_.data(), rows, res[2], dw.data(), RT, part_.data());
+            WSIM_LAUNCH_CHECK();
+        };
+        if (RT == 10) blur(std::integral_constant<int, 10>{});
+        else if (RT == 16) blur(std::integral_constant<int, 16>{});
+        else blur(std::integral_constant<int, 0>{});
         gmax = max_of(part_.data(), nparts);
     } else {
         k_mesh_to_float<<<gv, kMeshThreads, 0, s>>>(count, grid_.data(), nv);
