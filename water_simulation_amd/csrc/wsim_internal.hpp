@@ -181,7 +181,7 @@ private:
     DeviceBuffer<float> grid_, tmp_, verts_, part_;
     DeviceBuffer<u32> tris_, count_, eoff_;
     DeviceBuffer<u64> bits_, local_, sums_, totals_;  // per 64-point row segment, scan blocks
-    DeviceBuffer<u32> base_, list_;
+    DeviceBuffer<u32> base_;
     DeviceBuffer<uint8_t> emask_;
     DeviceBuffer<double> pts_[2];  // binary64 points, smoothed in place
     DeviceBuffer<u32> knn_keys_[2], knn_vals_[2], knn_hist_, knn_cs_;
