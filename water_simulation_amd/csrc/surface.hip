@@ -874,15 +874,16 @@ __global__ __launch_bounds__(256) void k_blur_rows(const float* __restrict__ in,
 
 __global__ __launch_bounds__(kMeshThreads) void k_mesh_max(const float* __restrict__ g, u64 nv,
                                                            float* __restrict__ part) {
-    __shared__ float s[kMeshThreads];
+    __shared__ float s[kMeshThreads / 64];
     float m = -INFINITY;
     const u64 stride = static_cast<u64>(gridDim.x) * kMeshThreads;
     for (u64 i = static_cast<u64>(blockIdx.x) * kMeshThreads + threadIdx.x; i < nv; i += stride)
         m = fmaxf(m, g[i]);
-    s[threadIdx.x] = m;
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = m;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int k = 1; k < kMeshThreads; ++k) m = fmaxf(m, s[k]);
+        for (int k = 1; k < kMeshThreads / 64; ++k) m = fmaxf(m, s[k]);
         part[blockIdx.x] = m;
     }
 }
@@ -1510,15 +1511,26 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
     }
     k_mesh_points<<<gp, kMeshThreads, 0, s>>>(xyz, n, P.swap_yz ? 1 : 0, pts_[0].data());
     WSIM_LAUNCH_CHECK();
-    const u32 nbb = std::min<u32>(gp, 1024);
-    DeviceBuffer<double> part(kBoundsPart * static_cast<size_t>(nbb));
-    auto bounds = [&](const double* pts, double* mn, double* mx) {
-        k_mesh_bounds<<<nbb, kMeshThreads, 0, s>>>(pts, n, part.data());
-        WSIM_LAUNCH_CHECK();
-        std::vector<double> hp(kBoundsPart * static_cast<size_t>(nbb));
-        WSIM_HIP(hipMemcpyAsync(hp.data(), part.data(), hp.size() * sizeof(double),
-                                hipMemcpyDeviceToHost, s));
+    // small results are read through one pinned buffer, and the small device
+    // buffers stay allocated between runs (an allocation or a free waits for
+    // the device)
+    auto fit = [](auto& b, u64 want) {
+        if (b.size() < want) b = std::remove_reference_t<decltype(b)>(want);
+    };
+    constexpr u32 kBoundsBlocks = 256;
+    const u32 nbb = std::min<u32>(gp, kBoundsBlocks);
+    fit(bpart_, kBoundsPart * static_cast<u64>(kBoundsBlocks));
+    fit(hostbuf_, kBoundsPart * static_cast<u64>(kBoundsBlocks));
+    auto read_back = [&](void* dst, const void* src, size_t bytes) {
+        WSIM_HIP(hipMemcpyAsync(hostbuf_.data(), src, bytes, hipMemcpyDeviceToHost, s));
         WSIM_HIP(hipStreamSynchronize(s));
+        std::memcpy(dst, hostbuf_.data(), bytes);
+    };
+    auto bounds = [&](const double* pts, double* mn, double* mx) {
+        k_mesh_bounds<<<nbb, kMeshThreads, 0, s>>>(pts, n, bpart_.data());
+        WSIM_LAUNCH_CHECK();
+        double hp[kBoundsPart * kBoundsBlocks];
+        read_back(hp, bpart_.data(), kBoundsPart * static_cast<size_t>(nbb) * sizeof(double));
         for (int a = 0; a < 3; ++a) {
             mn[a] = INFINITY;
             mx[a] = -INFINITY;
@@ -1630,9 +1642,6 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
     info_.spacing[0] = G.sp0, info_.spacing[1] = G.sp1, info_.spacing[2] = G.sp2;
     const u32 gv = static_cast<u32>((nv + kMeshThreads - 1) / kMeshThreads);
     // grid-sized work buffers are kept between runs and grow as needed
-    auto fit = [](auto& b, u64 want) {
-        if (b.size() < want) b = std::remove_reference_t<decltype(b)>(want);
-    };
     fit(grid_, nv);
     fit(tmp_, nv);
     fit(count_, nv);
@@ -1646,7 +1655,6 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
     // 4. blur and 5. the maximum for the iso level
     int R = 0;
     std::vector<double> w;
-    DeviceBuffer<double> dw;
     if (P.smooth_sigma > 0.0) {
         w = gaussian_weights(P.smooth_sigma, &R);
         if (P.weights) std::memcpy(w.data(), P.weights, w.size() * sizeof(double));
@@ -1655,21 +1663,23 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
             w.insert(w.begin(), pad, 0.0);
             w.insert(w.end(), pad, 0.0);
         }
-        dw = DeviceBuffer<double>(w.size());
-        WSIM_HIP(hipMemcpyAsync(dw.data(), w.data(), w.size() * sizeof(double),
+        fit(weights_, w.size());
+        WSIM_HIP(hipMemcpyAsync(weights_.data(), w.data(), w.size() * sizeof(double),
                                 hipMemcpyHostToDevice, s));
     }
     auto max_of = [&](const float* a, u64 na) {
-        const u32 nbm = static_cast<u32>(std::min<u64>((na + kMeshThreads - 1) / kMeshThreads, 1024));
-        DeviceBuffer<float> mpart(nbm);
-        k_mesh_max<<<nbm, kMeshThreads, 0, s>>>(a, na, mpart.data());
+        constexpr u32 kMaxBlocks = 1024;
+        static_assert(kMaxBlocks * sizeof(float) <= kBoundsPart * kBoundsBlocks * sizeof(double),
+                      "read through hostbuf_");
+        const u32 nbm = static_cast<u32>(
+            std::min<u64>((na + kMeshThreads - 1) / kMeshThreads, kMaxBlocks));
+        fit(mpart_, kMaxBlocks);
+        k_mesh_max<<<nbm, kMeshThreads, 0, s>>>(a, na, mpart_.data());
         WSIM_LAUNCH_CHECK();
-        std::vector<float> hm(nbm);
-        WSIM_HIP(hipMemcpyAsync(hm.data(), mpart.data(), nbm * sizeof(float),
-                                hipMemcpyDeviceToHost, s));
-        WSIM_HIP(hipStreamSynchronize(s));
+        float hm[kMaxBlocks];
+        read_back(hm, mpart_.data(), nbm * sizeof(float));
         float m = -INFINITY;
-        for (float v : hm) m = std::fmax(m, v);
+        for (u32 k = 0; k < nbm; ++k) m = std::fmax(m, hm[k]);
         return m;
     };
     float gmax;
@@ -1688,15 +1698,15 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
             constexpr int T = decltype(rt)::value;
             const size_t lds = static_cast<size_t>(kBlurTile + 2 * RT) * 64 * sizeof(float);
             k_blur_strided<u32, T><<<g0, 256, lds, s>>>(count, grid_.data(), area, res[0], nv,
-                                                        dw.data(), RT);
+                                                        weights_.data(), RT);
             WSIM_LAUNCH_CHECK();
             k_blur_strided<float, T><<<g1, 256, lds, s>>>(grid_.data(), tmp_.data(),
                                                           static_cast<u32>(res[2]), res[1], area,
-                                                          dw.data(), RT);
+                                                          weights_.data(), RT);
             WSIM_LAUNCH_CHECK();
             k_blur_rows<T><<<static_cast<u32>(nparts), 256,
                              4 * blur_row_floats(RT) * sizeof(float), s>>>(
-                tmp_.data(), grid_.data(), rows, res[2], dw.data(), RT, part_.data());
+                tmp_.data(), grid_.data(), rows, res[2], weights_.data(), RT, part_.data());
             WSIM_LAUNCH_CHECK();
         };
         if (RT == 10) blur(std::integral_constant<int, 10>{});
@@ -1711,7 +1721,7 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
             float* dst = tmp_.data();
             for (int axis = 0; axis < 3; ++axis) {
                 k_mesh_blur<<<gv, kMeshThreads, 0, s>>>(src, dst, res[0], res[1], res[2], axis,
-                                                        dw.data(), R);
+                                                        weights_.data(), R);
                 WSIM_LAUNCH_CHECK();
                 std::swap(src, dst);
             }
@@ -1728,8 +1738,12 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
     // 6. marching cubes
     const McTable& T = mc_table();
     static_assert(sizeof(McDev) == sizeof(McTable), "table layout");
-    DeviceBuffer<McDev> dT(1);
-    WSIM_HIP(hipMemcpyAsync(dT.data(), &T, sizeof(McTable), hipMemcpyHostToDevice, s));
+    if (table_.size() == 0) {  // uploaded once
+        DeviceBuffer<uint8_t> t(sizeof(McTable));
+        WSIM_HIP(hipMemcpyAsync(t.data(), &T, sizeof(McTable), hipMemcpyHostToDevice, s));
+        table_ = std::move(t);
+    }
+    const McDev* dT = reinterpret_cast<const McDev*>(table_.data());
     const u32 ntx = static_cast<u32>((res[2] + 63) / 64);
     const u64 rows = static_cast<u64>(res[0]) * res[1];
     const u64 nseg = rows * ntx;  // < 2^31: at most one per voxel
@@ -1745,13 +1759,12 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
                                  bits_.data());
     WSIM_LAUNCH_CHECK();
     const McGrid M{res[0], res[1], res[2], ntx, static_cast<u32>(nseg), bits_.data()};
-    k_mc_count<<<nb, kMeshThreads, 0, s>>>(M, dT.data(), local_.data(), sums_.data());
+    k_mc_count<<<nb, kMeshThreads, 0, s>>>(M, dT, local_.data(), sums_.data());
     WSIM_LAUNCH_CHECK();
     k_mc_sums<<<1, kSumThreads, 0, s>>>(sums_.data(), nb, base, totals_.data());
     WSIM_LAUNCH_CHECK();
     u64 totals[2];
-    WSIM_HIP(hipMemcpyAsync(totals, totals_.data(), sizeof(totals), hipMemcpyDeviceToHost, s));
-    WSIM_HIP(hipStreamSynchronize(s));
+    read_back(totals, totals_.data(), sizeof(totals));
     const u64 nvert = totals[0], ntri = totals[1];
     if (nvert > 0xFFFFFFFFull || ntri > 0xFFFFFFFFull)
         fail(kOutOfRange, "SurfaceMesher: more than 2^32 - 1 elements");
@@ -1768,7 +1781,7 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
             grid_.data(), G, M, iso, local_.data(), sums_.data(), base, emask_.data(), eoff_.data(),
             verts_.data(), post ? vd_[0].data() : nullptr, post ? vpt_.data() : nullptr);
         WSIM_LAUNCH_CHECK();
-        k_mc_triangles<<<nb, kMeshThreads, 0, s>>>(M, dT.data(), local_.data(), sums_.data(), base,
+        k_mc_triangles<<<nb, kMeshThreads, 0, s>>>(M, dT, local_.data(), sums_.data(), base,
                                                    emask_.data(), eoff_.data(), tris_.data());
         WSIM_LAUNCH_CHECK();
     }
@@ -1779,13 +1792,9 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
         fit(adj_over_, 1);
         WSIM_HIP(hipMemsetAsync(adj_over_.data(), 0, sizeof(u32), s));
         k_mc_adjacency<<<static_cast<u32>((nvert + 255) / 256), 256, 0, s>>>(
-            M, dT.data(), nvert, vpt_.data(), emask_.data(), eoff_.data(), adj_.data(), deg_.data(),
+            M, dT, nvert, vpt_.data(), emask_.data(), eoff_.data(), adj_.data(), deg_.data(),
             adj_over_.data());
         WSIM_LAUNCH_CHECK();
-        u32 over = 0;
-        WSIM_HIP(hipMemcpyAsync(&over, adj_over_.data(), sizeof(u32), hipMemcpyDeviceToHost, s));
-        WSIM_HIP(hipStreamSynchronize(s));
-        if (over) fail(kRuntimeError, "SurfaceMesher: a vertex with more than 24 neighbours");
         const u64 n3 = 3 * nvert;
         const u32 g3 = static_cast<u32>((n3 + kMeshThreads - 1) / kMeshThreads);
         const u32 g1 = static_cast<u32>((nvert + kMeshThreads - 1) / kMeshThreads);
@@ -1798,6 +1807,9 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
         }
         k_verts_narrow<<<g3, kMeshThreads, 0, s>>>(vd_[cur].data(), n3, verts_.data());
         WSIM_LAUNCH_CHECK();
+        u32 over = 0;  // (the lists are cut at their capacity, so the passes above stay in bounds)
+        read_back(&over, adj_over_.data(), sizeof(u32));
+        if (over) fail(kRuntimeError, "SurfaceMesher: a vertex with more than 24 neighbours");
     }
     WSIM_HIP(hipStreamSynchronize(s));
     info_.n_vertices = nvert;

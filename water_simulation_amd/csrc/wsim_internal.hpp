@@ -182,6 +182,10 @@ private:
     DeviceBuffer<u32> tris_, count_, eoff_;
     DeviceBuffer<u64> bits_, local_, sums_, totals_;  // per 64-point row segment, scan blocks
     DeviceBuffer<u32> base_;
+    DeviceBuffer<double> bpart_, weights_;
+    DeviceBuffer<float> mpart_;
+    DeviceBuffer<uint8_t> table_;   // marching-cubes table, uploaded once
+    PinnedBuffer<double> hostbuf_;  // small results on their way to the host
     DeviceBuffer<uint8_t> emask_;
     DeviceBuffer<double> pts_[2];  // binary64 points, smoothed in place
     DeviceBuffer<u32> knn_keys_[2], knn_vals_[2], knn_hist_, knn_cs_;
