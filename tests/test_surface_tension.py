@@ -191,6 +191,22 @@ def test_gpu_tension_step_matches_oracle(coincident):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,squeeze", [
+    (1, 1.0), (2, 1.0), (63, 1.0), (64, 1.0), (65, 1.0),  # a workgroup holds 64 particles
+    (257, 0.75),   # one tile and a particle; lists past the four lanes' first 32 entries
+    (1000, 0.45),  # lists past their depth: the stencil walk
+])
+def test_gpu_tension_edges_match_oracle(n, squeeze):
+    x, v, _, cfg = random_box(n=1000, seed=n, boundary=False, enable_surface_tension=True,
+                              surface_tension=GAMMA)
+    x, v = (0.2 + squeeze * (x[:n] - 0.2)).astype(np.float32), v[:n]
+    p = Pair(x, v, None, cfg)
+    for k in range(2):
+        p.step(2e-4)
+        p.compare(f"step {k}")
+
+
+@pytest.mark.gpu
 def test_gpu_tension_changes_the_step():
     x, v, xb, cfg = _tension_box(7)
     on = Pair(x, v, xb, cfg)

@@ -643,93 +643,58 @@ __device__ __forceinline__ float cohesion_C(float r, const TensionArgs& T) {
     return T.sig * (2.0f * t - T.c6);
 }
 
-template <int NT>
-__global__ __launch_bounds__(NT) void k_tension_normals(Nbr P, PairList L,
-                                                        const float4* __restrict__ xs,
-                                                        const float* __restrict__ rho,
-                                                        TensionArgs T, float4* __restrict__ nrm) {
-    const u32 i = slot_index<NT>(P.remap);
-    if (i >= P.nslots) return;
-    const SceneSeg& G = P.seg[scene_of_slot(P, i)];
-    if (i - G.off >= G.n) return;
-    const float4 p = xs[i];
-    float sx = 0.0f, sy = 0.0f, sz = 0.0f;
-    // zero-gradient pairs add +-0 to sums that never hold -0: left out
-    auto add = [&](const float4& q, float c, float rj) {
-        const float gx = (p.x - q.x) * c, gy = (p.y - q.y) * c, gz = (p.z - q.z) * c;
-        const float f = P.mass / rj;
-        sx += f * gx;
-        sy += f * gy;
-        sz += f * gz;
-    };
-    const u32 cf = L.cnt[i] & 0xFFFFu;
-    if (cf <= L.kf) {
-        const StageRanges R = L.plan[i / kTile];
-        for (u32 k = 0; k < cf; ++k) {
-            u32 j;
-            float c;
-            fluid_entry(L, R, k, i, j, c);
-            const float4 q = xs[j];
-            add(q, R.total ? pair_c(p, q, P.sp) : c, rho[j]);
-        }
-    } else {
-        for_stencil(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, [&](u32 s) {
-            if (s == i) return;
-            const float4 q = xs[s];
-            const float r2 = dist2(p.x - q.x, p.y - q.y, p.z - q.z);
-            if (r2 >= P.sp.far2) return;
-            const float c = spline_gradc(pair_sqrt(r2, P.sp), P.sp);
-            if (c != 0.0f) add(q, c, rho[s]);
-        });
-    }
-    nrm[i] = make_float4(T.L * sx, T.L * sy, T.L * sz, 0.0f);
+__device__ __forceinline__ float3 tension_normal_term(const float4& p, const float4& q, float c,
+                                                      float rj, float mass) {
+    const float gx = (p.x - q.x) * c, gy = (p.y - q.y) * c, gz = (p.z - q.z) * c;
+    const float f = mass / rj;
+    return make_float3(f * gx, f * gy, f * gz);
 }
-
-template <int NT>
-__global__ __launch_bounds__(NT) void k_tension_force(Nbr P, PairList L,
-                                                      const float4* __restrict__ xs,
-                                                      const float* __restrict__ rho,
-                                                      const float4* __restrict__ nrm,
-                                                      TensionArgs T, float4* __restrict__ vs) {
-    const u32 i = slot_index<NT>(P.remap);
-    if (i >= P.nslots) return;
-    const SceneSeg& G = P.seg[scene_of_slot(P, i)];
-    if (i - G.off >= G.n) return;
-    const float4 p = xs[i];
-    const float4 ni = nrm[i];
-    const float rho_i = rho[i];
-    const float mg = -T.gamma * P.mass;
-    float ax = 0.0f, ay = 0.0f, az = 0.0f;
-    auto add = [&](const float4& q, float rj, const float4& nj) {
-        const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
-        const float d = sqrtf(dist2(rx, ry, rz));
-        const float K = 2.0f * T.rho0 / (rho_i + rj);
-        const float sc = d > 0.0f ? mg * cohesion_C(d, T) / d : 0.0f;
-        ax += K * (sc * rx + -T.gamma * (ni.x - nj.x));
-        ay += K * (sc * ry + -T.gamma * (ni.y - nj.y));
-        az += K * (sc * rz + -T.gamma * (ni.z - nj.z));
-    };
-    const u32 cf = L.cnt[i] & 0xFFFFu;
-    if (cf <= L.kf) {
-        // a complete list holds every in-support pair but the self pair
-        const StageRanges R = L.plan[i / kTile];
-        for (u32 k = 0; k < cf; ++k) {
-            u32 j;
-            float c;
-            fluid_entry(L, R, k, i, j, c);
-            add(xs[j], rho[j], nrm[j]);
-        }
-    } else {
-        for_stencil(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, [&](u32 s) {
-            if (s == i) return;
-            const float4 q = xs[s];
-            if (dist2(p.x - q.x, p.y - q.y, p.z - q.z) >= P.sp.far2) return;
-            add(q, rho[s], nrm[s]);
-        });
-    }
-    const float4 v = vs[i];
-    const float dt = G.dt;
-    vs[i] = make_float4(v.x + dt * ax, v.y + dt * ay, v.z + dt * az, 0.0f);
+__device__ __forceinline__ float3 tension_force_term(const float4& p, const float4& ni,
+                                                     float rho_i, const float4& q,
+                                                     const float4& nj, float rj, float mass,
+                                                     const TensionArgs& T) {
+    const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
+    const float d = sqrtf(dist2(rx, ry, rz));
+    const float K = 2.0f * T.rho0 / (rho_i + rj);
+    const float mg = -T.gamma * mass;
+    const float sc = d > 0.0f ? mg * cohesion_C(d, T) / d : 0.0f;
+    return make_float3(K * (sc * rx + -T.gamma * (ni.x - nj.x)),
+                       K * (sc * ry + -T.gamma * (ni.y - nj.y)),
+                       K * (sc * rz + -T.gamma * (ni.z - nj.z)));
+}
+// The sums over the stencil, for particles whose list is incomplete.
+__device__ __forceinline__ void tension_normal_walk(const Nbr& P, const SceneSeg& G, u32 i,
+                                                    const float4& p, const float4* xs,
+                                                    const float* rho, float& sx, float& sy,
+                                                    float& sz) {
+    for_stencil(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, [&](u32 s) {
+        if (s == i) return;
+        const float4 q = xs[s];
+        const float r2 = dist2(p.x - q.x, p.y - q.y, p.z - q.z);
+        if (r2 >= P.sp.far2) return;
+        const float c = spline_gradc(pair_sqrt(r2, P.sp), P.sp);
+        // zero-gradient pairs add +-0 to sums that never hold -0: left out
+        if (c == 0.0f) return;
+        const float3 t = tension_normal_term(p, q, c, rho[s], P.mass);
+        sx += t.x;
+        sy += t.y;
+        sz += t.z;
+    });
+}
+__device__ __forceinline__ void tension_force_walk(const Nbr& P, const SceneSeg& G, u32 i,
+                                                   const float4& p, const float4& ni, float rho_i,
+                                                   const float4* xs, const float* rho,
+                                                   const float4* nrm, const TensionArgs& T,
+                                                   float& ax, float& ay, float& az) {
+    for_stencil(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, [&](u32 s) {
+        if (s == i) return;
+        const float4 q = xs[s];
+        if (dist2(p.x - q.x, p.y - q.y, p.z - q.z) >= P.sp.far2) return;
+        const float3 t = tension_force_term(p, ni, rho_i, q, nrm[s], rho[s], P.mass, T);
+        ax += t.x;
+        ay += t.y;
+        az += t.z;
+    });
 }
 
 // rho_dot terms (dfsph_kernels.cu:210, 222) for one pair with gradient scalar c.
@@ -2174,6 +2139,88 @@ __global__ __launch_bounds__(NS) void k_xsph_q(Nbr P, PairList L, const float4* 
     if (g == 0) vout[i] = make_float4(vi.x + dx, vi.y + dy, vi.z + dz, 0.0f);
 }
 
+// Surface tension, four lanes per particle at every size: one lane's chain of
+// gathers, a root and quotients per pair bounds these passes, and no staged
+// variant competes.  One lane -> four lanes per particle, us:
+//   normals  4k 17.6 -> 5.3   64k 21.3 -> 9.2    262k 34.4 -> 26.1   1M 121.7 -> 83.5
+//   force    4k 18.7 -> 5.8   64k 20.4 -> 12.3   262k 39.8 -> 36.0   1M 178.9 -> 112.5
+__global__ __launch_bounds__(NS) void k_tension_normals(Nbr P, PairList L,
+                                                          const float4* __restrict__ xs,
+                                                          const float* __restrict__ rho,
+                                                          TensionArgs T,
+                                                          float4* __restrict__ nrm) {
+    const QuadLane Q(P);
+    const u32 i = Q.i, g = Q.g;
+    const SceneSeg& G = P.seg[scene_of_slot(P, i)];
+    const StageRanges R = L.plan[i / kTile];
+    const float4 p = xs[i];
+    const u32 cf = L.cnt[i] & 0xFFFFu;
+    const QuadHead H(L, R, i, g);
+    if (i - G.off >= G.n) return;
+    float sx = 0.0f, sy = 0.0f, sz = 0.0f;
+    if (cf <= L.kf) {
+        float4 q[kQuadHead];
+        float rj[kQuadHead];
+        for_quads(
+            L, R, H, i, g, cf,
+            [&](int u, u32 j) {
+                q[u] = xs[j];
+                rj[u] = rho[j];
+            },
+            [&](int u, float c0, bool valid) {
+                const float c = R.total ? pair_c(p, q[u], P.sp) : c0;
+                const float3 t = tension_normal_term(p, q[u], c, rj[u], P.mass);
+                quad_add(sx, valid ? t.x : -0.0f);  // adding -0.0f: no change
+                quad_add(sy, valid ? t.y : -0.0f);
+                quad_add(sz, valid ? t.z : -0.0f);
+            });
+    } else {
+        tension_normal_walk(P, G, i, p, xs, rho, sx, sy, sz);
+    }
+    if (g == 0) nrm[i] = make_float4(T.L * sx, T.L * sy, T.L * sz, 0.0f);
+}
+
+__global__ __launch_bounds__(NS) void k_tension_force(Nbr P, PairList L,
+                                                        const float4* __restrict__ xs,
+                                                        const float* __restrict__ rho,
+                                                        const float4* __restrict__ nrm,
+                                                        TensionArgs T, float4* __restrict__ vs) {
+    const QuadLane Q(P);
+    const u32 i = Q.i, g = Q.g;
+    const SceneSeg& G = P.seg[scene_of_slot(P, i)];
+    const StageRanges R = L.plan[i / kTile];
+    const float4 p = xs[i];
+    const float4 ni = nrm[i];
+    const float rho_i = rho[i];
+    const u32 cf = L.cnt[i] & 0xFFFFu;
+    const QuadHead H(L, R, i, g);
+    if (i - G.off >= G.n) return;
+    float ax = 0.0f, ay = 0.0f, az = 0.0f;
+    if (cf <= L.kf) {
+        float4 q[kQuadHead], nj[kQuadHead];
+        float rj[kQuadHead];
+        for_quads(
+            L, R, H, i, g, cf,
+            [&](int u, u32 j) {
+                q[u] = xs[j];
+                nj[u] = nrm[j];
+                rj[u] = rho[j];
+            },
+            [&](int u, float, bool valid) {
+                const float3 t = tension_force_term(p, ni, rho_i, q[u], nj[u], rj[u], P.mass, T);
+                quad_add(ax, valid ? t.x : -0.0f);
+                quad_add(ay, valid ? t.y : -0.0f);
+                quad_add(az, valid ? t.z : -0.0f);
+            });
+    } else {
+        tension_force_walk(P, G, i, p, ni, rho_i, xs, rho, nrm, T, ax, ay, az);
+    }
+    if (g == 0) {
+        const float4 v = vs[i];
+        vs[i] = make_float4(v.x + G.dt * ax, v.y + G.dt * ay, v.z + G.dt * az, 0.0f);
+    }
+}
+
 // k_change_st's sums, four lanes per particle.  Writes one error partial per
 // 64 slots, the wave sum that the one-lane kernels add up per tile
 // (finish_error's `quarters`).
@@ -2653,6 +2700,15 @@ void launch_density_alpha(u32 nt, hipStream_t s, u32 nslots, const Nbr& P, const
                           DeviceState* open = nullptr) {
     if (fast) density_alpha_mode<true>(nt, s, nslots, P, L, xs, rho, alpha, open);
     else density_alpha_mode<false>(nt, s, nslots, P, L, xs, rho, alpha, open);
+}
+
+void launch_tension(hipStream_t s, u32 nslots, const Nbr& P, const PairList& L, const float4* xs,
+                    const float* rho, const TensionArgs& T, float4* nrm, float4* vs) {
+    const u32 b = nslots / kQuadGroup;
+    k_tension_normals<<<b, NS, 0, s>>>(P, L, xs, rho, T, nrm);
+    WSIM_LAUNCH_CHECK();
+    k_tension_force<<<b, NS, 0, s>>>(P, L, xs, rho, nrm, T, vs);
+    WSIM_LAUNCH_CHECK();
 }
 
 template <bool F>
@@ -3497,13 +3553,8 @@ void DFSPHSolver::phase_prefix_solve(bool gravity) {
         const TensionArgs T{Lsup, 32.0f / (3.14159265358979323846f * std::pow(Lsup, 9.0f)),
                             std::pow(Lsup, 6.0f) / 64.0f, cfg_.surface_tension, cfg_.rest_density};
         tbegin(kKTension);
-        k_tension_normals<NS><<<nslots_ / NS, NS, 0, stream_>>>(P, pair_list(), xs_.data(),
-                                                                rho_.data(), T, nrm_.data());
-        WSIM_LAUNCH_CHECK();
-        k_tension_force<NS><<<nslots_ / NS, NS, 0, stream_>>>(P, pair_list(), xs_.data(),
-                                                              rho_.data(), nrm_.data(), T,
-                                                              vs_.data());
-        WSIM_LAUNCH_CHECK();
+        launch_tension(stream_, nslots_, P, pair_list(), xs_.data(), rho_.data(), T, nrm_.data(),
+                       vs_.data());
         tend();
     }
     if (!grid_sorted_) {
