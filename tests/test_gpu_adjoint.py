@@ -89,6 +89,26 @@ def test_adjoint_substep_matches_dual(case):
         assert abs(got - want) <= 1e-6 * abs(want), (case, k, got, want)
 
 
+@pytest.mark.parametrize("n,squeeze", [
+    (1, 1.0), (63, 1.0), (65, 0.9),  # a workgroup holds 64 particles
+    (257, 0.8),                      # a tile and a particle
+    (343, 0.6),                      # lists past their depth: the stencil walk
+])
+def test_adjoint_of_a_cluster_ignores_a_distant_one(n, squeeze):
+    # a second cluster beyond the support moves the first one's working slots
+    # (other lanes, workgroups and tiles) and leaves its lists alone: the same bits
+    x, v, xb, cfg = random_box(n=343, seed=n, max_density_iters=4, eta_density=0.0)
+    a = (0.78 - squeeze * (x[:n] - 0.2)).astype(np.float32)  # beside three walls
+    rng = np.random.default_rng(n)
+    gx, gv = rng.normal(size=(n + 343, 3)), rng.normal(size=(n + 343, 3))
+    one, _ = make_solver(a, v[:n], xb, cfg)
+    two, _ = make_solver(np.concatenate([a, x]), np.concatenate([v[:n], v]), xb, cfg)
+    wx, wv, _ = A.adjoint_step(one, 2e-4, gx[:n], gv[:n])
+    bx, bv, _ = A.adjoint_step(two, 2e-4, gx, gv)
+    assert np.abs(wx).max() > 0.0
+    assert np.array_equal(bx[:n], wx) and np.array_equal(bv[:n], wv)
+
+
 def test_adjoint_clamps_match_dual():
     # fast particles (|v| clamp at 5 m/s) next to the walls (domain clamp)
     x, v, xb, cfg = random_box(n=343, seed=4, max_density_iters=4)

@@ -39,7 +39,8 @@ namespace {
 using namespace dev;
 
 constexpr int NA = 256;  // workgroup size of the adjoint kernels (one tile)
-constexpr int kAdjointLanes = 4;  // lanes per particle in the per-iteration kernels
+constexpr int kAdjointLanes = 4;  // lanes per particle
+static_assert(kAdjointLanes == kQuad, "k_adj_alpha shares the launch grid");
 
 struct D3 {
     double x, y, z;
@@ -464,38 +465,73 @@ __global__ __launch_bounds__(NA) void k_adj_xsph(Nbr P, PairList L, const float4
 
 // alpha = rho / (|G|^2 + Q) (dfsph_kernels.cu:117-169): recomputes G and the
 // denominator exactly as the forward pass and turns alpha_bar into
-// G_bar = 2 D_bar G, Q_bar = D_bar (and rho_bar += alpha_bar / D).
+// G_bar = 2 D_bar G, Q_bar = D_bar (and rho_bar += alpha_bar / D).  Four
+// lanes per particle, whose binary32 terms are added in list order: one
+// lane's chain of gathers and roots bounds this pass (32,768 particles: one
+// lane 22.2 us, four 8.5).  The binary64 kernels around it are bound by their
+// quotients and roots: 8 lanes, or more gathers in flight per lane, give
+// nothing (13.2 -> 12.8 / 13.0 us for the transposed pressure update).
 __global__ __launch_bounds__(NA) void k_adj_alpha(Nbr P, PairList L, const float4* __restrict__ xs,
                                                   const float* __restrict__ rho,
                                                   const double* __restrict__ alphabar,
                                                   double* __restrict__ rhobar,
                                                   double4* __restrict__ gbar) {
-    const u32 i = slot_index<NA>(P.remap);
+    const u32 t = slot_index<NA>(P.remap);
+    const u32 i = t / kQuad, g = t % kQuad;
     if (i >= P.nslots) return;
     const SceneSeg& G = P.seg[scene_of_slot(P, i)];
-    if (i - G.off >= G.n) return;
+    if (i - G.off >= G.n) return;  // uniform in a quad, as every branch below
     const float4 p = xs[i];
     float sx = 0.0f, sy = 0.0f, sz = 0.0f, sq = 0.0f;
-    for_pairs(
-        P, L, G, i, p, xs,
-        [&](u32 j, float c) {
-            const float4 q = xs[j];
+    const u32 cw = L.cnt[i];
+    const u32 cf = cw & 0xFFFFu, cb = cw >> 16;
+    if (cf <= L.kf && cb <= L.kb) {
+        const auto add = [&](const float4& q, float c, float m, bool valid) {
             const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
-            const float mx = P.mass * (rx * c), my = P.mass * (ry * c), mz = P.mass * (rz * c);
+            const float mx = m * (rx * c), my = m * (ry * c), mz = m * (rz * c);
+            quad_add(sx, valid ? mx : -0.0f);  // adding -0.0f: no change
+            quad_add(sy, valid ? my : -0.0f);
+            quad_add(sz, valid ? mz : -0.0f);
+            quad_add(sq, valid ? mx * mx + my * my + mz * mz : -0.0f);
+        };
+        const StageRanges R = L.plan[i / kTile];
+        constexpr int U = 2;  // quads in flight
+        for (u32 k = 0; k < cf; k += U * kQuad) {
+            u32 j[U];
+            float c[U];
+            float4 q[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                j[u] = i;
+                c[u] = 0.0f;
+                const u32 e = k + kQuad * u + g;
+                if (e < cf) fluid_entry(L, R, e, i, j[u], c[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) q[u] = xs[j[u]];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                add(q[u], R.total ? pair_c(p, q[u], P.sp) : c[u], P.mass, k + kQuad * u + g < cf);
+        }
+        for (u32 k = 0; k < cb; k += kQuad) {
+            uint2 e = make_uint2(0u, 0u);
+            if (k + g < cb) e = ld_pair(L.b + pair_at(k + g, i, L.kb));
+            const float4 q = P.xb[e.x];
+            add(q, __uint_as_float(e.y), q.w, k + g < cb);
+        }
+    } else {
+        const auto add = [&](const float4& q, float c, float m) {
+            const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
+            const float mx = m * (rx * c), my = m * (ry * c), mz = m * (rz * c);
             sx += mx;
             sy += my;
             sz += mz;
             sq += mx * mx + my * my + mz * mz;
-        },
-        [&](u32 b, float c) {
-            const float4 q = P.xb[b];
-            const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
-            const float mx = q.w * (rx * c), my = q.w * (ry * c), mz = q.w * (rz * c);
-            sx += mx;
-            sy += my;
-            sz += mz;
-            sq += mx * mx + my * my + mz * mz;
-        });
+        };
+        for_pairs(P, L, G, i, p, xs, [&](u32 j, float c) { add(xs[j], c, P.mass); },
+                  [&](u32 b, float c) { add(P.xb[b], c, P.xb[b].w); });
+    }
+    if (g != 0) return;
     const float denom = sx * sx + sy * sy + sz * sz + sq;
     const double ab = alphabar[i];
     if (denom > 1e-9f && ab != 0.0) {
@@ -645,8 +681,8 @@ double DFSPHSolver::adjoint_step(const SubstepTape& t, const double* gx_out, con
                                                  adj_.rhobar.data(), adj_.xbar.data(),
                                                  adj_.part.data());
     WSIM_LAUNCH_CHECK();
-    k_adj_alpha<<<blocks, NA, 0, stream_>>>(P, L, xs_.data(), rho_.data(), adj_.alphabar.data(),
-                                             adj_.rhobar.data(), adj_.gbar.data());
+    k_adj_alpha<<<gblocks, NA, 0, stream_>>>(P, L, xs_.data(), rho_.data(), adj_.alphabar.data(),
+                                              adj_.rhobar.data(), adj_.gbar.data());
     WSIM_LAUNCH_CHECK();
     k_adj_geom<GL><<<gblocks, NA, 0, stream_>>>(P, L, fluid_grid_.sorted_indices(), xs_.data(),
                                                  adj_.rhobar.data(), adj_.gbar.data(),

@@ -1944,25 +1944,8 @@ __global__ void k_frame_begin(FrameParams fp, FrameParams* __restrict__ dst,
 // sum rounds exactly as the one-lane kernels' sums do.  Neighbours come
 // straight from L2 (the whole scene fits there), without a staging round or a
 // barrier.  Every branch around a broadcast is uniform in a quad.
-constexpr int kQuad = 4;
 constexpr u32 kQuadGroup = NS / kQuad;  // slots of a 256-thread workgroup
 
-template <int K>
-__device__ __forceinline__ float quad_get(float v) {
-    return __int_as_float(
-        __builtin_amdgcn_mov_dpp(__float_as_int(v), K * 0x55, 0xF, 0xF, true));
-}
-template <int K>
-__device__ __forceinline__ u32 quad_get(u32 v) {
-    return static_cast<u32>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), K * 0x55, 0xF, 0xF, true));
-}
-// acc + t of lane 0, then of lane 1, 2, 3
-__device__ __forceinline__ void quad_add(float& acc, float t) {
-    acc += quad_get<0>(t);
-    acc += quad_get<1>(t);
-    acc += quad_get<2>(t);
-    acc += quad_get<3>(t);
-}
 __device__ __forceinline__ void quad_sub(float& acc, float t) {
     acc -= quad_get<0>(t);
     acc -= quad_get<1>(t);

@@ -396,5 +396,25 @@ inline Nbr make_nbr(const CellGrid& fg, const CellGrid* bg, const float4* xb, co
     return P;
 }
 
+// Four lanes that share a particle.
+constexpr int kQuad = 4;
+// Value of lane K of this lane's quad (a DPP quad permutation).
+template <int K>
+__device__ __forceinline__ float quad_get(float v) {
+    return __int_as_float(
+        __builtin_amdgcn_mov_dpp(__float_as_int(v), K * 0x55, 0xF, 0xF, true));
+}
+template <int K>
+__device__ __forceinline__ u32 quad_get(u32 v) {
+    return static_cast<u32>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), K * 0x55, 0xF, 0xF, true));
+}
+// acc + t of lane 0, then of lane 1, 2, 3
+__device__ __forceinline__ void quad_add(float& acc, float t) {
+    acc += quad_get<0>(t);
+    acc += quad_get<1>(t);
+    acc += quad_get<2>(t);
+    acc += quad_get<3>(t);
+}
+
 }  // namespace dev
 }  // namespace wsim
