@@ -338,8 +338,17 @@ __global__ __launch_bounds__(NT) void k_density_alpha(Nbr P, PairList L,
         }
     };
     auto from_lds = [&](u32 s, int xk) { fluid_pair(s, xk, s_x[O.entry(s, xk)]); };
+    auto from_both = [&](u32 s, int xk) {
+        const u32 e = O.entry(s, xk);
+        float4 q = s_x[min(e, kStage ? kStageCap - 1u : 0u)];
+        if (e >= kStageCap) q = xs[s];
+        fluid_pair(s, xk, q);
+    };
     auto from_global = [&](u32 s, int xk) { fluid_pair(s, xk, xs[s]); };
-    if (lds) {
+    if (lds && __builtin_amdgcn_readfirstlane(R.total) > kStageCap) {
+        if (F) for_stencil_zrows(P.gf, cs, shift, p.x, p.y, p.z, from_both);
+        else for_stencil_rows(P.gf, cs, shift, p.x, p.y, p.z, from_both);
+    } else if (lds) {
         if (F) for_stencil_zrows(P.gf, cs, shift, p.x, p.y, p.z, from_lds);
         else for_stencil_rows(P.gf, cs, shift, p.x, p.y, p.z, from_lds);
     } else {
@@ -570,20 +579,40 @@ __global__ __launch_bounds__(kTile) void k_xsph_st(Nbr P, PairList L, const floa
     if (cf <= L.kf) {
         u32 k = 0;
         if (R.total) {
-            for_stage_quads(L, i, cf, [&](u32 a0, u32 a1, u32 a2, u32 a3, u32 m) {
-                const float r0 = rho[stage_source(R, a0)], r1 = rho[stage_source(R, a1)];
-                const float r2 = rho[stage_source(R, a2)], r3 = rho[stage_source(R, a3)];
-                const float4 q0 = s_a[a0], q1 = s_a[a1], q2 = s_a[a2], q3 = s_a[a3];
-                const float2 b0 = s_b[a0], b1 = s_b[a1], b2 = s_b[a2], b3 = s_b[a3];
-                const float4 w0 = make_float4(q0.w, b0.x, b0.y, 0.0f);
-                const float4 w1 = make_float4(q1.w, b1.x, b1.y, 0.0f);
-                const float4 w2 = make_float4(q2.w, b2.x, b2.y, 0.0f);
-                const float4 w3 = make_float4(q3.w, b3.x, b3.y, 0.0f);
-                xsph_listed<F>(dx, dy, dz, tx, ty, tz, p, vi, rho_i, q0, w0, r0, eps, P);
-                xsph_listed<F>(dx, dy, dz, tx, ty, tz, p, vi, rho_i, q1, w1, r1, eps, P, m > 1u);
-                xsph_listed<F>(dx, dy, dz, tx, ty, tz, p, vi, rho_i, q2, w2, r2, eps, P, m > 2u);
-                xsph_listed<F>(dx, dy, dz, tx, ty, tz, p, vi, rho_i, q3, w3, r3, eps, P, m > 3u);
-            });
+            const auto sums = [&](auto past) {
+                for_stage_quads(L, i, cf, [&](u32 a0, u32 a1, u32 a2, u32 a3, u32 m) {
+                    const u32 a[4] = {a0, a1, a2, a3};
+                    u32 j[4];
+                    float r[4];
+                    float4 q[4], w[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        j[u] = stage_source(R, a[u]);
+                        r[u] = rho[j[u]];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const u32 e = past ? min(a[u], kStageCap - 1u) : a[u];
+                        const float2 y = s_b[e];
+                        q[u] = s_a[e];
+                        w[u] = make_float4(q[u].w, y.x, y.y, 0.0f);
+                    }
+                    if (past && stage_past(a0, a1, a2, a3)) {
+#pragma unroll
+                        for (int u = 0; u < 4; ++u)
+                            if (a[u] >= kStageCap) {
+                                q[u] = xs[j[u]];
+                                w[u] = vin[j[u]];
+                            }
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        xsph_listed<F>(dx, dy, dz, tx, ty, tz, p, vi, rho_i, q[u], w[u], r[u], eps,
+                                       P, u == 0 || m > static_cast<u32>(u));
+                });
+            };
+            if (R.total > kStageCap) sums(std::true_type{});
+            else sums(std::false_type{});
         } else {
             // four pairs per trip: their gathers are issued together, the
             // terms added in list order
@@ -927,23 +956,33 @@ __global__ __launch_bounds__(kTile) void k_change_st(Nbr P, PairList L,
                 auto term = [&](const float4& q, const float4& w, bool keep) {
                     rho_dot_fluid<F>(racc, p, vi, q, w, pair_c_listed<F>(p, q, P.sp), mf, keep);
                 };
-                auto at = [&](u32 a, float4& q, float4& w) {
-                    const float4 x = s_a[a];
-                    const float2 y = s_b[a];
-                    q = make_float4(x.x, x.y, x.z, 0.0f);
-                    w = make_float4(x.w, y.x, y.y, 0.0f);
+                const auto sums = [&](auto past) {
+                    for_stage_quads(L, i, cf, [&](u32 a0, u32 a1, u32 a2, u32 a3, u32 m) {
+                        const u32 a[4] = {a0, a1, a2, a3};
+                        float4 q[4], w[4];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const u32 e = past ? min(a[u], kStageCap - 1u) : a[u];
+                            const float4 x = s_a[e];
+                            const float2 y = s_b[e];
+                            q[u] = make_float4(x.x, x.y, x.z, 0.0f);
+                            w[u] = make_float4(x.w, y.x, y.y, 0.0f);
+                        }
+                        if (past && stage_past(a0, a1, a2, a3)) {
+#pragma unroll
+                            for (int u = 0; u < 4; ++u)
+                                if (a[u] >= kStageCap) {
+                                    const u32 j = stage_source(R, a[u]);
+                                    q[u] = xs[j];
+                                    w[u] = vs[j];
+                                }
+                        }
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) term(q[u], w[u], u == 0 || m > static_cast<u32>(u));
+                    });
                 };
-                for_stage_quads(L, i, cf, [&](u32 a0, u32 a1, u32 a2, u32 a3, u32 m) {
-                    float4 q0, q1, q2, q3, w0, w1, w2, w3;
-                    at(a0, q0, w0);
-                    at(a1, q1, w1);
-                    at(a2, q2, w2);
-                    at(a3, q3, w3);
-                    term(q0, w0, true);
-                    term(q1, w1, m > 1u);
-                    term(q2, w2, m > 2u);
-                    term(q3, w3, m > 3u);
-                });
+                if (R.total > kStageCap) sums(std::true_type{});
+                else sums(std::false_type{});
             } else {
                 for (; k + PU <= cf; k += PU) {
                     uint2 e[PU];
@@ -1258,13 +1297,23 @@ __global__ __launch_bounds__(kTile) void k_apply_st(Nbr P, PairList L,
             auto term = [&](const float4& q, bool keep) {
                 kappa_term<F>(fx, fy, fz, p, q, pair_c_listed<F>(p, q, P.sp), mk(q.w), fdt, keep);
             };
-            for_stage_quads(L, i, cf, [&](u32 a0, u32 a1, u32 a2, u32 a3, u32 m) {
-                const float4 q0 = s_x[a0], q1 = s_x[a1], q2 = s_x[a2], q3 = s_x[a3];
-                term(q0, true);
-                term(q1, m > 1u);
-                term(q2, m > 2u);
-                term(q3, m > 3u);
-            });
+            const auto sums = [&](auto past) {
+                for_stage_quads(L, i, cf, [&](u32 a0, u32 a1, u32 a2, u32 a3, u32 m) {
+                    const u32 a[4] = {a0, a1, a2, a3};
+                    float4 q[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) q[u] = s_x[past ? min(a[u], kStageCap - 1u) : a[u]];
+                    if (past && stage_past(a0, a1, a2, a3)) {
+#pragma unroll
+                        for (int u = 0; u < 4; ++u)
+                            if (a[u] >= kStageCap) q[u] = xk[stage_source(R, a[u])];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) term(q[u], u == 0 || m > static_cast<u32>(u));
+                });
+            };
+            if (R.total > kStageCap) sums(std::true_type{});
+            else sums(std::false_type{});
         } else {
             for (; k + PU <= cf; k += PU) {
                 uint2 e[PU];

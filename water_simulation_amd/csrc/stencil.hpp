@@ -196,11 +196,26 @@ __device__ __forceinline__ bool finite3(float a, float b, float c) {
 // Keys grow fastest along z, so the stencil cells of a tile of consecutive
 // cell-sorted particles, whose keys span [kmin, kmax], lie for each x offset
 // dx in the key range [kmin + dx Dy Dz - Dz - 1, kmax + dx Dy Dz + Dz + 1]:
-// three contiguous slot ranges hold every fluid neighbour of the tile.  A
-// tile stages them in LDS when they are disjoint and fit; otherwise (sparse
-// tiles, particles outside the grid) it gathers from global memory.
+// three contiguous slot ranges hold every fluid neighbour of the tile, at
+// rest about 3 (256 + 2 W) particles for fluid W particles wide along z.  A
+// tile with disjoint ranges of up to kStageMax entries has a plan: it stages
+// the first kStageCap in LDS and reads the others from global memory (L2);
+// other tiles (particles outside the grid, very wide fluid) gather everything
+// and keep 8-byte list entries.
+//
+// The staged part sets how many workgroups share a CU: with 2,048 entries a
+// 100-wide exact block, whose tiles fit in 1,536, went from 187 to 223 us
+// (density) and 64 to 76 (change).  Planning past the staged part costs such
+// tiles nothing (the branch is tile-uniform).  One million particles, no
+// plan -> plan up to 4,096, us per launch:
+//   tolerance mode  W 187 (1,896 entries)  density 158 -> 103  XSPH 103 -> 62   change 88 -> 66   apply 52 -> 38
+//                   W 385 (3,078)          density 154 -> 104  XSPH 112 -> 80   change 91 -> 84   apply 56 -> 43
+//   exact           W 187                  density 233 -> 195  XSPH 133 -> 82   change 119 -> 90  apply 70 -> 56
+//                   W 385                  density 245 -> 193  XSPH 138 -> 101  change 127 -> 103 apply 76 -> 59
 constexpr u32 kStageCap = 1536;  // staged fluid particles per 256-slot tile
 static_assert(kStageCap % kTile == 0, "whole staging rounds per thread");
+constexpr u32 kStageMax = 4096;  // neighbourhood of a tile with a plan
+static_assert(kStageMax >= kStageCap && kStageMax <= 65536, "2-byte list entries");
 
 // (StageRanges is declared in wsim_internal.hpp; an empty range sits where
 // the previous one ends.)
@@ -245,7 +260,7 @@ __device__ inline StageRanges stage_ranges(const Nbr& P, const SceneSeg& G, u32 
     R.b1 = e0 - R.s0;
     R.b2 = R.b1 + (e1 - R.s1);
     const u32 total = R.b2 + (e2 - R.s2);
-    R.total = total <= kStageCap ? total : 0u;
+    R.total = total <= kStageMax ? total : 0u;
     return R;
 }
 
@@ -267,6 +282,11 @@ struct StageOffsets {
 // Working slot of staged entry e.
 __device__ __forceinline__ u32 stage_source(const StageRanges& R, u32 e) {
     return e >= R.b2 ? R.s2 + (e - R.b2) : (e >= R.b1 ? R.s1 + (e - R.b1) : R.s0 + e);
+}
+
+// Any of four entries past the staged ones.
+__device__ __forceinline__ bool stage_past(u32 a, u32 b, u32 c, u32 d) {
+    return max(max(a, b), max(c, d)) >= kStageCap;
 }
 
 // Fluid list entry k of particle i.  A tile whose neighbourhood is staged
