@@ -85,3 +85,26 @@ def test_four_lanes_equal_one_lane(n, clump, walls, over, fast):
         assert_bitexact(a[k], b[k], k)
     for k in ("density_iters", "divergence_iters", "mean_density_error", "max_velocity"):
         assert sa[k] == sb[k], (k, sa, sb)
+
+
+@pytest.mark.parametrize("fast", [False, True], ids=["exact", "fast"])
+def test_non_finite_particles_stay_their_own(fast):
+    """A particle at a non-finite position has no neighbours and keeps a finite
+    velocity; one with an infinite velocity gives its neighbours what the
+    one-lane kernels give them."""
+    x, v = cloud(3000, False)
+    x[5] = [np.nan, 0.3, 0.3]
+    x[700] = [np.inf, 0.2, np.nan]
+    x[701] = [0.2, -np.inf, 0.2]
+    v[1500] = [np.inf, 0.0, 0.0]  # a listed particle
+    xb = O.sample_aabb_boundary([0, 0, 0], [1, 1, 1], 2 * R, 3)
+    cfg = dict(rest_density=1000.0, particle_radius=R, smoothing_length=2 * R, viscosity=0.01,
+               damping=0.5, domain_min=(0, 0, 0), domain_max=(1, 1, 1), max_density_iters=1,
+               eta_density=1e-3, fast_math=fast)
+    a, sa = run(x, v, xb, cfg, None)
+    b, sb = run(x, v, xb, cfg, ONE_LANE)
+    assert np.isfinite(b["v"][[5, 700, 701]]).all()
+    for k in b:
+        assert np.array_equal(np.isnan(a[k]), np.isnan(b[k])), k
+        assert_bitexact(np.nan_to_num(a[k], nan=0.0), np.nan_to_num(b[k], nan=0.0), k)
+    assert sa["nan_count"] == sb["nan_count"]

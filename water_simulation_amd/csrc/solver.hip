@@ -2001,7 +2001,9 @@ __device__ __forceinline__ void quad_sub(float& acc, float t) {
     acc -= quad_get<2>(t);
     acc -= quad_get<3>(t);
 }
-// acc = fma(a, b, acc) with the a and b of lane 0, then of lane 1, 2, 3
+// acc = fma(a, b, acc) with the a and b of lane 0, then of lane 1, 2, 3.  A
+// lane without a term passes a = b = 0: b from its own particle's data would
+// be NaN where that is not finite, and 0 NaN is NaN.
 __device__ __forceinline__ void quad_fma(float& acc, float a, float b) {
     acc = __builtin_fmaf(quad_get<0>(a), quad_get<0>(b), acc);
     acc = __builtin_fmaf(quad_get<1>(a), quad_get<1>(b), acc);
@@ -2147,9 +2149,9 @@ __global__ __launch_bounds__(NS) void k_xsph_q(Nbr P, PairList L, const float4* 
                     const float k =
                         valid ? wv * __builtin_amdgcn_rcpf(fmaxf(rho_i + rj[u], 2.0f * 1e-9f))
                               : 0.0f;
-                    quad_fma(tx, k, w[u].x - vi.x);
-                    quad_fma(ty, k, w[u].y - vi.y);
-                    quad_fma(tz, k, w[u].z - vi.z);
+                    quad_fma(tx, k, valid ? w[u].x - vi.x : 0.0f);
+                    quad_fma(ty, k, valid ? w[u].y - vi.y : 0.0f);
+                    quad_fma(tz, k, valid ? w[u].z - vi.z : 0.0f);
                 } else {
                     float ax = -0.0f, ay = -0.0f, az = -0.0f;  // adding -0.0f: no change
                     xsph_term<false>(ax, ay, az, p, vi, rho_i, q[u], w[u], rj[u], eps, P, valid);
@@ -2303,7 +2305,7 @@ __global__ __launch_bounds__(NS) void k_change_q(Nbr P, PairList L, const float4
                         const float dot = __builtin_fmaf(
                             ux, p.x - q[u].x,
                             __builtin_fmaf(uy, p.y - q[u].y, uz * (p.z - q[u].z)));
-                        quad_fma(rf, valid ? c : 0.0f, dot);
+                        quad_fma(rf, valid ? c : 0.0f, valid ? dot : 0.0f);
                     } else {
                         const float gx = (p.x - q[u].x) * c, gy = (p.y - q[u].y) * c,
                                     gz = (p.z - q[u].z) * c;
@@ -2404,9 +2406,9 @@ __global__ __launch_bounds__(NS) void k_apply_q(Nbr P, PairList L, const float4*
         const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
         if (F) {
             const float k = valid ? -(h * c2 * c) : 0.0f;
-            quad_fma(sx, k, rx);
-            quad_fma(sy, k, ry);
-            quad_fma(sz, k, rz);
+            quad_fma(sx, k, valid ? rx : 0.0f);
+            quad_fma(sy, k, valid ? ry : 0.0f);
+            quad_fma(sz, k, valid ? rz : 0.0f);
         } else {
             const float gx = rx * c, gy = ry * c, gz = rz * c;
             quad_sub(sx, valid ? h * c2 * gx : 0.0f);  // subtracting +0.0f: no change
