@@ -108,3 +108,61 @@ def test_non_finite_particles_stay_their_own(fast):
         assert np.array_equal(np.isnan(a[k]), np.isnan(b[k])), k
         assert_bitexact(np.nan_to_num(a[k], nan=0.0), np.nan_to_num(b[k], nan=0.0), k)
     assert sa["nan_count"] == sb["nan_count"]
+
+
+def pile(n):
+    """n particles in one cell: stencils of n candidates, over every list."""
+    return (0.5 + np.random.default_rng(n).uniform(0.1 * R, 1.9 * R, (n, 3))).astype(np.float32)
+
+
+def kernel_us(x, xb, cfg, shapes, steps=5):
+    """Median time of each kernel kind's launches over `steps` equal steps, us."""
+    v = np.random.default_rng(0).normal(0.0, 0.3, x.shape).astype(np.float32)
+    f = ws.ParticleStore(len(x))
+    f.resize(len(x))
+    b = None
+    if xb is not None:
+        b = ws.ParticleStore(len(xb))
+        b.resize(len(xb))
+        b.set_positions(xb)
+    s = ws.DFSPHSolver(f, b, ws.DFSPHConfig(**cfg))
+    if shapes:
+        s.set_shapes(**shapes)
+    s.set_timing(True)
+    rec = []
+    for _ in range(steps + 1):
+        f.set_positions(x)
+        f.set_velocities(v)
+        s.reset_timing()
+        s.step(1e-5)
+        rec.append({k: 1e3 * ms / n for k, (n, ms) in s.kernel_times().items() if n})
+    s.close()
+    return {k: float(np.median([r[k] for r in rec[1:]])) for k in rec[0]}
+
+
+DENSE_CFG = dict(rest_density=1000.0, particle_radius=R, smoothing_length=2 * R, viscosity=0.01,
+                 damping=0.5, domain_min=(0, 0, 0), domain_max=(1, 1, 1), max_density_iters=2,
+                 eta_density=1e-9, pressure_form=1)
+
+
+@pytest.mark.parametrize("fast", [False, True], ids=["exact", "fast"])
+@pytest.mark.parametrize("case", ["pile", "plate"])
+def test_density_time_is_linear_in_the_stencil(case, fast):
+    """The four-lane density walk of stencils of thousands of candidates, of
+    the fluid and of the boundary, takes no longer than the one-lane walk (it
+    needs a quarter to half of its time; a walk that passes over the whole stencil once
+    per window of candidates took 2 to 11 times as long)."""
+    xb = None
+    if case == "pile":
+        x = pile(3000)
+    else:
+        x, _ = cloud(4000, False)
+        m = 400
+        g = np.stack(np.meshgrid(np.arange(m), np.arange(m), indexing="ij"), -1).reshape(-1, 2)
+        xb = np.full((m * m, 3), 0.045, np.float32)
+        xb[:, [0, 2]] = 0.03 + (0.4 / m) * g
+    cfg = dict(DENSE_CFG, fast_math=fast)
+    quads = kernel_us(x, xb, cfg, None)["density_alpha"]
+    one = kernel_us(x, xb, cfg, ONE_LANE)["density_alpha"]
+    print(f"{case}: four lanes {quads:.0f} us, one lane {one:.0f} us")
+    assert quads < 1.3 * one

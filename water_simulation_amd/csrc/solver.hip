@@ -2536,13 +2536,19 @@ __device__ __forceinline__ void for_candidates(const QuadRows<F ? 1 : 3>& W, u32
     for (u32 w0 = 0; w0 < W.total; w0 += kCand) {
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
-            u32 pos = W.base[t] - w0;  // wraps below the window: the test fails
+            u32 first = W.base[t];  // place of the range's first candidate
             const u32 rk = (g + 4u * t) / 3u;
 #pragma unroll
-            for (int k = 0; k < (F ? 1 : 3); ++k)
-                for (u32 s = W.b[t][k]; s < W.e[t][k]; ++s, ++pos)
-                    if (pos < kCand)
-                        cand[pos] = (s + shift) | ((F ? rk : static_cast<u32>(k)) << kCandRow);
+            for (int k = 0; k < (F ? 1 : 3); ++k) {
+                // the part of the range inside the window, so that all windows
+                // together pass over every candidate once
+                const u32 n = W.e[t][k] - W.b[t][k];
+                const u32 skip = w0 > first ? min(w0 - first, n) : 0u;
+                u32 pos = first + skip - w0;
+                for (u32 s = W.b[t][k] + skip; s < W.e[t][k] && pos < kCand; ++s, ++pos)
+                    cand[pos] = (s + shift) | ((F ? rk : static_cast<u32>(k)) << kCandRow);
+                first += n;
+            }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         const u32 n = min(W.total - w0, kCand);
