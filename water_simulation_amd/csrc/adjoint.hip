@@ -485,15 +485,15 @@ __global__ __launch_bounds__(NA) void k_adj_alpha(Nbr P, PairList L, const float
     float sx = 0.0f, sy = 0.0f, sz = 0.0f, sq = 0.0f;
     const u32 cw = L.cnt[i];
     const u32 cf = cw & 0xFFFFu, cb = cw >> 16;
+    const auto add = [&](const float4& q, float c, float m, bool valid) {
+        const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
+        const float mx = m * (rx * c), my = m * (ry * c), mz = m * (rz * c);
+        quad_add(sx, valid ? mx : -0.0f);  // adding -0.0f: no change
+        quad_add(sy, valid ? my : -0.0f);
+        quad_add(sz, valid ? mz : -0.0f);
+        quad_add(sq, valid ? mx * mx + my * my + mz * mz : -0.0f);
+    };
     if (cf <= L.kf && cb <= L.kb) {
-        const auto add = [&](const float4& q, float c, float m, bool valid) {
-            const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
-            const float mx = m * (rx * c), my = m * (ry * c), mz = m * (rz * c);
-            quad_add(sx, valid ? mx : -0.0f);  // adding -0.0f: no change
-            quad_add(sy, valid ? my : -0.0f);
-            quad_add(sz, valid ? mz : -0.0f);
-            quad_add(sq, valid ? mx * mx + my * my + mz * mz : -0.0f);
-        };
         const StageRanges R = L.plan[i / kTile];
         constexpr int U = 2;  // quads in flight
         for (u32 k = 0; k < cf; k += U * kQuad) {
@@ -520,16 +520,24 @@ __global__ __launch_bounds__(NA) void k_adj_alpha(Nbr P, PairList L, const float
             add(q, __uint_as_float(e.y), q.w, k + g < cb);
         }
     } else {
-        const auto add = [&](const float4& q, float c, float m) {
-            const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
-            const float mx = m * (rx * c), my = m * (ry * c), mz = m * (rz * c);
-            sx += mx;
-            sy += my;
-            sz += mz;
-            sq += mx * mx + my * my + mz * mz;
-        };
-        for_pairs(P, L, G, i, p, xs, [&](u32 j, float c) { add(xs[j], c, P.mass); },
-                  [&](u32 b, float c) { add(P.xb[b], c, P.xb[b].w); });
+        // candidates of zero gradient add nothing (their sums never hold -0)
+        for_stencil_quads(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, g,
+                          [&](bool valid, u32 s) {
+                              const float4 q = xs[s];
+                              const float r2 = dist2(p.x - q.x, p.y - q.y, p.z - q.z);
+                              const bool in = valid && s != i && !(r2 >= P.sp.far2);
+                              const float c = spline_gradc(pair_sqrt(in ? r2 : 0.0f, P.sp), P.sp);
+                              add(q, c, P.mass, in && c != 0.0f);
+                          });
+        if (P.nb) {
+            for_stencil_quads(P.gb, P.csb, 0u, p.x, p.y, p.z, g, [&](bool valid, u32 s) {
+                const float4 q = P.xb[s];
+                const float r2 = dist2(p.x - q.x, p.y - q.y, p.z - q.z);
+                const bool in = valid && !(r2 >= P.sp.far2);
+                const float c = spline_gradc(pair_sqrt(in ? r2 : 0.0f, P.sp), P.sp);
+                add(q, c, q.w, in && c != 0.0f);
+            });
+        }
     }
     if (g != 0) return;
     const float denom = sx * sx + sy * sy + sz * sz + sq;

@@ -691,41 +691,6 @@ __device__ __forceinline__ float3 tension_force_term(const float4& p, const floa
                        K * (sc * ry + -T.gamma * (ni.y - nj.y)),
                        K * (sc * rz + -T.gamma * (ni.z - nj.z)));
 }
-// The sums over the stencil, for particles whose list is incomplete.
-__device__ __forceinline__ void tension_normal_walk(const Nbr& P, const SceneSeg& G, u32 i,
-                                                    const float4& p, const float4* xs,
-                                                    const float* rho, float& sx, float& sy,
-                                                    float& sz) {
-    for_stencil(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, [&](u32 s) {
-        if (s == i) return;
-        const float4 q = xs[s];
-        const float r2 = dist2(p.x - q.x, p.y - q.y, p.z - q.z);
-        if (r2 >= P.sp.far2) return;
-        const float c = spline_gradc(pair_sqrt(r2, P.sp), P.sp);
-        // zero-gradient pairs add +-0 to sums that never hold -0: left out
-        if (c == 0.0f) return;
-        const float3 t = tension_normal_term(p, q, c, rho[s], P.mass);
-        sx += t.x;
-        sy += t.y;
-        sz += t.z;
-    });
-}
-__device__ __forceinline__ void tension_force_walk(const Nbr& P, const SceneSeg& G, u32 i,
-                                                   const float4& p, const float4& ni, float rho_i,
-                                                   const float4* xs, const float* rho,
-                                                   const float4* nrm, const TensionArgs& T,
-                                                   float& ax, float& ay, float& az) {
-    for_stencil(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, [&](u32 s) {
-        if (s == i) return;
-        const float4 q = xs[s];
-        if (dist2(p.x - q.x, p.y - q.y, p.z - q.z) >= P.sp.far2) return;
-        const float3 t = tension_force_term(p, ni, rho_i, q, nrm[s], rho[s], P.mass, T);
-        ax += t.x;
-        ay += t.y;
-        az += t.z;
-    });
-}
-
 // rho_dot terms (dfsph_kernels.cu:210, 222) for one pair with gradient scalar c.
 // v . Gb (tolerance mode's boundary term of the density change)
 __device__ __forceinline__ float dot_gb(const float4& v, const float4& g) {
@@ -2162,13 +2127,26 @@ __global__ __launch_bounds__(NS) void k_xsph_q(Nbr P, PairList L, const float4* 
             });
         xsph_listed_scale<F>(dx, dy, dz, tx, ty, tz, eps, P);
     } else {
-        for_stencil(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, [&](u32 s) {
-            if (s == i) return;
-            const float4 q = xs[s];
-            const float r2 = PairMath<F>::r2(p.x - q.x, p.y - q.y, p.z - q.z);
-            if (r2 >= P.sp.far2) return;  // W = 0
-            xsph_term_r2<F>(dx, dy, dz, r2, vi, rho_i, vin[s], rho[s], eps, P);
-        });
+        for_stencil_quads(
+            P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, g, [&](bool valid, u32 s) {
+                const float4 q = xs[s], w = vin[s];
+                const float r2 = PairMath<F>::r2(p.x - q.x, p.y - q.y, p.z - q.z);
+                const bool in = valid && s != i && !(r2 >= P.sp.far2);  // else W = 0
+                if (F) {
+                    const float c = eps * PairMath<F>::div(P.mass, fmaxf(0.5f * (rho_i + rho[s]), 1e-9f)) *
+                                    PairMath<F>::w(r2, P.sp);
+                    const float k = in ? c : 0.0f;
+                    quad_fma(dx, k, in ? w.x - vi.x : 0.0f);
+                    quad_fma(dy, k, in ? w.y - vi.y : 0.0f);
+                    quad_fma(dz, k, in ? w.z - vi.z : 0.0f);
+                } else {
+                    float ax = -0.0f, ay = -0.0f, az = -0.0f;
+                    xsph_term_r2<false>(ax, ay, az, r2, vi, rho_i, w, rho[s], eps, P, in);
+                    quad_add(dx, ax);
+                    quad_add(dy, ay);
+                    quad_add(dz, az);
+                }
+            });
     }
     if (g == 0) vout[i] = make_float4(vi.x + dx, vi.y + dy, vi.z + dz, 0.0f);
 }
@@ -2209,7 +2187,19 @@ __global__ __launch_bounds__(NS) void k_tension_normals(Nbr P, PairList L,
                 quad_add(sz, valid ? t.z : -0.0f);
             });
     } else {
-        tension_normal_walk(P, G, i, p, xs, rho, sx, sy, sz);
+        for_stencil_quads(
+            P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, g, [&](bool valid, u32 s) {
+                const float4 q = xs[s];
+                const float r2 = dist2(p.x - q.x, p.y - q.y, p.z - q.z);
+                const bool in = valid && s != i && !(r2 >= P.sp.far2);
+                const float c = spline_gradc(pair_sqrt(in ? r2 : 0.0f, P.sp), P.sp);
+                // zero-gradient pairs add +-0 to sums that never hold -0: left out
+                const bool add = in && c != 0.0f;
+                const float3 t = tension_normal_term(p, q, c, rho[s], P.mass);
+                quad_add(sx, add ? t.x : -0.0f);
+                quad_add(sy, add ? t.y : -0.0f);
+                quad_add(sz, add ? t.z : -0.0f);
+            });
     }
     if (g == 0) nrm[i] = make_float4(T.L * sx, T.L * sy, T.L * sz, 0.0f);
 }
@@ -2247,7 +2237,16 @@ __global__ __launch_bounds__(NS) void k_tension_force(Nbr P, PairList L,
                 quad_add(az, valid ? t.z : -0.0f);
             });
     } else {
-        tension_force_walk(P, G, i, p, ni, rho_i, xs, rho, nrm, T, ax, ay, az);
+        for_stencil_quads(
+            P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, g, [&](bool valid, u32 s) {
+                const float4 q = xs[s];
+                const bool in = valid && s != i &&
+                                !(dist2(p.x - q.x, p.y - q.y, p.z - q.z) >= P.sp.far2);
+                const float3 t = tension_force_term(p, ni, rho_i, q, nrm[s], rho[s], P.mass, T);
+                quad_add(ax, in ? t.x : -0.0f);
+                quad_add(ay, in ? t.y : -0.0f);
+                quad_add(az, in ? t.z : -0.0f);
+            });
     }
     if (g == 0) {
         const float4 v = vs[i];
@@ -2289,6 +2288,28 @@ __global__ __launch_bounds__(NS) void k_change_q(Nbr P, PairList L, const float4
         // tolerance mode: the fluid terms sum c (u . r) in rf, times m once
         float rf = 0.0f;
         const u32 cf = cw & 0xFFFFu, cb = cw >> 16;
+        // the terms of rho_dot_fluid and rho_dot_boundary, in lane order
+        auto fluid = [&](const float4& q, const float4& w, float c, bool valid) {
+            const float ux = vi.x - w.x, uy = vi.y - w.y, uz = vi.z - w.z;
+            if (F) {
+                const float dot = __builtin_fmaf(ux, p.x - q.x,
+                                                 __builtin_fmaf(uy, p.y - q.y, uz * (p.z - q.z)));
+                quad_fma(rf, valid ? c : 0.0f, valid ? dot : 0.0f);
+            } else {
+                const float gx = (p.x - q.x) * c, gy = (p.y - q.y) * c, gz = (p.z - q.z) * c;
+                quad_add(rd, valid ? P.mass * (ux * gx + uy * gy + uz * gz) : -0.0f);
+            }
+        };
+        auto wall = [&](const float4& q, float c, bool valid) {
+            if (F) {
+                const float dot = __builtin_fmaf(
+                    vi.x, p.x - q.x, __builtin_fmaf(vi.y, p.y - q.y, vi.z * (p.z - q.z)));
+                quad_fma(rd, valid ? q.w * c : 0.0f, valid ? dot : 0.0f);
+            } else {
+                const float gx = (p.x - q.x) * c, gy = (p.y - q.y) * c, gz = (p.z - q.z) * c;
+                quad_add(rd, valid ? q.w * (vi.x * gx + vi.y * gy + vi.z * gz) : -0.0f);
+            }
+        };
         if (cf <= L.kf && cb <= L.kb) {
             float4 q[kQuadHead];
             float4 w[kQuadHead];
@@ -2299,45 +2320,24 @@ __global__ __launch_bounds__(NS) void k_change_q(Nbr P, PairList L, const float4
                     w[u] = vs[j];
                 },
                 [&](int u, float c0, bool valid) {
-                    const float c = R.total ? pair_c_listed<F>(p, q[u], P.sp) : c0;
-                    const float ux = vi.x - w[u].x, uy = vi.y - w[u].y, uz = vi.z - w[u].z;
-                    if (F) {
-                        const float dot = __builtin_fmaf(
-                            ux, p.x - q[u].x,
-                            __builtin_fmaf(uy, p.y - q[u].y, uz * (p.z - q[u].z)));
-                        quad_fma(rf, valid ? c : 0.0f, valid ? dot : 0.0f);
-                    } else {
-                        const float gx = (p.x - q[u].x) * c, gy = (p.y - q[u].y) * c,
-                                    gz = (p.z - q[u].z) * c;
-                        quad_add(rd, valid ? P.mass * (ux * gx + uy * gy + uz * gz) : -0.0f);
-                    }
+                    fluid(q[u], w[u], R.total ? pair_c_listed<F>(p, q[u], P.sp) : c0, valid);
                 });
-            for_quads_boundary(P, L, i, g, cb, [&](const float4& q, float c, bool valid) {
-                if (F) {
-                    const float dot = __builtin_fmaf(
-                        vi.x, p.x - q.x, __builtin_fmaf(vi.y, p.y - q.y, vi.z * (p.z - q.z)));
-                    quad_fma(rd, valid ? q.w * c : 0.0f, valid ? dot : 0.0f);
-                } else {
-                    const float gx = (p.x - q.x) * c, gy = (p.y - q.y) * c, gz = (p.z - q.z) * c;
-                    quad_add(rd, valid ? q.w * (vi.x * gx + vi.y * gy + vi.z * gz) : -0.0f);
-                }
-            });
+            for_quads_boundary(P, L, i, g, cb, wall);
         } else {
-            float& racc = F ? rf : rd;
-            const float mf = F ? 1.0f : P.mass;
-            for_stencil(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, [&](u32 s) {
-                if (s == i) return;
-                const float4 q = xs[s];
-                const float r2 = PairMath<F>::r2(p.x - q.x, p.y - q.y, p.z - q.z);
-                if (r2 >= P.sp.far2) return;
-                rho_dot_fluid<F>(racc, p, vi, q, vs[s], stencil_c<F>(r2, P.sp), mf);
-            });
+            for_stencil_quads(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, g,
+                              [&](bool valid, u32 s) {
+                                  const float4 q = xs[s];
+                                  const float r2 =
+                                      PairMath<F>::r2(p.x - q.x, p.y - q.y, p.z - q.z);
+                                  const bool in = valid && s != i && !(r2 >= P.sp.far2);
+                                  fluid(q, vs[s], stencil_c<F>(in ? r2 : 0.0f, P.sp), in);
+                              });
             if (P.nb && !(F && L.gb)) {
-                for_stencil(P.gb, P.csb, 0u, p.x, p.y, p.z, [&](u32 s) {
+                for_stencil_quads(P.gb, P.csb, 0u, p.x, p.y, p.z, g, [&](bool valid, u32 s) {
                     const float4 q = P.xb[s];
                     const float r2 = PairMath<F>::r2(p.x - q.x, p.y - q.y, p.z - q.z);
-                    if (r2 >= P.sp.far2) return;
-                    rho_dot_boundary<F>(rd, p, vi, q, stencil_c<F>(r2, P.sp));
+                    const bool in = valid && !(r2 >= P.sp.far2);
+                    wall(q, stencil_c<F>(in ? r2 : 0.0f, P.sp), in);
                 });
             }
         }
@@ -2433,19 +2433,19 @@ __global__ __launch_bounds__(NS) void k_apply_q(Nbr P, PairList L, const float4*
             add(dx, dy, dz, b, c, b.w * (ki + bf), dt, valid);
         });
     } else {
-        for_stencil(P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, [&](u32 s) {
-            if (s == i) return;
-            const float4 b = xk[s];
-            const float r2 = PairMath<F>::r2(p.x - b.x, p.y - b.y, p.z - b.z);
-            if (r2 >= P.sp.far2) return;
-            kappa_term<F>(fx, fy, fz, p, b, stencil_c<F>(r2, P.sp), mk(b.w), fdt);
-        });
+        for_stencil_quads(
+            P.gf, P.csf + G.key_base, G.off - G.start, p.x, p.y, p.z, g, [&](bool valid, u32 s) {
+                const float4 b = xk[s];
+                const float r2 = PairMath<F>::r2(p.x - b.x, p.y - b.y, p.z - b.z);
+                const bool in = valid && s != i && !(r2 >= P.sp.far2);
+                add(fx, fy, fz, b, stencil_c<F>(in ? r2 : 0.0f, P.sp), mk(b.w), fdt, in);
+            });
         if (P.nb && !(F && L.gb)) {
-            for_stencil(P.gb, P.csb, 0u, p.x, p.y, p.z, [&](u32 s) {
+            for_stencil_quads(P.gb, P.csb, 0u, p.x, p.y, p.z, g, [&](bool valid, u32 s) {
                 const float4 b = P.xb[s];
                 const float r2 = PairMath<F>::r2(p.x - b.x, p.y - b.y, p.z - b.z);
-                if (r2 >= P.sp.far2) return;
-                kappa_term<F>(dx, dy, dz, p, b, stencil_c<F>(r2, P.sp), b.w * (ki + bf), dt);
+                const bool in = valid && !(r2 >= P.sp.far2);
+                add(dx, dy, dz, b, stencil_c<F>(in ? r2 : 0.0f, P.sp), b.w * (ki + bf), dt, in);
             });
         }
     }

@@ -436,5 +436,48 @@ __device__ __forceinline__ void quad_add(float& acc, float t) {
     acc += quad_get<3>(t);
 }
 
+// for_stencil_rows by the lanes of a quad: use(valid, slot), lane g with
+// candidates g, g + 4, ... of each (dz, dy) row, so that adding the terms in
+// lane order is the walk's order.  Lanes past the row's end get a candidate of
+// the row and valid = false.  For particles whose lists are incomplete: with
+// every lane making the whole walk, four lanes were slower than one once they
+// filled the card (64,000 particles at 465 neighbours, XSPH: one lane 248 us,
+// four 323, sharing 127; a million at 79, both tension passes: 769, 2,316, 863).
+template <class F>
+__device__ __forceinline__ void for_stencil_quads(const GridGeom& g, const u32* __restrict__ cs,
+                                                  u32 shift, float px, float py, float pz,
+                                                  u32 lane, F&& use) {
+    const int cx = g.cx(px), cy = g.cy(py), cz = g.cz(pz);
+    for (int dz = -1; dz <= 1; ++dz) {
+        const int nz = cz + dz;
+        if (nz < 0 || nz >= g.dz) continue;
+        for (int dy = -1; dy <= 1; ++dy) {
+            const int ny = cy + dy;
+            if (ny < 0 || ny >= g.dy) continue;
+            u32 b[3], n[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const int nx = cx + k - 1;
+                const bool in = nx >= 0 && nx < g.dx;
+                const u32 c = in ? (static_cast<u32>(nx) * static_cast<u32>(g.dy) +
+                                    static_cast<u32>(ny)) *
+                                           static_cast<u32>(g.dz) +
+                                       static_cast<u32>(nz)
+                                 : 0u;
+                const u32 bk = cs[c], ek = cs[c + 1];  // c = 0 (in bounds) for skipped cells
+                b[k] = in ? bk : 0u;
+                n[k] = in ? ek - bk : 0u;
+            }
+            const u32 n01 = n[0] + n[1], total = n01 + n[2];
+            for (u32 k0 = 0; k0 < total; k0 += kQuad) {
+                const bool valid = k0 + lane < total;
+                const u32 k = valid ? k0 + lane : k0;
+                const u32 s = k < n[0] ? b[0] + k : k < n01 ? b[1] + (k - n[0]) : b[2] + (k - n01);
+                use(valid, s + shift);
+            }
+        }
+    }
+}
+
 }  // namespace dev
 }  // namespace wsim
