@@ -4048,8 +4048,7 @@ void DFSPHSolver::autotune(int reps) {
                   rho_adv_.data(), kappa_.data(), xk_.data(), cfg_.fast_math != 0};
     ApplyArgs aa{xk_.data(), kappa_.data(), cfg_.rest_density, static_cast<int>(cfg_.pressure_form),
                  0, 0, static_cast<double>(cfg_.eta_density * cfg_.rest_density), part_d_.data(),
-                 sweeps_by_quads(shapes_.change_nt, nslots_, cfg_.fast_math != 0) ? 1 : 0,
-                 dstate_.data(), vs_.data(), vs_.data(), cfg_.fast_math != 0};
+                 0, dstate_.data(), vs_.data(), vs_.data(), cfg_.fast_math != 0};
     try {
         // cell_start pass
         // cell_start entries: C + 1 for one scene, scenes * (C + 1) + 1 segmented
@@ -4096,6 +4095,9 @@ void DFSPHSolver::autotune(int reps) {
                     tune_log_.push_back({kKDensityChange, nt, pu, remap, 0, ms});
                     if (ms < b_ch) b_ch = ms, cand.change_nt = nt, cand.change_pu = pu;
                 }
+            // the error partials in the layout that the chosen k_change leaves
+            launch_change<0>(cand.change_nt, cand.change_pu, stream_, nslots_, P, L, ca);
+            aa.quarters = sweeps_by_quads(cand.change_nt, nslots_, cfg_.fast_math != 0) ? 1 : 0;
             for (u32 nt : {0u, 64u, 128u, 256u, 512u})
                 for (u32 pu : {2u, 4u, 8u}) {
                     const double ms =
