@@ -255,13 +255,16 @@ wsim_status wsim_solver_kernel_time(wsim_solver solver, int kind, uint64_t* laun
  * No counterpart in the reference (its kernels use fixed 128/256-thread
  * blocks, dfsph.cu:137-326).  Every shape computes the same bits. */
 typedef struct {
-    uint32_t density_alpha_nt;   /* workgroup size: 64, 128, 256 (small working sets: four
-                                    lanes per particle), 512 */
-    uint32_t xsph_nt;            /* 0 (staged in LDS; small working sets: four lanes per
-                                    particle), 64, 128, 256, 512 */
-    uint32_t change_nt;          /* 0 (as xsph_nt, 256 threads), 256, 512, 1024 */
+    /* Kernel of each pass: 4 takes four lanes per particle, 1 one lane per
+     * particle with the neighbourhood staged in LDS (256 threads), and the
+     * default, 256 for density_alpha_nt and 0 for the others, the better of
+     * the two for the size of the working set; larger values are workgroup
+     * sizes of the kernels that stage nothing. */
+    uint32_t density_alpha_nt;   /* 1, 4, 64, 128, 256, 512 */
+    uint32_t xsph_nt;            /* 0, 1, 4, 64, 128, 256, 512 */
+    uint32_t change_nt;          /* 0, 1, 4, 256, 512, 1024 */
     uint32_t change_pu;          /* pairs per trip of the list loops: 2, 4, 8 */
-    uint32_t apply_nt;           /* 0 (as xsph_nt), 64, 128, 256, 512 */
+    uint32_t apply_nt;           /* 0, 1, 4, 64, 128, 256, 512 */
     uint32_t apply_pu;           /* 2, 4, 8 */
     uint32_t cell_cpt;           /* cells per thread of the cell_start pass: 4, 8, 16 */
     uint32_t remap;              /* 1: XCD-aware workgroup order */

@@ -2695,31 +2695,43 @@ u32 grid_for(u32 nslots, u32 nt) { return div_up(nslots, nt); }
 // Working slots up to which the default shapes (0, and 256 threads for
 // density/alpha) take the four-lane kernels.  Where the chip is idle they
 // shorten a lane's serial chain; once every CU holds several workgroups the
-// staged kernels move fewer bytes per pair.  Measured per launch (stirred
-// block with walls, us, one lane -> four lanes):
-//   exact   density  4k 50.7 -> 15.6   65k 46.0 -> 26.2   130k 46.2 -> 39.6
-//           change   4k  8.3 ->  6.1   65k 11.6 -> 10.6    95k 12.6 -> 12.8
-//           apply    4k  7.5 ->  5.8   65k 11.0 ->  9.0    95k 11.6 -> 11.6
-//           XSPH     4k  9.8 ->  5.0   49k 10.5 ->  9.8    65k 10.5 -> 10.7
+// staged kernels move fewer bytes per pair.  Measured per launch, us, one lane
+// -> four lanes (stirred block with walls below 100k slots, jittered block
+// without walls above; b: a batch of 64 box scenes):
+//   exact   density  4k 50.7 -> 15.6   65k 46.0 -> 26.2   131k 51.8 -> 43.8   197k 57.4 -> 59.2
+//                    b 65k 66.1 -> 33.2  b 107k 66.4 -> 42.1  b 239k 69.6 -> 79.5
+//           change   4k  8.3 ->  6.1   65k 11.6 -> 10.6    95k 12.6 -> 12.8   b 65k 11.6 -> 11.3
+//           apply    4k  7.5 ->  5.8   65k 11.0 ->  9.0    95k 11.6 -> 11.6   b 65k 11.0 -> 10.4
+//           XSPH     4k  9.8 ->  5.0   65k 13.4 -> 12.5    98k 14.4 -> 15.5   b 65k 16.3 -> 13.0
 //   tolerance mode
-//           density  4k 28.4 -> 12.9   65k 26.3 -> 21.4    95k 27.5 -> 26.4
-//           change   4k  8.0 ->  5.4   33k  7.3 ->  6.2    49k  7.3 ->  7.3
-//           apply    4k  6.6 ->  4.5   33k  6.0 ->  5.3    49k  6.2 ->  6.8
-//           XSPH     4k  8.4 ->  4.6   65k  8.4 ->  8.0    95k 10.4 -> 10.5
+//           density  4k 28.4 -> 12.9   65k 26.3 -> 21.4    95k 27.5 -> 26.4   131k 24.9 -> 35.2
+//                    b 65k 36.4 -> 26.0  b 107k 37.8 -> 33.7
+//           change   4k  8.0 ->  5.4   33k  7.3 ->  6.2    49k  7.3 ->  7.3   b 30k 9.1 -> 8.2
+//           apply    4k  6.6 ->  4.5   33k  6.0 ->  5.3    49k  6.2 ->  6.8   b 30k 7.9 -> 7.5
+//           XSPH     4k  8.4 ->  4.6   65k  8.4 ->  8.0    95k 10.4 -> 10.5   b 65k 14.0 -> 11.3
+// The lines lie inside the range where four lanes win (exact density: it ends
+// between 131k and 197k).
 struct QuadLimits {
     u32 density, xsph, sweeps;
 };
 constexpr QuadLimits quad_limits(bool fast) {
     return fast ? QuadLimits{98304, 65536, 40960} : QuadLimits{131072, 65536, 65536};
 }
+// Shape values 1 and 4: one lane per particle (256 threads, staged in LDS) and
+// four lanes per particle, at any size.
+constexpr u32 kOneLane = 1, kFourLanes = 4;
+static_assert(kFourLanes == kQuad);
+bool by_quads(u32 nt, u32 by_size, u32 nslots, u32 limit) {
+    return nt == kFourLanes || (nt == by_size && nslots <= limit);
+}
 bool sweeps_by_quads(u32 nt, u32 nslots, bool fast) {
-    return nt == 0 && nslots <= quad_limits(fast).sweeps;
+    return by_quads(nt, 0, nslots, quad_limits(fast).sweeps);
 }
 
 template <bool F>
 void density_alpha_mode(u32 nt, hipStream_t s, u32 nslots, const Nbr& P, const PairList& L,
                         const float4* xs, float* rho, float* alpha, DeviceState* open) {
-    if (nt == 256 && nslots <= quad_limits(F).density) {
+    if (by_quads(nt, 256, nslots, quad_limits(F).density)) {
         k_density_alpha_q<F><<<nslots / kQuadGroup, NS, 0, s>>>(P, L, xs, rho, alpha, open);
         WSIM_LAUNCH_CHECK();
         return;
@@ -2727,6 +2739,7 @@ void density_alpha_mode(u32 nt, hipStream_t s, u32 nslots, const Nbr& P, const P
     switch (nt) {
     case 64: k_density_alpha<64, F><<<grid_for(nslots, 64), 64, 0, s>>>(P, L, xs, rho, alpha, nullptr, open); break;
     case 128: k_density_alpha<128, F><<<grid_for(nslots, 128), 128, 0, s>>>(P, L, xs, rho, alpha, nullptr, open); break;
+    case kOneLane:
     case 256: k_density_alpha<256, F><<<grid_for(nslots, 256), 256, 0, s>>>(P, L, xs, rho, alpha, nullptr, open); break;
     case 512: k_density_alpha<512, F><<<grid_for(nslots, 512), 512, 0, s>>>(P, L, xs, rho, alpha, nullptr, open); break;
     default: fail(kInvalidArgument, "density_alpha workgroup size");
@@ -2755,12 +2768,13 @@ template <bool F>
 void xsph_mode(u32 nt, hipStream_t s, u32 nslots, const Nbr& P, const PairList& L,
                const float4* xs, const float4* vin, const float* rho, float4* vout) {
     constexpr int XPU = 4;
-    if (nt == 0 && nslots <= quad_limits(F).xsph) {
+    if (by_quads(nt, 0, nslots, quad_limits(F).xsph)) {
         k_xsph_q<F><<<nslots / kQuadGroup, NS, 0, s>>>(P, L, xs, vin, rho, vout);
         WSIM_LAUNCH_CHECK();
         return;
     }
     switch (nt) {
+    case kOneLane:
     case 0: k_xsph_st<XPU, F><<<nslots / kTile, kTile, 0, s>>>(P, L, xs, vin, rho, vout); break;
     case 64: k_xsph<64, XPU, F><<<grid_for(nslots, 64), 64, 0, s>>>(P, L, xs, vin, rho, vout); break;
     case 128: k_xsph<128, XPU, F><<<grid_for(nslots, 128), 128, 0, s>>>(P, L, xs, vin, rho, vout); break;
@@ -2829,7 +2843,7 @@ void change_mode(u32 nt, u32 pu, hipStream_t s, u32 nslots, const Nbr& P, const 
         WSIM_LAUNCH_CHECK();
         return;
     }
-    if (nt == 0) {
+    if (nt == 0 || nt == kOneLane) {
         switch (pu) {
         case 2: change_staged<MODE, 2, F>(s, nslots, P, L, a); break;
         case 4: change_staged<MODE, 4, F>(s, nslots, P, L, a); break;
@@ -2895,7 +2909,6 @@ void apply_staged(hipStream_t s, u32 nslots, const Nbr& P, const PairList& L, co
                                                        a.quarters, a.st, a.vin, a.vout);
 }
 
-// nt == 0 selects the LDS-staged kernel.
 template <bool F>
 void apply_mode(u32 nt, u32 pu, hipStream_t s, u32 nslots, const Nbr& P, const PairList& L,
                 const ApplyArgs& a) {
@@ -2907,7 +2920,7 @@ void apply_mode(u32 nt, u32 pu, hipStream_t s, u32 nslots, const Nbr& P, const P
         WSIM_LAUNCH_CHECK();
         return;
     }
-    if (nt == 0) {
+    if (nt == 0 || nt == kOneLane) {
         switch (pu) {
         case 2: apply_staged<2, F>(s, nslots, P, L, a); break;
         case 4: apply_staged<4, F>(s, nslots, P, L, a); break;
@@ -2981,9 +2994,10 @@ bool valid_shapes(const KernelShapes& s) {
     auto in = [](u32 v, std::initializer_list<u32> set) {
         return std::find(set.begin(), set.end(), v) != set.end();
     };
-    return in(s.density_alpha_nt, {64, 128, 256, 512}) && in(s.xsph_nt, {0, 64, 128, 256, 512}) &&
-           in(s.change_nt, {0, 256, 512, 1024}) && in(s.change_pu, {2, 4, 8}) &&
-           in(s.apply_nt, {0, 64, 128, 256, 512}) && in(s.apply_pu, {2, 4, 8}) &&
+    return in(s.density_alpha_nt, {1, 4, 64, 128, 256, 512}) &&
+           in(s.xsph_nt, {0, 1, 4, 64, 128, 256, 512}) &&
+           in(s.change_nt, {0, 1, 4, 256, 512, 1024}) && in(s.change_pu, {2, 4, 8}) &&
+           in(s.apply_nt, {0, 1, 4, 64, 128, 256, 512}) && in(s.apply_pu, {2, 4, 8}) &&
            in(s.cell_cpt, {4, 8, 16}) && in(s.remap, {0, 1});
 }
 
@@ -4068,7 +4082,7 @@ void DFSPHSolver::autotune(int reps) {
             const Nbr P = nbr(remap);
             double b_da = 1e300, b_xs = 1e300, b_ch = 1e300, b_ap = 1e300;
             KernelShapes cand = best;
-            for (u32 nt : {64u, 128u, 256u, 512u}) {
+            for (u32 nt : {kOneLane, kFourLanes, 64u, 128u, 512u}) {
                 const double ms = time_ms([&] {
                     launch_density_alpha(nt, stream_, nslots_, P, L, xs_.data(), rho_.data(),
                                          alpha_.data(), cfg_.fast_math != 0);
@@ -4077,7 +4091,7 @@ void DFSPHSolver::autotune(int reps) {
                 if (ms < b_da) b_da = ms, cand.density_alpha_nt = nt;
             }
             if (any_xsph_) {
-                for (u32 nt : {0u, 64u, 128u, 256u, 512u}) {
+                for (u32 nt : {kOneLane, kFourLanes, 64u, 128u, 256u, 512u}) {
                     const double ms = time_ms([&] {
                         launch_xsph(nt, stream_, nslots_, P, L, xs_.data(), vpre_.data(),
                                     rho_.data(), vs_.data(), cfg_.fast_math != 0);
@@ -4088,8 +4102,9 @@ void DFSPHSolver::autotune(int reps) {
             } else {
                 b_xs = 0.0;
             }
-            for (u32 nt : {0u, 256u, 512u, 1024u})
-                for (u32 pu : {2u, 4u, 8u}) {
+            for (u32 nt : {kOneLane, kFourLanes, 256u, 512u, 1024u})
+                for (u32 pu : {4u, 2u, 8u}) {
+                    if (nt == kFourLanes && pu != 4u) continue;  // has no such parameter
                     const double ms = time_ms(
                         [&] { launch_change<0>(nt, pu, stream_, nslots_, P, L, ca); });
                     tune_log_.push_back({kKDensityChange, nt, pu, remap, 0, ms});
@@ -4098,8 +4113,9 @@ void DFSPHSolver::autotune(int reps) {
             // the error partials in the layout that the chosen k_change leaves
             launch_change<0>(cand.change_nt, cand.change_pu, stream_, nslots_, P, L, ca);
             aa.quarters = sweeps_by_quads(cand.change_nt, nslots_, cfg_.fast_math != 0) ? 1 : 0;
-            for (u32 nt : {0u, 64u, 128u, 256u, 512u})
-                for (u32 pu : {2u, 4u, 8u}) {
+            for (u32 nt : {kOneLane, kFourLanes, 64u, 128u, 256u, 512u})
+                for (u32 pu : {4u, 2u, 8u}) {
+                    if (nt == kFourLanes && pu != 4u) continue;
                     const double ms =
                         time_ms([&] { launch_apply(nt, pu, stream_, nslots_, P, L, aa); });
                     tune_log_.push_back({kKApplyKappa, nt, pu, remap, 0, ms});

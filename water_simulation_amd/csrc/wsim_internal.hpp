@@ -434,13 +434,14 @@ constexpr u32 kPairDepthBoundary = 48;
 // Launch shapes of the stencil kernels.  Every choice computes the same bits;
 // the autotuner times them on the solver's own data and keeps the fastest.
 struct KernelShapes {
-    u32 density_alpha_nt = 256;  // workgroup size: 64, 128, 256 (small sets: four lanes per
-                                 // particle), 512
-    u32 xsph_nt = 0;             // 0 (LDS-staged neighbourhood, 256; small sets: four lanes per
-                                 // particle), 64, 128, 256, 512
-    u32 change_nt = 0;           // 0 (as xsph_nt), 256, 512, 1024
+    // 1: one lane per particle, staged in LDS; 4: four lanes per particle; 256
+    // (density) or 0 (the others): one of the two by size; other values:
+    // workgroup sizes of the kernels without staging
+    u32 density_alpha_nt = 256;  // 1, 4, 64, 128, 256, 512
+    u32 xsph_nt = 0;             // 0, 1, 4, 64, 128, 256, 512
+    u32 change_nt = 0;           // 0, 1, 4, 256, 512, 1024
     u32 change_pu = 4;           // pairs per trip of the list loops: 2, 4, 8
-    u32 apply_nt = 0;            // 0 (as xsph_nt), 64, 128, 256, 512
+    u32 apply_nt = 0;            // 0, 1, 4, 64, 128, 256, 512
     u32 apply_pu = 4;            // 2, 4, 8
     u32 cell_cpt = 16;           // cells per thread of the cell_start pass: 4, 8, 16
     u32 remap = 1;               // XCD-aware workgroup -> tile order
