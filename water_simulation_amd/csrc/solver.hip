@@ -2702,7 +2702,7 @@ u32 grid_for(u32 nslots, u32 nt) { return div_up(nslots, nt); }
 //                    b 65k 66.1 -> 33.2  b 107k 66.4 -> 42.1  b 239k 69.6 -> 79.5
 //           change   4k  8.3 ->  6.1   65k 11.6 -> 10.6    95k 12.6 -> 12.8   b 65k 11.6 -> 11.3
 //           apply    4k  7.5 ->  5.8   65k 11.0 ->  9.0    95k 11.6 -> 11.6   b 65k 11.0 -> 10.4
-//           XSPH     4k  9.8 ->  5.0   65k 13.4 -> 12.5    98k 14.4 -> 15.5   b 65k 16.3 -> 13.0
+//           XSPH     4k  9.8 ->  5.0   49k 10.5 ->  9.8    65k 10.5 -> 10.7   b 65k 16.3 -> 13.0
 //   tolerance mode
 //           density  4k 28.4 -> 12.9   65k 26.3 -> 21.4    95k 27.5 -> 26.4   131k 24.9 -> 35.2
 //                    b 65k 36.4 -> 26.0  b 107k 37.8 -> 33.7
@@ -2710,12 +2710,15 @@ u32 grid_for(u32 nslots, u32 nt) { return div_up(nslots, nt); }
 //           apply    4k  6.6 ->  4.5   33k  6.0 ->  5.3    49k  6.2 ->  6.8   b 30k 7.9 -> 7.5
 //           XSPH     4k  8.4 ->  4.6   65k  8.4 ->  8.0    95k 10.4 -> 10.5   b 65k 14.0 -> 11.3
 // The lines lie inside the range where four lanes win (exact density: it ends
-// between 131k and 197k).
+// between 131k and 197k).  In tolerance mode the density walk of scenes without
+// a boundary, whose lanes all have the same little work, crosses earlier:
+// 65k 23.7 -> 22.7, 98k 24.4 -> 28.0.
 struct QuadLimits {
     u32 density, xsph, sweeps;
 };
-constexpr QuadLimits quad_limits(bool fast) {
-    return fast ? QuadLimits{98304, 65536, 40960} : QuadLimits{131072, 65536, 65536};
+constexpr QuadLimits quad_limits(bool fast, bool walls = true) {
+    return fast ? QuadLimits{walls ? 98304u : 65536u, 65536, 40960}
+                : QuadLimits{131072, 65536, 65536};
 }
 // Shape values 1 and 4: one lane per particle (256 threads, staged in LDS) and
 // four lanes per particle, at any size.
@@ -2731,7 +2734,7 @@ bool sweeps_by_quads(u32 nt, u32 nslots, bool fast) {
 template <bool F>
 void density_alpha_mode(u32 nt, hipStream_t s, u32 nslots, const Nbr& P, const PairList& L,
                         const float4* xs, float* rho, float* alpha, DeviceState* open) {
-    if (by_quads(nt, 256, nslots, quad_limits(F).density)) {
+    if (by_quads(nt, 256, nslots, quad_limits(F, P.nb != 0).density)) {
         k_density_alpha_q<F><<<nslots / kQuadGroup, NS, 0, s>>>(P, L, xs, rho, alpha, open);
         WSIM_LAUNCH_CHECK();
         return;
