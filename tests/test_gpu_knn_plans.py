@@ -47,3 +47,21 @@ def test_smoothing_equals_brute_force(case, k, monkeypatch):
     m = WM.SurfaceMesher()
     m.run(x, radius=R, smooth_pre=2, k_neighbors=k)
     _compare(m, M.reconstruct_splat(x, radius=R, smooth_pre=2, k=k), f"{case} k={k}")
+
+
+def test_more_points_than_one_launch_holds_groups():
+    """2,097,152 points fill the launch of the point groups; the rest are taken
+    in a second stride (2^29 points would be 2^32 threads, more than a launch
+    may hold)."""
+    from water_simulation_amd import mesh as WM
+
+    n = 65536 * 32 + 4099
+    side = 129
+    rng = np.random.default_rng(11)
+    g = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    x = (0.1 + 2.0 * R * (g + rng.uniform(-0.2, 0.2, g.shape))).astype(np.float32)
+    assert len(x) == n
+    m = WM.SurfaceMesher()
+    opt = dict(radius=R, smooth_pre=1, smooth_post=0)
+    m.run(x, k_neighbors=8, grid_voxel_factor=6.0, smooth_sigma=1.0, **opt)
+    _compare(m, M.reconstruct_splat(x, k=8, voxel_factor=6.0, sigma=1.0, **opt), "strided groups")

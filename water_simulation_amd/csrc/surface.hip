@@ -1437,7 +1437,10 @@ static void knn_pass(const double* in, u32 n, const KnnGrid& kg, const u32* sort
     auto list = [&](int k) { return lists + static_cast<u64>(k) * n; };
     enum { few, many, fewer, rest, far };
     static_assert(far + 1 == kKnnLists, "one list each");
-    auto blocks = [&](u32 lanes) { return div_up(n, kMeshThreads / lanes); };
+    // (a launch holds fewer than 2^32 threads, eight a point here: 2^29 points;
+    // the groups stride over what is left)
+    constexpr u32 kGroupBlocks = 1u << 16;
+    auto blocks = [&](u32 lanes) { return std::min(div_up(n, kMeshThreads / lanes), kGroupBlocks); };
     k_knn_group<K, 1, kNear, true><<<blocks(kNear), kMeshThreads, 0, s>>>(
         n, nullptr, nullptr, kg, sorted, ps, cs, out, counts + few, list(few), counts + many,
         list(many));
