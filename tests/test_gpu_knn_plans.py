@@ -65,3 +65,48 @@ def test_more_points_than_one_launch_holds_groups():
     opt = dict(radius=R, smooth_pre=1, smooth_post=0)
     m.run(x, k_neighbors=8, grid_voxel_factor=6.0, smooth_sigma=1.0, **opt)
     _compare(m, M.reconstruct_splat(x, k=8, voxel_factor=6.0, sigma=1.0, **opt), "strided groups")
+
+
+def block(side, spacing, seed=3):
+    rng = np.random.default_rng(seed)
+    g = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    x = 0.1 + spacing * (g + rng.uniform(-0.2, 0.2, g.shape))
+    return x[rng.permutation(len(x))].astype(np.float32)
+
+
+@pytest.mark.parametrize("k", [8, 15, 30])
+@pytest.mark.parametrize("ratio", [3.0, 20.0])
+def test_spacing_well_above_the_radius(ratio, k, monkeypatch):
+    """The radius says a spacing, the points lie `ratio` times as far apart: the
+    search takes the spacing from the points."""
+    from water_simulation_amd import mesh as WM
+
+    monkeypatch.setattr(M, "smooth_positions_knn", brute)
+    x = block(9, ratio * 2.0 * R)
+    x[:20] = x[20:40] + 0.01 * R  # close pairs
+    opt = dict(radius=R, smooth_pre=2, smooth_post=0)
+    m = WM.SurfaceMesher()
+    m.run(x, k_neighbors=k, grid_voxel_factor=2.0 * ratio, **opt)
+    _compare(m, M.reconstruct_splat(x, k=k, voxel_factor=2.0 * ratio, **opt), f"{ratio} k={k}")
+
+
+def test_time_does_not_hang_on_the_radius():
+    """97,336 points with the radius right, and 3 and 10 times too small: about
+    the same time (4 and 40 times as long while every point went through the
+    wide searches)."""
+    import time
+
+    from water_simulation_amd import mesh as WM
+
+    x = block(46, 2.0 * R)
+    ms = {}
+    for ratio in (1.0, 3.0, 10.0):
+        m = WM.SurfaceMesher()
+        t = []
+        for k in range(8):
+            t0 = time.perf_counter()
+            m.run(x, radius=R / ratio, grid_voxel_factor=ratio, smooth_sigma=1.0, smooth_post=0)
+            t.append(time.perf_counter() - t0)
+        ms[ratio] = 1e3 * float(np.median(t[2:]))
+    print(ms)
+    assert ms[3.0] < 2.5 * ms[1.0] and ms[10.0] < 2.5 * ms[1.0]

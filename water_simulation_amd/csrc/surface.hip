@@ -273,6 +273,17 @@ __device__ __forceinline__ void knn_scan(u32 lo, u32 hi, double px, double py, d
 // out go to a list that k_knn_far searches a wave per point.
 constexpr int kKnnLaneRings = 3;
 
+// Number of different keys among n sorted ones, added to *used.
+__global__ __launch_bounds__(kMeshThreads) void k_knn_used(const u32* __restrict__ keys, u32 n,
+                                                           u32* __restrict__ used) {
+    u32 c = 0;
+    for (u64 k = static_cast<u64>(blockIdx.x) * kMeshThreads + threadIdx.x; k < n;
+         k += static_cast<u64>(gridDim.x) * kMeshThreads)
+        c += k == 0 || keys[k] != keys[k - 1] ? 1u : 0u;
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(used, c);
+}
+
 template <int K>
 __device__ __forceinline__ void knn_lane(const double* __restrict__ P, KnnGrid g,
                                          const u32* __restrict__ sorted,
@@ -1554,6 +1565,7 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
     // 1. k-nearest-neighbour position smoothing (:61-74)
     int cur = 0;
     double mn[3], mx[3];
+    double dia = 2.0 * P.particle_radius;  // expected spacing
     for (int it = 0; it < P.smooth_pre_iters; ++it) {
         bounds(pts_[cur].data(), mn, mx);
         KnnGrid kg{};
@@ -1563,33 +1575,70 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
         // a cell's edge is the guess, so rings 0..1 reach it (a pass of
         // 1,001,385 points: 312 us; 353 with cells 1.15 times as wide; with
         // 0.85 most points fall short and take 1,400).
-        const double dia = 2.0 * P.particle_radius;
         const double box = (mx[0] - mn[0] + dia) * (mx[1] - mn[1] + dia) * (mx[2] - mn[2] + dia);
-        const double spacing = std::min(dia, std::cbrt(box / static_cast<double>(n)));
-        const double gr = knn_radius(P.k_neighbors + 4.0) * spacing;
-        kg.guess = gr * gr;
+        const double room = std::cbrt(box / static_cast<double>(n));
+        const double unit = knn_radius(P.k_neighbors + 4.0);
+        double gr = unit * std::min(dia, room);
         kg.cell = gr;
-        u64 cells = 0;
-        for (;;) {
-            kg.d0 = static_cast<int>((mx[0] - mn[0]) / kg.cell) + 1;
-            kg.d1 = static_cast<int>((mx[1] - mn[1]) / kg.cell) + 1;
-            kg.d2 = static_cast<int>((mx[2] - mn[2]) / kg.cell) + 1;
-            cells = static_cast<u64>(kg.d0) * kg.d1 * kg.d2;
-            if (cells <= (1ull << 26)) break;
-            kg.cell *= 2.0;
-        }
         if (knn_keys_[0].size() < n) {
             for (auto& b : knn_keys_) b = DeviceBuffer<u32>(n);
             for (auto& b : knn_vals_) b = DeviceBuffer<u32>(n);
             knn_hist_ = DeviceBuffer<u32>(radix_hist_elems(n));
         }
+        if (knn_farc_.size() < kKnnLists) knn_farc_ = DeviceBuffer<u32>(kKnnLists);
+        int w = 0;
+        auto sort_cells = [&] {
+            u64 cells = 0;
+            for (;;) {
+                kg.d0 = static_cast<int>((mx[0] - mn[0]) / kg.cell) + 1;
+                kg.d1 = static_cast<int>((mx[1] - mn[1]) / kg.cell) + 1;
+                kg.d2 = static_cast<int>((mx[2] - mn[2]) / kg.cell) + 1;
+                cells = static_cast<u64>(kg.d0) * kg.d1 * kg.d2;
+                if (cells <= (1ull << 26)) break;
+                kg.cell *= 2.0;
+            }
+            k_knn_keys<<<gp, kMeshThreads, 0, s>>>(pts_[cur].data(), nn, kg, knn_keys_[0].data(),
+                                                   knn_vals_[0].data());
+            WSIM_LAUNCH_CHECK();
+            w = radix_sort_pairs(knn_keys_[0].data(), knn_vals_[0].data(), knn_keys_[1].data(),
+                                 knn_vals_[1].data(), n, key_bits(static_cast<u32>(cells - 1)),
+                                 knn_hist_.data(), s);
+            return cells;
+        };
+        u64 cells = sort_cells();
+        // A box with room for ten times the points at that spacing is one of
+        // spray, or the radius is well below the spacing: then nearly every
+        // point would fall short of the guess and go through all the wide
+        // searches.  A cell that holds little more than a point tells, and
+        // doubled cells until they hold as many as the guess does give the
+        // spacing, once a run.  Two passes over 97,290 points, us: radius 3
+        // times too small 2,104 -> 499, 10 times 20,519 -> 598 (right: 340;
+        // 17,550 points, half the radius: 312 -> 382, the price of the waits).
+        if (it == 0 && room > 2.2 * dia) {
+            auto points_per_cell = [&] {
+                u32 used = 0;
+                WSIM_HIP(hipMemsetAsync(knn_farc_.data(), 0, sizeof(u32), s));
+                k_knn_used<<<std::min<u32>(gp, 256), kMeshThreads, 0, s>>>(knn_keys_[w].data(), nn,
+                                                                           knn_farc_.data());
+                WSIM_LAUNCH_CHECK();
+                read_back(&used, knn_farc_.data(), sizeof(u32));
+                return static_cast<double>(n) / static_cast<double>(used);
+            };
+            double held = points_per_cell();
+            if (held < 1.3) {
+                while (cells > 1 && held < unit * unit * unit) {
+                    kg.cell *= 2.0;
+                    cells = sort_cells();
+                    held = points_per_cell();
+                }
+                dia = kg.cell / std::cbrt(held);
+                gr = unit * dia;
+                kg.cell = gr;
+                cells = sort_cells();
+            }
+        }
+        kg.guess = gr * gr;
         if (knn_cs_.size() < cells + 1) knn_cs_ = DeviceBuffer<u32>(cells + 1);
-        k_knn_keys<<<gp, kMeshThreads, 0, s>>>(pts_[cur].data(), nn, kg, knn_keys_[0].data(),
-                                               knn_vals_[0].data());
-        WSIM_LAUNCH_CHECK();
-        const int w = radix_sort_pairs(knn_keys_[0].data(), knn_vals_[0].data(), knn_keys_[1].data(),
-                                       knn_vals_[1].data(), n, key_bits(static_cast<u32>(cells - 1)),
-                                       knn_hist_.data(), s);
         build_cell_start(knn_keys_[w].data(), nn, static_cast<u32>(cells + 1), knn_cs_.data(), s,
                          0);
         const u32* sorted = knn_vals_[w].data();
@@ -1601,7 +1650,6 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
         const double* ps = knn_ps_.data();
         const u32* cs = knn_cs_.data();
         if (knn_far_.size() < kKnnLists * n) knn_far_ = DeviceBuffer<u32>(kKnnLists * n);
-        if (knn_farc_.size() < kKnnLists) knn_farc_ = DeviceBuffer<u32>(kKnnLists);
         u32* fc = knn_farc_.data();  // counts of the lists
         WSIM_HIP(hipMemsetAsync(fc, 0, kKnnLists * sizeof(u32), s));
         u32* lists = knn_far_.data();
