@@ -350,6 +350,16 @@ template <> struct PairMath<true> {
     }
 };
 
+// LDS writes of a wave's lanes before this are read by its other lanes behind
+// it.  The wave's LDS instructions stay in order; the fence keeps the compiler
+// from moving accesses across, the barrier (no instruction) from giving lanes
+// on the two sides of a branch copies of what follows, which would run one
+// after the other.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Workgroup id remap so that each XCD walks a contiguous run of tiles: the
 // dispatcher hands workgroup b to XCD (b % 8), so neighbouring tiles (which
 // gather the same cell-sorted particles) land in the same L2.

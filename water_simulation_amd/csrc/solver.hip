@@ -2550,7 +2550,7 @@ __device__ __forceinline__ void for_candidates(const QuadRows<F ? 1 : 3>& W, u32
                 first += n;
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        wave_lds_sync();
         const u32 n = min(W.total - w0, kCand);
         constexpr int U = 4;
         for (u32 q0 = 0; q0 < n; q0 += 4 * U) {
@@ -2567,7 +2567,7 @@ __device__ __forceinline__ void for_candidates(const QuadRows<F ? 1 : 3>& W, u32
             for (int u = 0; u < U; ++u)
                 use(q0 + 4u * u + g < n, s[u] & ((1u << kCandRow) - 1u), s[u] >> kCandRow, q[u]);
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        wave_lds_sync();
     }
 }
 

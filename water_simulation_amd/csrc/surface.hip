@@ -409,7 +409,7 @@ __global__ __launch_bounds__(kMeshThreads) void k_knn_group(
     const int pt = threadIdx.x / G, lane = threadIdx.x % G;
     const u32 total = list ? *list_count : n;
     // LDS below is private to the group, whose lanes share a wave
-    auto sync = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+    auto sync = [] { wave_lds_sync(); };
     for (u32 f = blockIdx.x * kPts + pt; f < total; f += gridDim.x * kPts) {
         const u32 q = list ? list[f] : f;
         const double px = Ps[3ull * q], py = Ps[3ull * q + 1], pz = Ps[3ull * q + 2];
@@ -417,6 +417,7 @@ __global__ __launch_bounds__(kMeshThreads) void k_knn_group(
         const int h1 = knn_cell(py, g.lo1, g.cell, g.d1);
         const int h2 = knn_cell(pz, g.lo2, g.cell, g.d2);
         const int c0 = max(h2 - R, 0), c1 = min(h2 + R, g.d2 - 1);
+        sync();  // (the point before may have ended at a continue)
         for (int r = lane; r < kRows; r += G) {
             const int a = h0 - R + r / W, b = h1 - R + r % W;
             const bool in = a >= 0 && a < g.d0 && b >= 0 && b < g.d1;
@@ -813,7 +814,7 @@ __global__ __launch_bounds__(256) void k_blur_rows(const float* __restrict__ in,
     const u64 first = (static_cast<u64>(blockIdx.x) * 4 + wave) * kBlurRows;
     const u64 last = min(first + kBlurRows, rows);
     // the wave's own LDS: its instructions stay in order
-    auto sync = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+    auto sync = [] { wave_lds_sync(); };
     // RT > 0: the next segment's loads are in flight while this one is summed
     constexpr int kLoads = RT > 0 ? (kBlurSeg + 2 * RT + 63) / 64 : 1;
     float ahead[kLoads];
