@@ -110,3 +110,47 @@ def test_time_does_not_hang_on_the_radius():
         ms[ratio] = 1e3 * float(np.median(t[2:]))
     print(ms)
     assert ms[3.0] < 2.5 * ms[1.0] and ms[10.0] < 2.5 * ms[1.0]
+
+
+@pytest.mark.parametrize("k", [8, 15, 30])
+def test_dense_spots_beside_the_expected_spacing(k, monkeypatch):
+    """Points at a tenth and a fiftieth of the expected spacing (the bins are
+    narrowed round by round), more at one place than a list holds, and rows too
+    long for the guess."""
+    from water_simulation_amd import mesh as WM
+
+    monkeypatch.setattr(M, "smooth_positions_knn", brute)
+    rng = np.random.default_rng(k)
+    x = block(9, 2.0 * R, seed=k).astype(np.float64)
+    dense = x[0] + rng.uniform(-1.0, 1.0, (700, 3)) * R
+    denser = x[300] + rng.uniform(-1.0, 1.0, (300, 3)) * 0.15 * R
+    x = np.concatenate([x, dense, denser, np.repeat(x[500:501], 90, 0)]).astype(np.float32)
+    x = x[rng.permutation(len(x))]
+    m = WM.SurfaceMesher()
+    m.run(x, radius=R, smooth_pre=2, k_neighbors=k, smooth_post=0)
+    _compare(m, M.reconstruct_splat(x, radius=R, smooth_pre=2, k=k, smooth_post=0), f"dense k={k}")
+
+
+def test_time_of_a_dense_spot():
+    """30,000 points at a sixth of the expected spacing inside 10,648 others:
+    every search there reads the same thousands of candidates, a few times.
+    About 24 times the time of the block alone (65 times while every such point
+    was binned once and then searched by one lane)."""
+    import time
+
+    from water_simulation_amd import mesh as WM
+
+    rng = np.random.default_rng(0)
+    b = block(22, 2.0 * R)
+    c = (0.3 + 2.5 * R * rng.uniform(-1.0, 1.0, (30000, 3))).astype(np.float32)
+    ms = []
+    for x in (b, np.concatenate([b, c])):
+        m = WM.SurfaceMesher()
+        t = []
+        for _ in range(7):
+            t0 = time.perf_counter()
+            m.run(x, radius=R, smooth_sigma=1.0, smooth_post=0)
+            t.append(1e3 * (time.perf_counter() - t0))
+        ms.append(float(np.median(t[2:])))
+    print(ms, ms[1] / ms[0])
+    assert ms[1] < 42.0 * ms[0]

@@ -379,15 +379,20 @@ __device__ __forceinline__ void wave_append(u32* __restrict__ list, u32* __restr
 //   GUESS: g.guess, the squared radius that holds about K + 4 points at the
 //     expected spacing, in one visit of the candidates;
 //   else: the first of kKnnBins bins of [0, reach^2) at which K points are
-//     counted, in two visits.
+//     counted, in two visits; where that bin brings more than the list holds
+//     (dense spots), the bins of the range up to it, and so on.
 // Either way it lies below the reach, the point's own distance to the faces
 // of the scanned block (none where the block ends the grid).  Points with
 // fewer than K neighbours in the limit go to `few`, with more than the list
 // holds to `many`.  A pass over 1,001,385 points, 15 neighbours, with the
 // guess: 312 us with 8 lanes, 412 with 4, 403 with 16 (one lane a point:
 // 1,267); 17,056 points: 18 us with 8 lanes (256).  Bins in both visits for
-// every point: 799 us.
+// every point: 799 us.  Two passes over 30,000 points at a sixth of the expected
+// spacing among 10,648 others, ms: narrowing 10.7, without (one lane a point
+// for those) 29, one lane for every point 13.3.
 constexpr int kKnnBins = 32;
+constexpr u32 kKnnLong = 512;  // candidates of a row (three cells of about k / 3 points)
+constexpr int kKnnRounds = 6;  // a round narrows the range to an eighth or less where it helps
 constexpr int kKnnLists = 5;  // of points, between the passes of knn_pass
 constexpr int knn_cap(int k) { return k <= 16 ? 32 : 64; }  // listed points
 template <int K, int R, int G, bool GUESS>
@@ -418,14 +423,18 @@ __global__ __launch_bounds__(kMeshThreads) void k_knn_group(
         const int h2 = knn_cell(pz, g.lo2, g.cell, g.d2);
         const int c0 = max(h2 - R, 0), c1 = min(h2 + R, g.d2 - 1);
         sync();  // (the point before may have ended at a continue)
+        if (lane == 0) s_cnt[pt] = 0;
+        sync();
         for (int r = lane; r < kRows; r += G) {
             const int a = h0 - R + r / W, b = h1 - R + r % W;
             const bool in = a >= 0 && a < g.d0 && b >= 0 && b < g.d1;
             const u32 row = in ? (static_cast<u32>(a) * g.d1 + b) * g.d2 : 0u;
-            s_lo[pt][r] = in ? cs[row + c0] : 0u;
-            s_hi[pt][r] = in ? cs[row + c1 + 1] : 0u;
+            const u32 first = in ? cs[row + c0] : 0u, end = in ? cs[row + c1 + 1] : 0u;
+            s_lo[pt][r] = first;
+            s_hi[pt][r] = end;
+            // forty times the expected points: not a place for the guess
+            if (GUESS && end - first > kKnnLong) s_cnt[pt] = kCap + 1;
         }
-        if (lane == 0) s_cnt[pt] = 0;
         // distance to the faces of the scanned block that other cells touch
         double reach = INFINITY;
         auto face = [&](double p, double lo, int h, int d) {
@@ -465,40 +474,61 @@ __global__ __launch_bounds__(kMeshThreads) void k_knn_group(
         if constexpr (GUESS) {
             const double lim = fmin(g.guess, reach * reach);
             sync();
-            visit([&](u32 s, double d) {
-                if (d < lim) append(s, d);
-            });
+            const bool crowded = s_cnt[pt] != 0;
+            sync();
+            if (!crowded)
+                visit([&](u32 s, double d) {
+                    if (d < lim) append(s, d);
+                });
             sync();
             m = s_cnt[pt];
         } else {
-            for (int k = lane; k < kKnnBins / 2; k += G) s_bin[pt][k] = 0;
             sync();
             u32 have = 0;
             for (int r = 0; r < kRows; ++r) have += s_hi[pt][r] - s_lo[pt][r];
             overfull = have > 0xFFFFu;
-            const float scale =
-                reach > 0.0 ? static_cast<float>(static_cast<double>(kKnnBins) / (reach * reach))
-                            : INFINITY;
+            double span = reach * reach;  // the bins' range
+            float scale = 0.0f;
             int top = -1;  // last bin of the list
-            if (!overfull) {
-                // the bin is monotone in d; the last one may miss points
-                // beyond the block and never counts
+            u32 last = 0;
+            for (int round = 0; !overfull && round < kKnnRounds; ++round) {
+                for (int k = lane; k < kKnnBins / 2; k += G) s_bin[pt][k] = 0;
+                sync();
+                scale = span > 0.0 ? static_cast<float>(static_cast<double>(kKnnBins) / span)
+                                   : INFINITY;
+                // the bin is monotone in d; the last one of the whole range
+                // may miss points beyond the block and never counts
+                const int bins = round == 0 ? kKnnBins - 1 : kKnnBins;
+                u32 same = 0;
                 visit([&](u32, double d) {
+                    same += d == 0.0 ? 1u : 0u;
                     const float bin = static_cast<float>(d) * scale;
-                    if (bin < static_cast<float>(kKnnBins - 1)) {
+                    if (bin < static_cast<float>(bins)) {
                         const u32 b = static_cast<u32>(bin);
                         atomicAdd(&s_bin[pt][b >> 1], b & 1u ? 0x10000u : 1u);
                     }
                 });
+                if (same) atomicAdd(&s_cnt[pt], same);
                 sync();
+                // more points at one place than the list holds: no bins part them
+                overfull = s_cnt[pt] > kCap;
+                sync();
+                if (lane == 0) s_cnt[pt] = 0;
+                m = 0;
 #pragma unroll
-                for (int b = 0; b < kKnnBins - 1; ++b) {
+                for (int b = 0; b < kKnnBins; ++b) {
                     const u32 c = (s_bin[pt][b >> 1] >> (16 * (b & 1))) & 0xFFFFu;
                     if (m < static_cast<u32>(K)) {
                         m += c;
                         top = b;
                     }
                 }
+                sync();
+                // a dense spot: the same again over the bins up to there, while
+                // that tells the points apart
+                if (m <= kCap || m == last) break;
+                last = m;
+                span *= static_cast<double>(top + 1) / static_cast<double>(kKnnBins);
             }
             if (m >= static_cast<u32>(K) && m <= kCap) {
                 const float lim = static_cast<float>(top + 1);
