@@ -491,3 +491,34 @@ def test_gpu_knn_smoothing_rejects_bad_k():
         m.run(_cloud(1, n_side=4), k_neighbors=7)
     with pytest.raises(InvalidArgument):
         m.run(np.zeros((10, 3), np.float32), k_neighbors=15)
+
+
+@pytest.mark.gpu
+def test_gpu_mesher_keeps_nothing_of_other_frames():
+    """One mesher on a small, a large and again a small frame with other blurs,
+    neighbour counts and smoothings: each equals the oracle."""
+    from water_simulation_amd import mesh as WM
+
+    rng = np.random.default_rng(9)
+    r = 0.012
+
+    def frame(n, wide):
+        g = np.stack(np.meshgrid(*[np.arange(n)] * 3, indexing="ij"), -1).reshape(-1, 3)
+        x = 0.1 + 2 * r * (g + rng.uniform(-0.3, 0.3, g.shape))
+        if wide:  # spray far above: a box mostly empty
+            x = np.concatenate([x, rng.uniform(0.0, 1.5, (60, 3))])
+        return x.astype(np.float32)
+
+    m = WM.SurfaceMesher()
+    for k, (n, wide, o) in enumerate([
+        (6, False, dict()),
+        (14, False, dict(sigma=4.2, k=8, smooth_post=5)),
+        (7, True, dict(sigma=1.0, k=30, smooth_pre=1)),
+        (5, False, dict(sigma=0.0, smooth_pre=0, smooth_post=0)),
+        (12, True, dict(sigma=3.0, smooth_pre=3, smooth_post=0)),
+        (6, False, dict()),
+    ]):
+        x = frame(n, wide)
+        names = dict(sigma="smooth_sigma", k="k_neighbors")
+        m.run(x, radius=r, **{names.get(a, a): b for a, b in o.items()})
+        _compare(m, M.reconstruct_splat(x, radius=r, **o), f"frame {k}")
