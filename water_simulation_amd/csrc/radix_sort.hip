@@ -28,6 +28,9 @@
 // cells, us, three kernels a digit -> now: 1,000 keys 42.3 -> 15.6, 4,000
 // 43.4 -> 21.6, 8,192 42.6 -> 30.8 (one workgroup) and 8,193 41.8 -> 29.9
 // (tiles): the lines cross there; 100,000 42.8 -> 36.1, 131,072 43.0 -> 35.0.
+// The tiles' own sums stay ahead of the row scan beyond kRadixFew (216,000
+// cells: 262,144 keys 47.9 -> 44.5, 400,000 53.8 -> 53.0) and fall behind from
+// 256 tiles on (524,288 keys 57.9 -> 59.9, 1,000,000 78.8 -> 103.9).
 #include "device_math.hpp"
 #include "radix_sort.hpp"
 
