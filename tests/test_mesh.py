@@ -522,3 +522,26 @@ def test_gpu_mesher_keeps_nothing_of_other_frames():
         names = dict(sigma="smooth_sigma", k="k_neighbors")
         m.run(x, radius=r, **{names.get(a, a): b for a, b in o.items()})
         _compare(m, M.reconstruct_splat(x, radius=r, **o), f"frame {k}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,split", [(9000, False), (30000, True)])
+def test_gpu_laplacian_of_rugged_surfaces(n, split):
+    """Vertices with more neighbours than the short list holds, on both sides of
+    the vertex count from which they have a launch of their own."""
+    from water_simulation_amd import mesh as WM
+
+    r = 0.012
+    x = np.random.default_rng(n).uniform(0.0, 2.2 * r * n ** (1 / 3), (n, 3)).astype(np.float32)
+    opt = dict(radius=r, smooth_pre=0, smooth_sigma=0.8, iso_factor=0.1)
+    m = WM.SurfaceMesher()
+    m.run(x, smooth_post=0, **opt)
+    v, t = m.vertices(), m.triangles()
+    assert (len(v) >= 262144) == split
+    a, b = np.sort(t[:, [0, 1, 1, 2, 2, 0]].reshape(-1, 2), 1).T
+    degree = np.bincount(np.unique(np.stack([a, b], 1), axis=0).ravel(), minlength=len(v))
+    assert (degree > 9).sum() > 100 and degree.max() <= 24
+    m.run(x, smooth_post=2, **opt)
+    want = M.laplacian_smooth(v, t, 2)
+    assert np.array_equal(m.triangles(), t)
+    assert np.array_equal(m.vertices().view(np.uint32), want.view(np.uint32))

@@ -1383,44 +1383,68 @@ __device__ __forceinline__ u32 mc_neighbours(const McGrid& M, const McDev& T, u3
     return n;
 }
 
-// Neighbours of every vertex, a thread each: in a short register list first
-// (a vertex has about six; every insertion passes the whole list), in the
-// full one for the few with more.
+// Neighbours of every vertex, a thread each: in a short register list first (a
+// vertex has about six, and every insertion passes the whole list), in the
+// full one for the vertices with more.  Those are few on smooth surfaces, and
+// kAdjAll takes them on the spot.  On rugged ones they make nearly every wave
+// go through both lists, so from kAdjSplit vertices on kAdjFirst lists them for
+// a launch of their own, kAdjRest (18.5 million vertices of a splash: 4,209 ->
+// 3,300 us; below, the launch costs what it saves).
 constexpr int kAdjShort = 9;
+constexpr u64 kAdjSplit = 262144;
+enum { kAdjAll, kAdjFirst, kAdjRest };
+template <int CAP>
+__device__ __forceinline__ void adj_store(u32* __restrict__ row, const u32 (&L)[CAP], u32 n) {
+#pragma unroll
+    for (int k = 0; k < CAP; ++k)
+        if (static_cast<u32>(k) < n) row[k] = L[k];
+}
+template <int MODE>
 __global__ __launch_bounds__(256) void k_mc_adjacency(McGrid M, const McDev* __restrict__ T,
                                                       u64 nvert, const u32* __restrict__ vpt,
                                                       const uint8_t* __restrict__ emask,
                                                       const u32* __restrict__ eoff,
                                                       u32* __restrict__ adj,
                                                       u32* __restrict__ deg,
+                                                      u32* __restrict__ more_count,
+                                                      u32* __restrict__ more,
                                                       u32* __restrict__ over) {
     __shared__ __align__(16) McDev sT;  // the table, read per lane below
     for (u32 k = threadIdx.x; k < sizeof(McDev) / 4; k += 256)
         reinterpret_cast<u32*>(&sT)[k] = reinterpret_cast<const u32*>(T)[k];
     __syncthreads();
+    constexpr bool kRest = MODE == kAdjRest;
     // an XCD takes a run of vertices: neighbours lie within a few planes, in its L2
-    const u64 v = static_cast<u64>(xcd_tile(blockIdx.x, gridDim.x)) * 256 + threadIdx.x;
-    if (v >= nvert) return;
-    const u32 code = vpt[v];  // this vertex's grid edge: from grid point i (< 2^30) along an axis
-    u32* row = adj + v * kAdjCap;
-    u32 L[kAdjShort];
-    u32 n = mc_neighbours<kAdjShort>(M, sT, code >> 2, static_cast<int>(code & 3u), emask, eoff, L);
-    if (n <= static_cast<u32>(kAdjShort)) {
-#pragma unroll
-        for (int k = 0; k < kAdjShort; ++k)
-            if (static_cast<u32>(k) < n) row[k] = L[k];
-    } else {
-        u32 F[kAdjCap];
-        n = mc_neighbours<kAdjCap>(M, sT, code >> 2, static_cast<int>(code & 3u), emask, eoff, F);
-        if (n > static_cast<u32>(kAdjCap)) {
-            atomicOr(over, 1u);
-            n = kAdjCap;
+    const u32 b = kRest ? blockIdx.x : xcd_tile(blockIdx.x, gridDim.x);
+    const u64 count = kRest ? static_cast<u64>(*more_count) : nvert;
+    for (u64 t = static_cast<u64>(b) * 256 + threadIdx.x; t < count;
+         t += static_cast<u64>(gridDim.x) * 256) {
+        const u32 v = kRest ? more[t] : static_cast<u32>(t);
+        const u32 code = vpt[v];  // its grid edge: from grid point i (< 2^30) along an axis
+        const int ax = static_cast<int>(code & 3u);
+        u32* row = adj + static_cast<u64>(v) * kAdjCap;
+        u32 n = kAdjShort + 1;
+        if constexpr (!kRest) {
+            u32 L[kAdjShort];
+            n = mc_neighbours<kAdjShort>(M, sT, code >> 2, ax, emask, eoff, L);
+            if (n <= static_cast<u32>(kAdjShort)) adj_store(row, L, n);
         }
-#pragma unroll
-        for (int k = 0; k < kAdjCap; ++k)
-            if (static_cast<u32>(k) < n) row[k] = F[k];
+        if (n > static_cast<u32>(kAdjShort)) {
+            if constexpr (MODE == kAdjFirst) {
+                wave_append(more, more_count, v);
+                continue;
+            } else {
+                u32 F[kAdjCap];
+                n = mc_neighbours<kAdjCap>(M, sT, code >> 2, ax, emask, eoff, F);
+                if (n > static_cast<u32>(kAdjCap)) {
+                    atomicOr(over, 1u);
+                    n = kAdjCap;
+                }
+                adj_store(row, F, n);
+            }
+        }
+        deg[v] = n;
     }
-    deg[v] = n;
 }
 
 __global__ __launch_bounds__(kMeshThreads) void k_verts_narrow(const double* __restrict__ in,
@@ -1884,12 +1908,24 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
     if (post) {
         fit(adj_, nvert * kAdjCap);
         fit(deg_, nvert);
-        fit(adj_over_, 1);
-        WSIM_HIP(hipMemsetAsync(adj_over_.data(), 0, sizeof(u32), s));
-        k_mc_adjacency<<<static_cast<u32>((nvert + 255) / 256), 256, 0, s>>>(
-            M, dT, nvert, vpt_.data(), emask_.data(), eoff_.data(), adj_.data(), deg_.data(),
-            adj_over_.data());
-        WSIM_LAUNCH_CHECK();
+        fit(adj_over_, 2);
+        WSIM_HIP(hipMemsetAsync(adj_over_.data(), 0, 2 * sizeof(u32), s));
+        u32* const flags = adj_over_.data();  // overflow, vertices listed
+        // the listed vertices lie in the smoothing's second buffer until its first pass
+        u32* const more = reinterpret_cast<u32*>(vd_[1].data());
+        const u32 ga = static_cast<u32>((nvert + 255) / 256);
+        auto neighbours = [&](auto mode, u32 blocks) {
+            k_mc_adjacency<decltype(mode)::value><<<blocks, 256, 0, s>>>(
+                M, dT, nvert, vpt_.data(), emask_.data(), eoff_.data(), adj_.data(), deg_.data(),
+                flags + 1, more, flags);
+            WSIM_LAUNCH_CHECK();
+        };
+        if (nvert < kAdjSplit) {
+            neighbours(std::integral_constant<int, kAdjAll>{}, ga);
+        } else {
+            neighbours(std::integral_constant<int, kAdjFirst>{}, ga);
+            neighbours(std::integral_constant<int, kAdjRest>{}, 2048);
+        }
         const u64 n3 = 3 * nvert;
         const u32 g3 = static_cast<u32>((n3 + kMeshThreads - 1) / kMeshThreads);
         const u32 g1 = static_cast<u32>((nvert + kMeshThreads - 1) / kMeshThreads);
