@@ -154,3 +154,18 @@ def test_time_of_a_dense_spot():
         ms.append(float(np.median(t[2:])))
     print(ms, ms[1] / ms[0])
     assert ms[1] < 42.0 * ms[0]
+
+
+@pytest.mark.parametrize("n", [31, 2047, 2048, 2049, 4096, 6145])
+def test_every_point_through_the_lists(n):
+    """Points 1.6 times the expected spacing apart: every one falls short of the
+    guess, so the parts of the list are filled to their capacity (2,048 points
+    are one workgroup's for each part) and a little more."""
+    from water_simulation_amd import mesh as WM
+
+    side = int(np.ceil(n ** (1 / 3)))
+    x = block(side, 1.6 * 2.0 * R, seed=n)[:n]
+    opt = dict(radius=R, smooth_pre=2, smooth_post=0)
+    m = WM.SurfaceMesher()
+    m.run(x, k_neighbors=15, grid_voxel_factor=1.0, **opt)
+    _compare(m, M.reconstruct_splat(x, k=15, voxel_factor=1.0, **opt), f"lists {n}")

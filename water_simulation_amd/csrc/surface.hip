@@ -198,6 +198,39 @@ __global__ __launch_bounds__(kMeshThreads) void k_mesh_splat(const double* __res
 // rings of cells around the home cell are scanned until the k-th distance is
 // below the ring's reach (points outside rings 0..R lie at least R cells away).
 
+// A list that many waves append to, in kParts parts: one counter takes about
+// 130 million atomics a second, 1 ms where 600,000 of a million points fall
+// short of the guessed radius (k_knn_group on a splash: 1,314 -> 273 us with 64
+// counters).  Workgroup t fills part t % kParts, and a consumer's workgroup reads one
+// part and appends to the same part of its own lists, so a part holds no more
+// than the items of its first producer's workgroups.
+constexpr u32 kParts = 64;
+constexpr u32 kPartLine = 16;  // counters apart by a cache line
+constexpr u32 kPartCounts = kParts * kPartLine;
+struct SplitList {
+    u32* count;
+    u32* items;
+    u32 cap;  // of a part
+    __device__ __forceinline__ u32 size(u32 part) const { return count[part * kPartLine]; }
+    __device__ __forceinline__ u32 at(u32 part, u32 k) const {
+        return items[static_cast<u64>(part) * cap + k];
+    }
+    // Appends q of every active lane, one atomic a wave.
+    __device__ __forceinline__ void wave_append(u32 part, u32 q) const {
+        const unsigned long long act = __ballot(1);
+        const int first = __ffsll(act) - 1, lane = threadIdx.x & 63;
+        u32 k = 0;
+        if (lane == first)
+            k = atomicAdd(count + part * kPartLine, static_cast<u32>(__popcll(act)));
+        k = __shfl(k, first, 64) + static_cast<u32>(__popcll(act & ((1ull << lane) - 1ull)));
+        items[static_cast<u64>(part) * cap + k] = q;
+    }
+};
+// Capacity of a part when `blocks` workgroups append up to `per` items each.
+inline u32 part_capacity(u64 blocks, u32 per) {
+    return static_cast<u32>((blocks + kParts - 1) / kParts) * per;
+}
+
 struct KnnGrid {
     double lo0, lo1, lo2, cell;
     double guess;  // squared radius of about k + 4 points
@@ -289,8 +322,7 @@ __device__ __forceinline__ void knn_lane(const double* __restrict__ P, KnnGrid g
                                          const u32* __restrict__ sorted,
                                          const double* __restrict__ Ps,
                                          const u32* __restrict__ cs, double* __restrict__ out,
-                                         u32* __restrict__ far_count, u32* __restrict__ far,
-                                         u32 q) {
+                                         const SplitList& far, u32 part, u32 q) {
     const u32 i = sorted[q];
     const double px = Ps[3ull * q], py = Ps[3ull * q + 1], pz = Ps[3ull * q + 2];
     const int h0 = knn_cell(px, g.lo0, g.cell, g.d0);
@@ -328,7 +360,7 @@ __device__ __forceinline__ void knn_lane(const double* __restrict__ P, KnnGrid g
         }
     }
     if (!done && rlim < rmax) {  // rings beyond rlim hold cells: leave it to k_knn_far
-        far[atomicAdd(far_count, 1u)] = q;
+        far.wave_append(part, q);
         return;
     }
     double sx = 0.0, sy = 0.0, sz = 0.0;
@@ -350,23 +382,12 @@ __device__ __forceinline__ void knn_lane(const double* __restrict__ P, KnnGrid g
 template <int K>
 __global__ __launch_bounds__(kMeshThreads) void k_knn_smooth(
     const double* __restrict__ P, KnnGrid g, const u32* __restrict__ sorted,
-    const double* __restrict__ Ps, const u32* __restrict__ cs, const u32* __restrict__ count,
-    const u32* __restrict__ list, double* __restrict__ out, u32* __restrict__ far_count,
-    u32* __restrict__ far) {
-    const u32 n = *count;
-    for (u32 k = blockIdx.x * kMeshThreads + threadIdx.x; k < n; k += gridDim.x * kMeshThreads)
-        knn_lane<K>(P, g, sorted, Ps, cs, out, far_count, far, list[k]);
-}
-
-// Appends q of every active lane to the list, one atomic a wave.
-__device__ __forceinline__ void wave_append(u32* __restrict__ list, u32* __restrict__ count,
-                                            u32 q) {
-    const unsigned long long act = __ballot(1);
-    const int first = __ffsll(act) - 1, lane = threadIdx.x & 63;
-    u32 at = 0;
-    if (lane == first) at = atomicAdd(count, static_cast<u32>(__popcll(act)));
-    at = __shfl(at, first, 64);
-    list[at + static_cast<u32>(__popcll(act & ((1ull << lane) - 1ull)))] = q;
+    const double* __restrict__ Ps, const u32* __restrict__ cs, SplitList list,
+    double* __restrict__ out, SplitList far) {
+    const u32 part = blockIdx.x % kParts, n = list.size(part);
+    const u32 stride = gridDim.x / kParts * kMeshThreads;
+    for (u32 k = blockIdx.x / kParts * kMeshThreads + threadIdx.x; k < n; k += stride)
+        knn_lane<K>(P, g, sorted, Ps, cs, out, far, part, list.at(part, k));
 }
 
 // G lanes per point over the rings 0..R at once.  A lane that keeps the K
@@ -397,10 +418,9 @@ constexpr int kKnnLists = 5;  // of points, between the passes of knn_pass
 constexpr int knn_cap(int k) { return k <= 16 ? 32 : 64; }  // listed points
 template <int K, int R, int G, bool GUESS>
 __global__ __launch_bounds__(kMeshThreads) void k_knn_group(
-    u32 n, const u32* __restrict__ list_count, const u32* __restrict__ list, KnnGrid g,
-    const u32* __restrict__ sorted, const double* __restrict__ Ps, const u32* __restrict__ cs,
-    double* __restrict__ out, u32* __restrict__ few_count, u32* __restrict__ few,
-    u32* __restrict__ many_count, u32* __restrict__ many) {
+    u32 n, SplitList list, KnnGrid g, const u32* __restrict__ sorted,
+    const double* __restrict__ Ps, const u32* __restrict__ cs, double* __restrict__ out,
+    SplitList few, SplitList many) {
     constexpr u32 kCap = knn_cap(K);
     static_assert(K <= kCap && kCap <= 256, "list holds the K nearest, places in 8 bits");
     constexpr int W = 2 * R + 1, kRows = W * W;
@@ -412,11 +432,15 @@ __global__ __launch_bounds__(kMeshThreads) void k_knn_group(
     __shared__ u32 s_slot[kPts][kCap];
     __shared__ uint8_t s_ord[kPts][K];
     const int pt = threadIdx.x / G, lane = threadIdx.x % G;
-    const u32 total = list ? *list_count : n;
+    // GUESS takes all points, a tile of kPts after the other, the others a part
+    // of their list
+    const u32 own = blockIdx.x % kParts;
+    const u32 total = GUESS ? n : list.size(own);
+    const u32 stride = (GUESS ? gridDim.x : gridDim.x / kParts) * kPts;
     // LDS below is private to the group, whose lanes share a wave
     auto sync = [] { wave_lds_sync(); };
-    for (u32 f = blockIdx.x * kPts + pt; f < total; f += gridDim.x * kPts) {
-        const u32 q = list ? list[f] : f;
+    for (u32 f = (GUESS ? blockIdx.x : blockIdx.x / kParts) * kPts + pt; f < total; f += stride) {
+        const u32 q = GUESS ? f : list.at(own, f);
         const double px = Ps[3ull * q], py = Ps[3ull * q + 1], pz = Ps[3ull * q + 2];
         const int h0 = knn_cell(px, g.lo0, g.cell, g.d0);
         const int h1 = knn_cell(py, g.lo1, g.cell, g.d1);
@@ -540,8 +564,9 @@ __global__ __launch_bounds__(kMeshThreads) void k_knn_group(
         }
         if (overfull || m < static_cast<u32>(K) || m > kCap) {
             if (lane == 0) {
-                if (!overfull && m < static_cast<u32>(K)) wave_append(few, few_count, q);
-                else wave_append(many, many_count, q);
+                const u32 part = GUESS ? f / kPts % kParts : own;
+                if (!overfull && m < static_cast<u32>(K)) few.wave_append(part, q);
+                else many.wave_append(part, q);
             }
             continue;
         }
@@ -585,16 +610,15 @@ __global__ __launch_bounds__(kMeshThreads) void k_knn_far(const double* __restri
                                                           const u32* __restrict__ sorted,
                                                           const double* __restrict__ Ps,
                                                           const u32* __restrict__ cs,
-                                                          const u32* __restrict__ far_count,
-                                                          const u32* __restrict__ far,
+                                                          SplitList far,
                                                           double* __restrict__ out) {
     const int lane = threadIdx.x & 63;
-    const u32 wave = (blockIdx.x * kMeshThreads + threadIdx.x) >> 6;
-    const u32 nwaves = (gridDim.x * kMeshThreads) >> 6;
-    const u32 nfar = *far_count;
+    const u32 part = blockIdx.x % kParts, nfar = far.size(part);
+    const u32 wave = (blockIdx.x / kParts * kMeshThreads + threadIdx.x) >> 6;
+    const u32 nwaves = (gridDim.x / kParts * kMeshThreads) >> 6;
     const int rmax = max(g.d0, max(g.d1, g.d2));
     for (u32 f = wave; f < nfar; f += nwaves) {
-        const u32 q = far[f];
+        const u32 q = far.at(part, f);
         const double px = Ps[3ull * q], py = Ps[3ull * q + 1], pz = Ps[3ull * q + 2];
         const int h0 = knn_cell(px, g.lo0, g.cell, g.d0);
         const int h1 = knn_cell(py, g.lo1, g.cell, g.d1);
@@ -1405,9 +1429,7 @@ __global__ __launch_bounds__(256) void k_mc_adjacency(McGrid M, const McDev* __r
                                                       const uint8_t* __restrict__ emask,
                                                       const u32* __restrict__ eoff,
                                                       u32* __restrict__ adj,
-                                                      u32* __restrict__ deg,
-                                                      u32* __restrict__ more_count,
-                                                      u32* __restrict__ more,
+                                                      u32* __restrict__ deg, SplitList more,
                                                       u32* __restrict__ over) {
     __shared__ __align__(16) McDev sT;  // the table, read per lane below
     for (u32 k = threadIdx.x; k < sizeof(McDev) / 4; k += 256)
@@ -1415,11 +1437,12 @@ __global__ __launch_bounds__(256) void k_mc_adjacency(McGrid M, const McDev* __r
     __syncthreads();
     constexpr bool kRest = MODE == kAdjRest;
     // an XCD takes a run of vertices: neighbours lie within a few planes, in its L2
-    const u32 b = kRest ? blockIdx.x : xcd_tile(blockIdx.x, gridDim.x);
-    const u64 count = kRest ? static_cast<u64>(*more_count) : nvert;
-    for (u64 t = static_cast<u64>(b) * 256 + threadIdx.x; t < count;
-         t += static_cast<u64>(gridDim.x) * 256) {
-        const u32 v = kRest ? more[t] : static_cast<u32>(t);
+    const u32 part = blockIdx.x % kParts;
+    const u32 b = kRest ? blockIdx.x / kParts : xcd_tile(blockIdx.x, gridDim.x);
+    const u64 count = kRest ? static_cast<u64>(more.size(part)) : nvert;
+    const u64 stride = static_cast<u64>(kRest ? gridDim.x / kParts : gridDim.x) * 256;
+    for (u64 t = static_cast<u64>(b) * 256 + threadIdx.x; t < count; t += stride) {
+        const u32 v = kRest ? more.at(part, static_cast<u32>(t)) : static_cast<u32>(t);
         const u32 code = vpt[v];  // its grid edge: from grid point i (< 2^30) along an axis
         const int ax = static_cast<int>(code & 3u);
         u32* row = adj + static_cast<u64>(v) * kAdjCap;
@@ -1431,7 +1454,7 @@ __global__ __launch_bounds__(256) void k_mc_adjacency(McGrid M, const McDev* __r
         }
         if (n > static_cast<u32>(kAdjShort)) {
             if constexpr (MODE == kAdjFirst) {
-                wave_append(more, more_count, v);
+                more.wave_append(part, v);
                 continue;
             } else {
                 u32 F[kAdjCap];
@@ -1508,40 +1531,45 @@ static double numpy_sum(const double* a, size_t n) {
 // then the points it held too many or too few neighbours for (surfaces, other
 // spacings; rings 0..4 reach k points at four times the expected spacing),
 // then dense and far neighbourhoods.
+constexpr u32 kNearLanes = 8;  // lanes per point of the first searches
+constexpr u32 kNearPoints = kMeshThreads / kNearLanes;
 template <int K>
 static void knn_pass(const double* in, u32 n, const KnnGrid& kg, const u32* sorted,
                      const double* ps, const u32* cs, double* out, u32* counts, u32* lists,
                      hipStream_t s) {
-    constexpr u32 kNear = 8, kWide = 16, kWave4 = 64;
-    auto list = [&](int k) { return lists + static_cast<u64>(k) * n; };
-    enum { few, many, fewer, rest, far };
-    static_assert(far + 1 == kKnnLists, "one list each");
+    constexpr u32 kWideLanes = 16, kWaveLanes = 64;
+    const u32 tiles = div_up(n, kNearPoints), cap = part_capacity(tiles, kNearPoints);
+    auto list = [&](u32 k) {
+        return SplitList{counts + k * kPartCounts, lists + static_cast<u64>(k) * kParts * cap, cap};
+    };
+    static_assert(kKnnLists == 5, "one each");
+    const SplitList few = list(0), many = list(1), fewer = list(2), rest = list(3), far = list(4);
     // (a launch holds fewer than 2^32 threads, eight a point here: 2^29 points;
     // the groups stride over what is left)
     constexpr u32 kGroupBlocks = 1u << 16;
-    auto blocks = [&](u32 lanes) { return std::min(div_up(n, kMeshThreads / lanes), kGroupBlocks); };
-    k_knn_group<K, 1, kNear, true><<<blocks(kNear), kMeshThreads, 0, s>>>(
-        n, nullptr, nullptr, kg, sorted, ps, cs, out, counts + few, list(few), counts + many,
-        list(many));
+    // workgroups of a list's consumer: the same number for every part
+    auto blocks = [&](u32 per, u32 most) {
+        return std::min(div_up(div_up(n, per), kParts) * kParts, most);
+    };
+    k_knn_group<K, 1, kNearLanes, true><<<std::min(tiles, kGroupBlocks), kMeshThreads, 0, s>>>(
+        n, SplitList{}, kg, sorted, ps, cs, out, few, many);
     WSIM_LAUNCH_CHECK();
-    k_knn_group<K, 1, kNear, false><<<std::min<u32>(blocks(kNear), 2048), kMeshThreads, 0, s>>>(
-        n, counts + many, list(many), kg, sorted, ps, cs, out, counts + few, list(few),
-        counts + rest, list(rest));
+    k_knn_group<K, 1, kNearLanes, false><<<blocks(kNearPoints, 2048), kMeshThreads, 0, s>>>(
+        n, many, kg, sorted, ps, cs, out, few, rest);
     WSIM_LAUNCH_CHECK();
-    k_knn_group<K, 2, kWide, false><<<std::min<u32>(blocks(kWide), 2048), kMeshThreads, 0, s>>>(
-        n, counts + few, list(few), kg, sorted, ps, cs, out, counts + fewer, list(fewer),
-        counts + rest, list(rest));
+    k_knn_group<K, 2, kWideLanes, false>
+        <<<blocks(kMeshThreads / kWideLanes, 2048), kMeshThreads, 0, s>>>(
+            n, few, kg, sorted, ps, cs, out, fewer, rest);
     WSIM_LAUNCH_CHECK();
-    k_knn_group<K, 4, kWave4, false><<<std::min<u32>(blocks(kWave4), 2048), kMeshThreads, 0, s>>>(
-        n, counts + fewer, list(fewer), kg, sorted, ps, cs, out, counts + rest, list(rest),
-        counts + rest, list(rest));
+    k_knn_group<K, 4, kWaveLanes, false>
+        <<<blocks(kMeshThreads / kWaveLanes, 2048), kMeshThreads, 0, s>>>(
+            n, fewer, kg, sorted, ps, cs, out, rest, rest);
     WSIM_LAUNCH_CHECK();
-    const u32 gd = std::min<u32>(div_up(n, static_cast<u32>(kMeshThreads)), 1024);
-    k_knn_smooth<K><<<gd, kMeshThreads, 0, s>>>(in, kg, sorted, ps, cs, counts + rest, list(rest),
-                                                out, counts + far, list(far));
+    k_knn_smooth<K><<<blocks(kMeshThreads, 1024), kMeshThreads, 0, s>>>(in, kg, sorted, ps, cs,
+                                                                        rest, out, far);
     WSIM_LAUNCH_CHECK();
-    const u32 gf = std::min<u32>(gd, 256);  // 4 waves per block walk the list
-    k_knn_far<K><<<gf, kMeshThreads, 0, s>>>(in, kg, sorted, ps, cs, counts + far, list(far), out);
+    // 4 waves per workgroup walk the list
+    k_knn_far<K><<<blocks(kMeshThreads, 256), kMeshThreads, 0, s>>>(in, kg, sorted, ps, cs, far, out);
     WSIM_LAUNCH_CHECK();
 }
 
@@ -1653,7 +1681,7 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
             for (auto& b : knn_vals_) b = DeviceBuffer<u32>(n);
             knn_hist_ = DeviceBuffer<u32>(radix_hist_elems(n));
         }
-        if (knn_farc_.size() < kKnnLists) knn_farc_ = DeviceBuffer<u32>(kKnnLists);
+        fit(knn_farc_, kKnnLists * kPartCounts);
         int w = 0;
         auto sort_cells = [&] {
             u64 cells = 0;
@@ -1717,9 +1745,10 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
         const double* in = pts_[cur].data();
         const double* ps = knn_ps_.data();
         const u32* cs = knn_cs_.data();
-        if (knn_far_.size() < kKnnLists * n) knn_far_ = DeviceBuffer<u32>(kKnnLists * n);
+        fit(knn_far_, static_cast<u64>(kKnnLists) * kParts *
+                          part_capacity(div_up(n, kNearPoints), kNearPoints));
         u32* fc = knn_farc_.data();  // counts of the lists
-        WSIM_HIP(hipMemsetAsync(fc, 0, kKnnLists * sizeof(u32), s));
+        WSIM_HIP(hipMemsetAsync(fc, 0, kKnnLists * kPartCounts * sizeof(u32), s));
         u32* lists = knn_far_.data();
         switch (P.k_neighbors) {
         case 8: knn_pass<8>(in, nn, kg, sorted, ps, cs, out, fc, lists, s); break;
@@ -1908,16 +1937,18 @@ void SurfaceMesher::run(const float* xyz, size_t n, const MeshParams& P) {
     if (post) {
         fit(adj_, nvert * kAdjCap);
         fit(deg_, nvert);
-        fit(adj_over_, 2);
-        WSIM_HIP(hipMemsetAsync(adj_over_.data(), 0, 2 * sizeof(u32), s));
-        u32* const flags = adj_over_.data();  // overflow, vertices listed
-        // the listed vertices lie in the smoothing's second buffer until its first pass
-        u32* const more = reinterpret_cast<u32*>(vd_[1].data());
+        fit(adj_over_, kPartLine + kPartCounts);  // the overflow flag, counts of the list
+        WSIM_HIP(hipMemsetAsync(adj_over_.data(), 0, (kPartLine + kPartCounts) * sizeof(u32), s));
         const u32 ga = static_cast<u32>((nvert + 255) / 256);
+        // listed vertices lie in the smoothing's second buffer until its first pass:
+        // 24 bytes a vertex, and from kAdjSplit on all parts are full but one round
+        static_assert(kAdjSplit >= kParts * 256, "parts of whole workgroups fit in the buffer");
+        const SplitList more{adj_over_.data() + kPartLine, reinterpret_cast<u32*>(vd_[1].data()),
+                             part_capacity(ga, 256)};
         auto neighbours = [&](auto mode, u32 blocks) {
             k_mc_adjacency<decltype(mode)::value><<<blocks, 256, 0, s>>>(
                 M, dT, nvert, vpt_.data(), emask_.data(), eoff_.data(), adj_.data(), deg_.data(),
-                flags + 1, more, flags);
+                more, adj_over_.data());
             WSIM_LAUNCH_CHECK();
         };
         if (nvert < kAdjSplit) {
