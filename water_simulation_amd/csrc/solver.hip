@@ -599,11 +599,10 @@ __global__ __launch_bounds__(kTile) void k_xsph_st(Nbr P, PairList L, const floa
                     }
                     if (past && stage_past(a0, a1, a2, a3)) {
 #pragma unroll
-                        for (int u = 0; u < 4; ++u)
-                            if (a[u] >= kStageCap) {
-                                q[u] = xs[j[u]];
-                                w[u] = vin[j[u]];
-                            }
+                        for (int u = 0; u < 4; ++u) {
+                            q[u] = xs[j[u]];
+                            w[u] = vin[j[u]];
+                        }
                     }
 #pragma unroll
                     for (int u = 0; u < 4; ++u)
@@ -935,12 +934,11 @@ __global__ __launch_bounds__(kTile) void k_change_st(Nbr P, PairList L,
                         }
                         if (past && stage_past(a0, a1, a2, a3)) {
 #pragma unroll
-                            for (int u = 0; u < 4; ++u)
-                                if (a[u] >= kStageCap) {
-                                    const u32 j = stage_source(R, a[u]);
-                                    q[u] = xs[j];
-                                    w[u] = vs[j];
-                                }
+                            for (int u = 0; u < 4; ++u) {
+                                const u32 j = stage_source(R, a[u]);
+                                q[u] = xs[j];
+                                w[u] = vs[j];
+                            }
                         }
 #pragma unroll
                         for (int u = 0; u < 4; ++u) term(q[u], w[u], u == 0 || m > static_cast<u32>(u));
@@ -1270,8 +1268,7 @@ __global__ __launch_bounds__(kTile) void k_apply_st(Nbr P, PairList L,
                     for (int u = 0; u < 4; ++u) q[u] = s_x[past ? min(a[u], kStageCap - 1u) : a[u]];
                     if (past && stage_past(a0, a1, a2, a3)) {
 #pragma unroll
-                        for (int u = 0; u < 4; ++u)
-                            if (a[u] >= kStageCap) q[u] = xk[stage_source(R, a[u])];
+                        for (int u = 0; u < 4; ++u) q[u] = xk[stage_source(R, a[u])];
                     }
 #pragma unroll
                     for (int u = 0; u < 4; ++u) term(q[u], u == 0 || m > static_cast<u32>(u));

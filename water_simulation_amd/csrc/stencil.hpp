@@ -35,6 +35,7 @@ struct Nbr {
     int remap;              // XCD-aware workgroup order
     const u32* keys;        // fluid cell keys in sorted order (scene key base included)
     const u32* bnear;       // boundary proximity mask over the boundary grid, or nullptr
+    u32 stage_max;          // largest neighbourhood of a tile with a plan (see stage_ranges)
 };
 
 // 27-cell stencil of ITER_NEIGHBORS (dfsph_kernels.cu:13-35): dz, dy, dx in
@@ -198,24 +199,48 @@ __device__ __forceinline__ bool finite3(float a, float b, float c) {
 // dx in the key range [kmin + dx Dy Dz - Dz - 1, kmax + dx Dy Dz + Dz + 1]:
 // three contiguous slot ranges hold every fluid neighbour of the tile, at
 // rest about 3 (256 + 2 W) particles for fluid W particles wide along z.  A
-// tile with disjoint ranges of up to kStageMax entries has a plan: it stages
+// tile with disjoint ranges of up to stage_max entries has a plan: it stages
 // the first kStageCap in LDS and reads the others from global memory (L2);
 // other tiles (particles outside the grid, very wide fluid) gather everything
 // and keep 8-byte list entries.
 //
 // The staged part sets how many workgroups share a CU: with 2,048 entries a
 // 100-wide exact block, whose tiles fit in 1,536, went from 187 to 223 us
-// (density) and 64 to 76 (change).  Planning past the staged part costs such
-// tiles nothing (the branch is tile-uniform).  One million particles, no
-// plan -> plan up to 4,096, us per launch:
-//   tolerance mode  W 187 (1,896 entries)  density 158 -> 103  XSPH 103 -> 62   change 88 -> 66   apply 52 -> 38
-//                   W 385 (3,078)          density 154 -> 104  XSPH 112 -> 80   change 91 -> 84   apply 56 -> 43
-//   exact           W 187                  density 233 -> 195  XSPH 133 -> 82   change 119 -> 90  apply 70 -> 56
-//                   W 385                  density 245 -> 193  XSPH 138 -> 101  change 127 -> 103 apply 76 -> 59
+// (density) and 64 to 76 (change).
+//
+// Plans past the staged part pay on large working sets only (stage_max_of):
+// there the 8-byte lists and unstaged gathers are memory traffic, while with
+// few workgroups on a CU the tile that stages and then waits for L2 ends
+// last.  us per launch, plans up to 1,536 -> up to 4,096 entries (W = 164 to
+// 512 along z; a collapsing dam: 2 to 5 % of its tiles past 1,536, 16 % at
+// 1 M):
+//   tolerance        density       XSPH          change        apply
+//    64 k dam      30.7 ->  29.6  12.0 -> 12.1  10.5 -> 12.7   9.1 -> 10.7
+//    91 k W 187    22.7 ->  21.5  14.3 -> 13.3  12.7 -> 12.0   9.9 ->  9.7
+//   130 k W 200    23.6 ->  21.1  15.4 -> 14.1  13.7 -> 13.2  11.7 -> 11.0
+//   262 k dam      47.3 ->  45.4  21.0 -> 20.5  19.0 -> 18.2  14.4 -> 14.2
+//   246 k W 512    27.1 ->  28.7  23.9 -> 19.7  22.6 -> 20.6  16.3 -> 15.1
+//   991 k W 512    74.2 ->  69.8  85.0 -> 61.1  69.4 -> 62.9  47.2 -> 39.4
+//   1.1 M W 187    81.8 ->  74.4  96.5 -> 64.8  79.6 -> 61.4  54.0 -> 40.0
+//   exact
+//    91 k W 187    27.2 ->  26.9  17.0 -> 17.5  14.4 -> 17.3  12.4 -> 14.6
+//   262 k dam      81.3 ->  80.3  26.1 -> 26.5  25.8 -> 27.5  22.3 -> 23.0
+//   262 k W 164    41.0 ->  40.3  30.7 -> 27.8  27.0 -> 26.9  20.5 -> 19.9
+//   590 k W 256    74.3 ->  72.1  57.1 -> 55.3  52.1 -> 58.8  35.2 -> 38.2
+//   991 k W 512   117.1 -> 111.6   103 -> 89.8  91.3 -> 95.2  57.8 -> 60.9
+//   1.0 M dam     175.4 -> 169.7  73.7 -> 66.3  73.2 -> 72.3  50.0 -> 54.5
+//   1.1 M W 187   121.3 -> 120.8   116 -> 91.0   104 -> 91.2  66.4 -> 60.0
+//   1.5 M W 512   169.1 -> 150.9   156 ->  130   157 ->  135   104 -> 84.7
+// Exact pairs recompute c at the cost of a square root and a division, which
+// the 8-byte lists hold: up to 1 M they stay ahead in the pressure sweeps,
+// of which a substep has up to 100.
 constexpr u32 kStageCap = 1536;  // staged fluid particles per 256-slot tile
 static_assert(kStageCap % kTile == 0, "whole staging rounds per thread");
-constexpr u32 kStageMax = 4096;  // neighbourhood of a tile with a plan
+constexpr u32 kStageMax = 4096;  // neighbourhood of a tile with a plan, large working sets
 static_assert(kStageMax >= kStageCap && kStageMax <= 65536, "2-byte list entries");
+constexpr u32 stage_max_of(bool fast, u32 nslots) {
+    return nslots >= (fast ? 1u << 17 : 1u << 20) ? kStageMax : kStageCap;
+}
 
 // (StageRanges is declared in wsim_internal.hpp; an empty range sits where
 // the previous one ends.)
@@ -260,7 +285,7 @@ __device__ inline StageRanges stage_ranges(const Nbr& P, const SceneSeg& G, u32 
     R.b1 = e0 - R.s0;
     R.b2 = R.b1 + (e1 - R.s1);
     const u32 total = R.b2 + (e2 - R.s2);
-    R.total = total <= kStageMax ? total : 0u;
+    R.total = total <= P.stage_max ? total : 0u;
     return R;
 }
 
@@ -284,7 +309,10 @@ __device__ __forceinline__ u32 stage_source(const StageRanges& R, u32 e) {
     return e >= R.b2 ? R.s2 + (e - R.b2) : (e >= R.b1 ? R.s1 + (e - R.b1) : R.s0 + e);
 }
 
-// Any of four entries past the staged ones.
+// Any of four entries past the staged ones: all four are then loaded from
+// global memory in one go (a load under each entry's own test waits for the
+// one before: change took 13.7 instead of 12.7 us on the 64 k dam above and
+// 80.0 instead of 72.3 on the 1.0 M one).
 __device__ __forceinline__ bool stage_past(u32 a, u32 b, u32 c, u32 d) {
     return max(max(a, b), max(c, d)) >= kStageCap;
 }
@@ -413,6 +441,7 @@ inline Nbr make_nbr(const CellGrid& fg, const CellGrid* bg, const float4* xb, co
     P.tile_scene = tile_scene;
     P.remap = static_cast<int>(remap);
     P.keys = fg.sorted_keys();
+    P.stage_max = stage_max_of(cfg.fast_math != 0, nslots);
     return P;
 }
 
