@@ -5,7 +5,7 @@ entries past the staged ones from global memory.  At rest a tile of a block W
 particles wide along z has 3 (256 + 2 W) neighbourhood entries: every field
 must hold the bits of the kernels that stage nothing, on both sides of both
 limits, in both arithmetic modes.  The second limit is above the first from
-131,072 working slots in tolerance mode and from 1,048,576 in exact mode.
+262,144 working slots in tolerance mode and from 1,048,576 in exact mode.
 """
 from __future__ import annotations
 
@@ -22,10 +22,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("fast", [False, True], ids=["exact", "fast"])
 @pytest.mark.parametrize("dims", [
     (25, 44, 124),   # 1,512 entries: all staged
-    (25, 42, 132),   # 1,560: a few past the staged ones
+    (25, 42, 132),   # 1,560: past the staged part
     (22, 15, 420),   # 3,288
-    (21, 12, 544),   # 4,032: the last plans
-    (20, 12, 576),   # 4,224: most tiles without a plan
+    (21, 12, 544),   # 4,032
+    (20, 12, 576),   # 4,224
 ])
 def test_wide_tiles_equal_unstaged_kernels(dims, fast):
     rng = np.random.default_rng(dims[2])
@@ -45,19 +45,23 @@ def test_wide_tiles_equal_unstaged_kernels(dims, fast):
         assert sa[k] == sb[k], (k, sa, sb)
 
 
-@pytest.mark.parametrize("dims", [
-    (68, 66, 236),   # 2,184 entries
-    (46, 43, 544),   # 4,032: the last plans
-    (46, 41, 576),   # 4,224: most tiles without a plan
+@pytest.mark.parametrize("fast,dims", [
+    (False, (68, 66, 236)),   # 2,184 entries
+    (False, (46, 43, 544)),   # 4,032: the last plans
+    (False, (46, 41, 576)),   # 4,224: most tiles without a plan
+    (True, (48, 44, 132)),    # 1,560: a few past the staged ones
+    (True, (26, 25, 420)),    # 3,288
+    (True, (25, 20, 544)),
+    (True, (25, 19, 576)),
 ])
-def test_large_exact_wide_tiles_equal_unstaged_kernels(dims):
+def test_wide_tiles_of_large_sets_equal_unstaged_kernels(fast, dims):
     rng = np.random.default_rng(dims[2])
     g = np.stack(np.meshgrid(*map(np.arange, dims), indexing="ij"), -1).reshape(-1, 3)
-    assert len(g) > 1048576
+    assert len(g) > (262144 if fast else 1048576)
     x = (0.05 + 2 * R * g + rng.uniform(-0.2 * R, 0.2 * R, g.shape)).astype(np.float32)
     v = rng.normal(0.0, 0.4, g.shape).astype(np.float32)
     cfg = dict(DENSE_CFG, domain_max=tuple(0.1 + 2 * R * (d + 2) for d in dims), max_density_iters=3,
-               enable_divergence_solve=True, max_divergence_iters=2, fast_math=False)
+               enable_divergence_solve=True, max_divergence_iters=2, fast_math=fast)
     b, sb = run(x, v, None, cfg, ONE_LANE)
     for shapes in (None, LANES[4]):
         a, sa = run(x, v, None, cfg, shapes)

@@ -217,7 +217,7 @@ __device__ __forceinline__ bool finite3(float a, float b, float c) {
 //   tolerance        density       XSPH          change        apply
 //    64 k dam      30.7 ->  29.6  12.0 -> 12.1  10.5 -> 12.7   9.1 -> 10.7
 //    91 k W 187    22.7 ->  21.5  14.3 -> 13.3  12.7 -> 12.0   9.9 ->  9.7
-//   130 k W 200    23.6 ->  21.1  15.4 -> 14.1  13.7 -> 13.2  11.7 -> 11.0
+//   191 k W 187    25.1 ->  23.1  19.4 -> 15.9  17.4 -> 15.1  13.7 -> 12.5
 //   262 k dam      47.3 ->  45.4  21.0 -> 20.5  19.0 -> 18.2  14.4 -> 14.2
 //   246 k W 512    27.1 ->  28.7  23.9 -> 19.7  22.6 -> 20.6  16.3 -> 15.1
 //   991 k W 512    74.2 ->  69.8  85.0 -> 61.1  69.4 -> 62.9  47.2 -> 39.4
@@ -233,13 +233,15 @@ __device__ __forceinline__ bool finite3(float a, float b, float c) {
 //   1.5 M W 512   169.1 -> 150.9   156 ->  130   157 ->  135   104 -> 84.7
 // Exact pairs recompute c at the cost of a square root and a division, which
 // the 8-byte lists hold: up to 1 M they stay ahead in the pressure sweeps,
-// of which a substep has up to 100.
+// of which a substep has up to 100.  In tolerance mode the line lies where a
+// collapsing dam of 100 iterations a substep no longer loses: 140 k 2,162 ->
+// 2,247 us a substep, 262 k 2,663 -> 2,651, 512 k 3,912 -> 3,767.
 constexpr u32 kStageCap = 1536;  // staged fluid particles per 256-slot tile
 static_assert(kStageCap % kTile == 0, "whole staging rounds per thread");
 constexpr u32 kStageMax = 4096;  // neighbourhood of a tile with a plan, large working sets
 static_assert(kStageMax >= kStageCap && kStageMax <= 65536, "2-byte list entries");
 constexpr u32 stage_max_of(bool fast, u32 nslots) {
-    return nslots >= (fast ? 1u << 17 : 1u << 20) ? kStageMax : kStageCap;
+    return nslots >= (fast ? 1u << 18 : 1u << 20) ? kStageMax : kStageCap;
 }
 
 // (StageRanges is declared in wsim_internal.hpp; an empty range sits where
