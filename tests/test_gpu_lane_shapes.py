@@ -46,9 +46,11 @@ def test_small_scenes_match_oracle(over, lanes):
 
 def scene(case, n):
     """Clumps over the list depth, coincident pairs, escapees; `wide` is past
-    the staged part of a tile, with a squeezed corner."""
+    the staged part of a tile, with a squeezed corner (n layers; tiles of such
+    neighbourhoods have plans from 48 layers on in tolerance mode, 182 in exact
+    mode, and gather everything below)."""
     if case == "wide":
-        dims = (24, 44, 132)
+        dims = (n, 44, 132)
         g = np.stack(np.meshgrid(*map(np.arange, dims), indexing="ij"), -1).reshape(-1, 3)
         rng = np.random.default_rng(n)
         x = 0.05 + 2 * R * g + rng.uniform(-0.2 * R, 0.2 * R, g.shape)
@@ -68,7 +70,8 @@ def scene(case, n):
 @pytest.mark.parametrize("case,n,lanes", [
     ("clump", 300, 1), ("clump", 4000, 1), ("clump", 4000, 4),
     ("clump", 140000, None), ("clump", 140000, 4),  # None: the default, one lane at this size
-    ("wide", 0, None), ("wide", 0, 4),
+    ("wide", 24, None), ("wide", 24, 4), ("wide", 48, None), ("wide", 48, 4),
+    ("wide", 182, None), ("wide", 182, 4),
 ])
 def test_irregular_scenes_equal_unstaged_kernels(case, n, lanes, fast):
     x, v = scene(case, n)
